@@ -29,7 +29,8 @@
 // take two: prefill_dequant_kernel writes the attended keys once as dense
 // bf16 K and V^T, then prefill_dense_kernel runs the same products over
 // 128-key stages that direct-to-LDS buffer loads fill (no staging registers),
-// optionally split over key ranges with prefill_merge_kernel combining them.
+// with 256, 128 or 64 rows per workgroup and optionally split over key ranges
+// with prefill_merge_kernel combining them (dense_plan).
 #include <algorithm>
 
 #include "fq_common.h"
@@ -647,11 +648,22 @@ FQ_DEV void dma16_to_lds(i32x4 rsrc, const uint16_t* dst, int voff, int soff) {
                  :: "v"(voff), "s"(rsrc), "s"(soff), "{m0}"(lds) : "memory");
 }
 
-template <int QB>
+//
+// KG key groups (1, 2 or 4): the workgroup's waves are 8 / KG row groups of
+// 16 QB rows times KG key groups, key group kg taking keys [kg * 128 / KG,
+// (kg + 1) * 128 / KG) of every stage for its rows; the KG states of a row
+// group meet in LDS at the end.  KG = 1 (256 rows a workgroup) moves the
+// fewest K / V bytes per product and is the form that fills the matrix pipes
+// on long prompts; a shorter prompt has too few 256-row blocks for 256 CUs and
+// its last blocks' stages are the critical path, which KG = 2 and 4 cut to a
+// half and a quarter (dense_plan below chooses).
+template <int QB, int KG>
 __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2)))
 void prefill_dense_kernel(PrefillParams a) {
     constexpr int ST = kDenseKT;
-    constexpr int RW = 16 * QB, RWG = kPW * RW;
+    constexpr int RW = 16 * QB, RWG = kPW / KG * RW;
+    constexpr int NK = KG == 4 ? 2 : 4, NJ = NK / 2;     // 16-key blocks / 32-key steps of a wave's sub-tile
+    constexpr int SUB = 16 * NK;                         // keys of a sub-tile
     __shared__ __attribute__((aligned(1024))) uint16_t s_k[2][ST * kPD];
     __shared__ __attribute__((aligned(1024))) uint16_t s_v[2][kPD * ST];
 
@@ -675,7 +687,8 @@ void prefill_dense_kernel(PrefillParams a) {
     const int t_begin = min(nt_all, split * per);
     const int nt = min(nt_all, t_begin + per);
 
-    const int mw0 = m0 + w * RW;
+    const int kg = KG == 1 ? 0 : w / (kPW / KG);         // key group, row group w % (8 / KG)
+    const int mw0 = m0 + (KG == 1 ? w : w % (kPW / KG)) * RW;
     const bool wave_on = mw0 < Mtot;
     const int pmin = min(mw0, Mtot - 1) / a.nrep;
 
@@ -739,16 +752,16 @@ void prefill_dense_kernel(PrefillParams a) {
         for (int j = 0; j < 4; ++j) dma16_to_lds(vrw, s_v[buf] + (16 * wu + 4 * j) * ST, voff[j], key0 * 2);
     };
 
-    // S^T = K Q^T for one 64-key sub-tile (sk: its first key row; row & 15 = n)
-    auto qk = [&](const uint16_t* sk, v4f (&s)[QB][4]) {
+    // S^T = K Q^T for one sub-tile (sk: its first key row; row & 15 = n)
+    auto qk = [&](const uint16_t* sk, v4f (&s)[QB][NK]) {
 #pragma unroll
-        for (int kb = 0; kb < 4; ++kb)
+        for (int kb = 0; kb < NK; ++kb)
 #pragma unroll
             for (int qb = 0; qb < QB; ++qb) s[qb][kb] = v4f{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
         for (int ks = 0; ks < 4; ++ks)
 #pragma unroll
-            for (int kb = 0; kb < 4; ++kb) {
+            for (int kb = 0; kb < NK; ++kb) {
                 const v8bf ak = *(const v8bf*)(sk + (kb * 16 + n) * kPD + (((4 * ks + g) ^ n) * 8));
 #pragma unroll
                 for (int qb = 0; qb < QB; ++qb)
@@ -756,13 +769,13 @@ void prefill_dense_kernel(PrefillParams a) {
             }
     };
     // causal / length mask of a sub-tile starting at key k0 (only near the diagonal or the end)
-    auto diag_mask = [&](int k0, v4f (&s)[QB][4]) {
-        if (k0 + kPKT - 1 > pmin + a.causal_off || k0 + kPKT > a.Skv) {
+    auto diag_mask = [&](int k0, v4f (&s)[QB][NK]) {
+        if (k0 + SUB - 1 > pmin + a.causal_off || k0 + SUB > a.Skv) {
 #pragma unroll
             for (int qb = 0; qb < QB; ++qb) {
                 const int lim = min(qpos[qb] + a.causal_off, a.Skv - 1) - k0 - 4 * g;
 #pragma unroll
-                for (int kb = 0; kb < 4; ++kb)
+                for (int kb = 0; kb < NK; ++kb)
 #pragma unroll
                     for (int cc = 0; cc < 4; ++cc)
                         if (kb * 16 + cc > lim) s[qb][kb][cc] = -INFINITY;
@@ -773,14 +786,16 @@ void prefill_dense_kernel(PrefillParams a) {
     // more than 2^kLazyLog2: the reference then moves (raise_ref).  Until it
     // does, p <= 2^kLazyLog2 (exact in fp32, relative bf16 rounding unchanged)
     // and O and its denominator need no rescale.
-    auto tile_max = [&](const v4f (&s)[QB][4], float (&mx)[QB]) {
+    auto tile_max = [&](const v4f (&s)[QB][NK], float (&mx)[QB]) {
 #pragma unroll
         for (int qb = 0; qb < QB; ++qb) {
-            float t4[4];
+            float t4[NK];
 #pragma unroll
-            for (int kb = 0; kb < 4; ++kb)
+            for (int kb = 0; kb < NK; ++kb)
                 t4[kb] = fmaxf(fmaxf(s[qb][kb][0], s[qb][kb][1]), fmaxf(s[qb][kb][2], s[qb][kb][3]));
-            mx[qb] = rows_max(fmaxf(fmaxf(t4[0], t4[1]), fmaxf(t4[2], t4[3]))) * a.qk_scale;
+            float mm = fmaxf(t4[0], t4[1]);
+            if constexpr (NK == 4) mm = fmaxf(mm, fmaxf(t4[2], t4[3]));
+            mx[qb] = rows_max(mm) * a.qk_scale;
         }
     };
     auto moved = [&](const float (&mx)[QB]) {
@@ -800,12 +815,12 @@ void prefill_dense_kernel(PrefillParams a) {
         }
     };
     // P = exp2(s * qk_scale - reference) as the bf16 P^T operands
-    auto exp_p = [&](const v4f (&s)[QB][4], v8bf (&pb)[QB][2]) {
+    auto exp_p = [&](const v4f (&s)[QB][NK], v8bf (&pb)[QB][NJ]) {
 #pragma unroll
         for (int qb = 0; qb < QB; ++qb) {
             const float m_use = m_run[qb] == -INFINITY ? 0.f : m_run[qb];
 #pragma unroll
-            for (int j = 0; j < 2; ++j)
+            for (int j = 0; j < NJ; ++j)
 #pragma unroll
                 for (int cc = 0; cc < 4; ++cc) {
                     pb[qb][j][cc] = (__bf16)__builtin_amdgcn_exp2f(fmaf(s[qb][2 * j][cc], a.qk_scale, -m_use));
@@ -813,14 +828,14 @@ void prefill_dense_kernel(PrefillParams a) {
                 }
         }
     };
-    // O^T += V^T P^T (channel rows db * 16 + n, key chunks 8 sub + 4 j + g, vt_pos
-    // order) and the denominator block ones * P^T
-    auto pv = [&](const uint16_t* sv, int sub, const v8bf (&pb)[QB][2]) {
+    // O^T += V^T P^T (channel rows db * 16 + n, key chunks SUB / 8 * sub + 4 j + g,
+    // vt_pos order) and the denominator block ones * P^T
+    auto pv = [&](const uint16_t* sv, int sub, const v8bf (&pb)[QB][NJ]) {
 #pragma unroll
-        for (int j = 0; j < 2; ++j) {
+        for (int j = 0; j < NJ; ++j) {
 #pragma unroll
             for (int db = 0; db < 8; ++db) {
-                const v8bf av = *(const v8bf*)(sv + (db * 16 + n) * ST + (((8 * sub + 4 * j + g) ^ n) * 8));
+                const v8bf av = *(const v8bf*)(sv + (db * 16 + n) * ST + (((SUB / 8 * sub + 4 * j + g) ^ n) * 8));
 #pragma unroll
                 for (int qb = 0; qb < QB; ++qb)
                     o[qb][db] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(av, pb[qb][j], o[qb][db], 0, 0, 0);
@@ -831,69 +846,169 @@ void prefill_dense_kernel(PrefillParams a) {
         }
     };
 
-    // Stage t sits in buffer (t - t_begin) & 1.  The loop is pipelined across
-    // stages so that every phase pairs matrix work with vector work:
-    //   q.k of sub-tile 0 (stage t)        | exp of sub-tile 1 (stage t - 1)
-    //   p.v of sub-tile 1 (stage t - 1)    | maximum of sub-tile 0
-    //   -- barrier: V(t - 1) is free, V(t) has landed; V(t + 1) is issued --
-    //   q.k of sub-tile 1                  | exp of sub-tile 0
-    //   p.v of sub-tile 0                  | maximum of sub-tile 1
-    // O accumulates the sub-tiles in key order.  Every wave computes
-    // every sub-tile of the workgroup's stages (a wave with no rows computes
-    // none): the causal / length mask zeroes the keys past a wave's rows (exact
-    // zeros added to O and its denominator).
-    // K(t + 1) is issued at the top of iteration t, V(t + 1) after the middle
-    // barrier; the waits count the 4 loads per wave issued after the ones needed.
-    if (t_begin < nt) {
-        issue_k(0, t_begin * ST);
-        issue_v(0, t_begin * ST);
-    }
-    __builtin_amdgcn_s_waitcnt(0x0F70);   // vmcnt(0): the first stage and Q have landed
-    __syncthreads();
-    v4f s1p[QB][4];       // sub-tile 1 scores of the previous stage
-    for (int t = t_begin; t < nt; ++t) {
-        const int cur = (t - t_begin) & 1;
-        const int key0 = t * ST;
-        const bool more = t + 1 < nt;
-        // the other K buffer was last read before the previous iteration's end barrier
-        if (more) issue_k(cur ^ 1, key0 + ST);
-        v4f s0[QB][4];
-        float mx0[QB];
-        if (wave_on && t > t_begin) {
+    if constexpr (KG == 1) {
+        // Stage t sits in buffer (t - t_begin) & 1.  The loop is pipelined across
+        // stages so that every phase pairs matrix work with vector work:
+        //   q.k of sub-tile 0 (stage t)        | exp of sub-tile 1 (stage t - 1)
+        //   p.v of sub-tile 1 (stage t - 1)    | maximum of sub-tile 0
+        //   -- barrier: V(t - 1) is free, V(t) has landed; V(t + 1) is issued --
+        //   q.k of sub-tile 1                  | exp of sub-tile 0
+        //   p.v of sub-tile 0                  | maximum of sub-tile 1
+        // O accumulates the sub-tiles in key order.  Every wave computes
+        // every sub-tile of the workgroup's stages (a wave with no rows computes
+        // none): the causal / length mask zeroes the keys past a wave's rows (exact
+        // zeros added to O and its denominator).
+        // K(t + 1) is issued at the top of iteration t, V(t + 1) after the middle
+        // barrier; the waits count the 4 loads per wave issued after the ones needed.
+        if (t_begin < nt) {
+            issue_k(0, t_begin * ST);
+            issue_v(0, t_begin * ST);
+        }
+        __builtin_amdgcn_s_waitcnt(0x0F70);   // vmcnt(0): the first stage and Q have landed
+        __syncthreads();
+        v4f s1p[QB][4];       // sub-tile 1 scores of the previous stage
+        for (int t = t_begin; t < nt; ++t) {
+            const int cur = (t - t_begin) & 1;
+            const int key0 = t * ST;
+            const bool more = t + 1 < nt;
+            // the other K buffer was last read before the previous iteration's end barrier
+            if (more) issue_k(cur ^ 1, key0 + ST);
+            v4f s0[QB][4];
+            float mx0[QB];
+            if (wave_on && t > t_begin) {
+                v8bf pp[QB][2];
+                exp_p(s1p, pp);
+                qk(s_k[cur], s0);
+                diag_mask(key0, s0);
+                tile_max(s0, mx0);
+                pv(s_v[cur ^ 1], 1, pp);
+            } else if (wave_on) {
+                qk(s_k[cur], s0);
+                diag_mask(key0, s0);
+                tile_max(s0, mx0);
+            }
+            if (more) __builtin_amdgcn_s_waitcnt(0x0F74);   // vmcnt(4): V(t) is in LDS (K(t + 1) may be in flight)
+            else __builtin_amdgcn_s_waitcnt(0x0F70);
+            __syncthreads();
+            if (more) issue_v(cur ^ 1, key0 + ST);
+            if (wave_on) {
+                if (__builtin_amdgcn_ballot_w64(moved(mx0))) raise_ref(mx0);
+                v8bf p0[QB][2];
+                float mx1[QB];
+                exp_p(s0, p0);
+                qk(s_k[cur] + kPKT * kPD, s1p);
+                diag_mask(key0 + kPKT, s1p);
+                tile_max(s1p, mx1);
+                pv(s_v[cur], 0, p0);
+                if (__builtin_amdgcn_ballot_w64(moved(mx1))) raise_ref(mx1);
+            }
+            if (more) __builtin_amdgcn_s_waitcnt(0x0F74);   // vmcnt(4): K(t + 1) is in LDS (V(t + 1) may be in flight)
+            else __builtin_amdgcn_s_waitcnt(0x0F70);
+            __syncthreads();
+        }
+        if (wave_on && t_begin < nt) {   // the last stage's sub-tile 1 (its V buffer is not reloaded)
             v8bf pp[QB][2];
             exp_p(s1p, pp);
-            qk(s_k[cur], s0);
-            diag_mask(key0, s0);
-            tile_max(s0, mx0);
-            pv(s_v[cur ^ 1], 1, pp);
-        } else if (wave_on) {
-            qk(s_k[cur], s0);
-            diag_mask(key0, s0);
-            tile_max(s0, mx0);
+            pv(s_v[(nt - 1 - t_begin) & 1], 1, pp);
         }
-        if (more) __builtin_amdgcn_s_waitcnt(0x0F74);   // vmcnt(4): V(t) is in LDS (K(t + 1) may be in flight)
-        else __builtin_amdgcn_s_waitcnt(0x0F70);
+    } else {
+        // One sub-tile per wave and stage, pipelined across stages with one
+        // barrier each: iteration t pairs q.k of stage t with the exponentials
+        // and p.v of stage t - 1.  At its top every wave has finished stage
+        // t - 1's q.k and stage t - 2's p.v (the barrier), so K(t + 1) and
+        // V(t) stream into the buffers those read, for iteration t + 1.
+        if (t_begin < nt) issue_k(0, t_begin * ST);
+        __builtin_amdgcn_s_waitcnt(0x0F70);   // vmcnt(0): the first K stage and Q have landed
         __syncthreads();
-        if (more) issue_v(cur ^ 1, key0 + ST);
-        if (wave_on) {
-            if (__builtin_amdgcn_ballot_w64(moved(mx0))) raise_ref(mx0);
-            v8bf p0[QB][2];
-            float mx1[QB];
-            exp_p(s0, p0);
-            qk(s_k[cur] + kPKT * kPD, s1p);
-            diag_mask(key0 + kPKT, s1p);
-            tile_max(s1p, mx1);
-            pv(s_v[cur], 0, p0);
-            if (__builtin_amdgcn_ballot_w64(moved(mx1))) raise_ref(mx1);
+        v4f sp[QB][NK];
+        for (int t = t_begin; t < nt; ++t) {
+            const int cur = (t - t_begin) & 1;
+            const int key0 = t * ST;
+            if (t + 1 < nt) issue_k(cur ^ 1, key0 + ST);
+            issue_v(cur, key0);
+            if (wave_on) {
+                v4f sn[QB][NK];
+                float mx[QB];
+                if (t > t_begin) {
+                    v8bf pp[QB][NJ];
+                    exp_p(sp, pp);
+                    qk(s_k[cur] + kg * SUB * kPD, sn);
+                    diag_mask(key0 + kg * SUB, sn);
+                    tile_max(sn, mx);
+                    pv(s_v[cur ^ 1], kg, pp);
+                } else {
+                    qk(s_k[cur] + kg * SUB * kPD, sn);
+                    diag_mask(key0 + kg * SUB, sn);
+                    tile_max(sn, mx);
+                }
+                if (__builtin_amdgcn_ballot_w64(moved(mx))) raise_ref(mx);
+#pragma unroll
+                for (int qb = 0; qb < QB; ++qb)
+#pragma unroll
+                    for (int kb = 0; kb < NK; ++kb) sp[qb][kb] = sn[qb][kb];
+            }
+            __builtin_amdgcn_s_waitcnt(0x0F70);   // vmcnt(0): K(t + 1) and V(t) are in LDS
+            __syncthreads();
         }
-        if (more) __builtin_amdgcn_s_waitcnt(0x0F74);   // vmcnt(4): K(t + 1) is in LDS (V(t + 1) may be in flight)
-        else __builtin_amdgcn_s_waitcnt(0x0F70);
+        if (wave_on && t_begin < nt) {
+            v8bf pp[QB][NJ];
+            exp_p(sp, pp);
+            pv(s_v[(nt - 1 - t_begin) & 1], kg, pp);
+        }
+        // The key groups' states of a row group meet in key group 0's wave:
+        // the others hand theirs over in LDS (the K buffers: the loop's last
+        // barrier has passed every read of them), 16 bytes per lane and slot.
+        constexpr int NS = QB * 8;                       // O slots of a wave
+        static_assert(((KG - 1) * (kPW / KG)) * NS * 64 * 16 <= (int)(2 * ST * kPD * 2 * 2), "states fit K and V");
+        static_assert((kPW - kPW / KG) * QB * 64 * 8 <= 2 * 1024 * 8, "m, l fit");
+        __shared__ float2 s_ml[(kPW - kPW / KG) * QB * 64];
+        __syncthreads();                                 // the last p.v has read its V buffer
+        v4f* st_o = (v4f*)s_k[0];
+        v4f* st_o2 = (v4f*)s_v[0];
+        constexpr int kHalf = (int)(2 * ST * kPD * 2 / 16);      // v4f slots of the K (and of the V) buffers
+        auto slot = [&](int i) -> v4f* { return i < kHalf ? st_o + i : st_o2 + (i - kHalf); };
+        if (kg > 0) {
+            const int src = w - kPW / KG;                // 0 .. 8 - 8 / KG - 1
+#pragma unroll
+            for (int qb = 0; qb < QB; ++qb) {
+#pragma unroll
+                for (int db = 0; db < 8; ++db) *slot((src * NS + qb * 8 + db) * 64 + lane) = o[qb][db];
+                s_ml[(src * QB + qb) * 64 + lane] = make_float2(m_run[qb], o[qb][8][0]);
+            }
+        }
         __syncthreads();
-    }
-    if (wave_on && t_begin < nt) {   // the last stage's sub-tile 1 (its V buffer is not reloaded)
-        v8bf pp[QB][2];
-        exp_p(s1p, pp);
-        pv(s_v[(nt - 1 - t_begin) & 1], 1, pp);
+        if (kg > 0) return;
+#pragma unroll
+        for (int qb = 0; qb < QB; ++qb) {
+            float m[KG], l[KG], M = m_run[qb];
+            m[0] = m_run[qb]; l[0] = o[qb][8][0];
+#pragma unroll
+            for (int u = 1; u < KG; ++u) {
+                const float2 ml = s_ml[(((u - 1) * (kPW / KG) + w) * QB + qb) * 64 + lane];
+                m[u] = ml.x; l[u] = ml.y;
+                M = fmaxf(M, m[u]);
+            }
+            const float Mu = M == -INFINITY ? 0.f : M;       // no key of the slice attended: all weights 0
+            float wt[KG], Ls = 0.f;
+#pragma unroll
+            for (int u = 0; u < KG; ++u) {
+                wt[u] = __builtin_amdgcn_exp2f(m[u] - Mu);
+                Ls = fmaf(wt[u], l[u], Ls);
+            }
+#pragma unroll
+            for (int db = 0; db < 8; ++db) {
+                v4f acc = o[qb][db] * wt[0];
+#pragma unroll
+                for (int u = 1; u < KG; ++u) {
+                    const v4f x = *slot((((u - 1) * (kPW / KG) + w) * NS + qb * 8 + db) * 64 + lane);
+#pragma unroll
+                    for (int i = 0; i < 4; ++i) acc[i] = fmaf(wt[u], x[i], acc[i]);
+                }
+                o[qb][db] = acc;
+            }
+            m_run[qb] = M;
+            o[qb][8][0] = Ls;
+        }
     }
 
     if (!wave_on) return;
@@ -935,43 +1050,47 @@ void prefill_dense_kernel(PrefillParams a) {
 
 // Combines the key-range partials of the split path: per row (b, h, m)
 // M = max m_i, L = sum 2^(m_i - M) l_i, O = sum 2^(m_i - M) O_i / L, in split
-// order; one wave per row, lane = two channels.  The splits go in batches of
-// 8 whose loads are all issued before any is used; the running maximum moves
-// once per batch (earlier sums are rescaled by 2^(M_old - M_new)).
+// order; half a wave per row, lane = four channels.  The splits go in batches
+// of NB whose loads are all issued before any is used; the running maximum
+// moves once per batch (earlier sums are rescaled by 2^(M_old - M_new)).  It is
+// bound by its reads of the partials; NB is the smallest of 2, 4, 8 that takes
+// the splits in one batch, so that two splits don't cost eight splits' loads
+// (26400 rows of 2 splits: 13.7 -> 6.8 us).
+template <int NB>
 __global__ __launch_bounds__(256) void prefill_merge_kernel(PrefillParams a) {
-    constexpr int kBatch = 8;
     const int64_t rows = (int64_t)a.c.B * a.c.Hkv * a.Sq * a.nrep;
-    const int64_t row = ((int64_t)blockIdx.x * 256 + threadIdx.x) >> 6;
+    const int64_t row = ((int64_t)blockIdx.x * 256 + threadIdx.x) >> 5;
     if (row >= rows) return;
-    const int lane = threadIdx.x & 63;
+    const int ch = 4 * (threadIdx.x & 31);
     const int KS = a.kv_splits;
     const float* ml = a.part + (int64_t)KS * rows * kPD;
-    float M = -INFINITY, L = 0.f, o0 = 0.f, o1 = 0.f;
-    for (int sp0 = 0; sp0 < KS; sp0 += kBatch) {
-        float m[kBatch], l[kBatch];
-        float2 po[kBatch];
+    float M = -INFINITY, L = 0.f;
+    v4f o = {0.f, 0.f, 0.f, 0.f};
+    for (int sp0 = 0; sp0 < KS; sp0 += NB) {
+        float2 pm[NB];
+        v4f po[NB];
 #pragma unroll
-        for (int u = 0; u < kBatch; ++u) {
+        for (int u = 0; u < NB; ++u) {
             const int64_t sp = min(sp0 + u, KS - 1);
-            m[u] = ml[(sp * rows + row) * 2];
-            l[u] = ml[(sp * rows + row) * 2 + 1];
-            po[u] = *(const float2*)(a.part + (sp * rows + row) * kPD + 2 * lane);
+            pm[u] = *(const float2*)(ml + (sp * rows + row) * 2);
+            po[u] = *(const v4f*)(a.part + (sp * rows + row) * kPD + ch);
         }
         float Mb = M;
 #pragma unroll
-        for (int u = 0; u < kBatch; ++u)
-            if (sp0 + u < KS) Mb = fmaxf(Mb, m[u]);
+        for (int u = 0; u < NB; ++u)
+            if (sp0 + u < KS) Mb = fmaxf(Mb, pm[u].x);
         if (Mb == -INFINITY) continue;          // nothing attended yet
         const float r = M == -INFINITY ? 0.f : __builtin_amdgcn_exp2f(M - Mb);
-        L *= r; o0 *= r; o1 *= r;
+        L *= r;
+        o *= r;
         M = Mb;
 #pragma unroll
-        for (int u = 0; u < kBatch; ++u) {
+        for (int u = 0; u < NB; ++u) {
             if (sp0 + u >= KS) break;
-            const float wt = m[u] == -INFINITY ? 0.f : __builtin_amdgcn_exp2f(m[u] - M);
-            L = fmaf(wt, l[u], L);
-            o0 = fmaf(wt, po[u].x, o0);
-            o1 = fmaf(wt, po[u].y, o1);
+            const float wt = pm[u].x == -INFINITY ? 0.f : __builtin_amdgcn_exp2f(pm[u].x - M);
+            L = fmaf(wt, pm[u].y, L);
+#pragma unroll
+            for (int i = 0; i < 4; ++i) o[i] = fmaf(wt, po[u][i], o[i]);
         }
     }
     const int Mtot = a.Sq * a.nrep;
@@ -981,7 +1100,7 @@ __global__ __launch_bounds__(256) void prefill_merge_kernel(PrefillParams a) {
     const int hq = h * a.nrep + mi % a.nrep;
     uint16_t* orow = (uint16_t*)a.out + b * a.o_s[0] + hq * a.o_s[1] + (int64_t)(mi / a.nrep) * a.o_s[2];
     const float inv = 1.0f / L;
-    *(uint32_t*)(orow + 2 * lane) = pack_bf16(o0 * inv, o1 * inv);
+    *(u32x2*)(orow + ch) = u32x2{pack_bf16(o[0] * inv, o[1] * inv), pack_bf16(o[2] * inv, o[3] * inv)};
 }
 
 // The keys any query can attend: min(S_kv, S_q + causal_off).
@@ -990,32 +1109,55 @@ int64_t prefill_keys_needed(int Skv, int Sq, int causal_off) { return std::min<i
 int64_t prefill_row_blocks(int Sq, int nrep) { return ((int64_t)Sq * nrep + kPRows - 1) / kPRows; }
 
 constexpr int kDenseQB = 2;                       // 16-column query blocks per wave, dense path
-constexpr int kDenseRows = kPW * 16 * kDenseQB;   // query rows per dense workgroup
-int64_t dense_row_blocks(int Sq, int nrep) { return ((int64_t)Sq * nrep + kDenseRows - 1) / kDenseRows; }
 
 // The fused path (each workgroup dequantises the K/V tiles it attends) only
 // for one row block per KV head over at most 1024 keys; otherwise the
 // two-pass path (dequantise the needed keys once, in parallel, into dense
 // bf16 K and V^T, then attend plain bf16 tiles) is faster.
-// Key-range splits of the dense path: when the row blocks leave most CUs idle
-// (few query rows over many keys, e.g. a chunk with causal_off = S_kv - S_q),
-// workgroups take slices of at least 4 key stages and a merge launch combines
-// their partials.
-// Between 128 and 256 workgroups (one round on 256 CUs with some idle), the
-// split count k <= 8 with the fewest rounds per unit of work,
-// ceil(wgs k / 256) / k, evens the rounds out (192 workgroups: 4 splits, 3
-// full rounds of a quarter of the work each).
-int prefill_kv_splits(int64_t nblk, int64_t heads, int64_t keys) {
-    const int64_t wgs = nblk * heads;
+//
+// How the dense path covers the 256 CUs (one 8-wave workgroup each): key
+// groups per workgroup (kg: 256 / kg query rows a workgroup) and key-range
+// splits (ks > 1: workgroups take slices of at least 4 key stages, and a
+// merge launch combines their fp32 partials).
+struct DensePlan { int kg, ks; };
+
+// Estimated from the shape alone.  A stage of 128 keys takes 3.45 / 1.95 / 1.2
+// us with kg = 1 / 2 / 4 (256 workgroups running) and a workgroup about 6 us
+// besides; measured attention kernels (events, ~3 us over), 24 / 8 heads:
+//   1100-token prompt   kg 1: 41.1 (2 splits 33.0), kg 2: 27.7, kg 4: 26.4
+//   2048-token prompt   65.0 (45.7), 43.9, 57.6;  4096: 118.2, 125.9, 161.3
+//   512 queries over 24512 keys, kg 1: 4 / 5 / 6 splits 169 / 143 / 227 (6
+//   splits are 288 workgroups: a second round for 32 of them)
+// heads = batch x KV heads.  The workgroups run longest first.
+DensePlan dense_plan(int64_t rows, int64_t heads, int64_t keys, int causal_off) {
+    constexpr double kCus = 256.0;
+    constexpr double kStage[3] = {3.45, 1.95, 1.2};
+    constexpr double kFixed = 6.0;
+    constexpr double kMerge = 2.0, kPartRate = 4.5e6;       // us per merge launch, bytes of partials per us
     const int64_t stages = (keys + kDenseKT - 1) / kDenseKT;
-    if (stages < 8) return 1;
-    if (wgs < 128) return (int)std::max<int64_t>(1, std::min<int64_t>((256 + wgs - 1) / wgs, stages / 4));
-    if (wgs >= 256) return 1;
-    int best = 1;
-    double best_cost = 1.0;                  // rounds per unit of work with k = 1: one round
-    for (int k = 2; k <= 8 && stages / k >= 4; ++k) {
-        const double cost = (double)((wgs * k + 255) / 256) / k;
-        if (cost < best_cost - 1e-9) { best = k; best_cost = cost; }
+    const int64_t first = std::min<int64_t>(stages, ((int64_t)causal_off + kDenseKT) / kDenseKT);
+    const double r = (double)first / (double)stages;        // shortest row block / longest
+    DensePlan best{1, 1};
+    double best_t = 0.0;
+    for (int i = 0; i < 3; ++i) {
+        const int kg = 1 << i;
+        const int64_t wgs = heads * ((rows * kg + 255) / 256);
+        if (i > 0 && wgs > 16 * 256) break;                 // long prompts fill every round with kg = 1
+        for (int ks = 1; ks <= 32 && (ks == 1 || stages / ks >= 4); ++ks) {
+            const double n = (double)(wgs * ks) / kCus;
+            const double longest = (double)((stages + ks - 1) / ks) * kStage[i] + kFixed;
+            const double spread = (1.0 - r) * (longest - kFixed);
+            double t = longest;                             // one round
+            if (n > 2.0) {      // alike: whole rounds; of all lengths: the average, and a short one at the end
+                const double avg = longest - 0.5 * spread;
+                t = std::max(longest, r * std::ceil(n) * longest + (1.0 - r) * (n + 0.3) * avg);
+            } else if (n > 1.0) {   // the shortest of the first 256 is followed by the longest of the rest
+                t = std::max(longest, 2.0 * (longest - spread / n));
+            }
+            if (ks > 1) t += kMerge + 2.0 * ks * (double)(heads * rows) * (kPD + 2) * 4 / kPartRate;
+            if (best_t == 0.0 || t < best_t) { best = {kg, ks}; best_t = t; }
+            if (n > 8.0) break;
+        }
     }
     return best;
 }
@@ -1025,7 +1167,7 @@ size_t prefill_dense_bytes(int Hkv, int B, int Skv, int Sq, int nrep, int causal
     const int64_t keys = prefill_keys_needed(Skv, Sq, causal_off);
     const int64_t s_pad = (keys + kDenseKT - 1) / kDenseKT * kDenseKT;
     size_t n = (size_t)(2 * s_pad * kPD * 2) * Hkv * B;
-    const int ks = prefill_kv_splits(dense_row_blocks(Sq, nrep), (int64_t)Hkv * B, keys);
+    const int ks = dense_plan((int64_t)Sq * nrep, (int64_t)Hkv * B, keys, causal_off).ks;
     if (ks > 1) n += (size_t)ks * B * Hkv * Sq * nrep * (kPD + 2) * sizeof(float);
     return n;
 }
@@ -1039,17 +1181,23 @@ size_t prefill_workspace_bytes(const Int4Cache& c, int Skv, int Sq, int nrep, in
 // The attention launch of the dense path (a.kd / a.vtd / a.s_pad set), with
 // key-range splits and their merge when the row blocks are few.
 hipError_t launch_dense_attn(PrefillParams& a, int Sq, int nrep, hipStream_t st) {
-    const int64_t nblk = dense_row_blocks(Sq, nrep);
-    const int64_t heads = (int64_t)a.c.Hkv * a.c.B;
-    const int ks = prefill_kv_splits(nblk, heads, prefill_keys_needed(a.Skv, Sq, a.causal_off));
-    a.kv_splits = ks;
-    a.part = ks > 1 ? (float*)(a.vtd + (int64_t)a.s_pad * kPD * heads) : nullptr;
+    const int64_t heads = (int64_t)a.c.Hkv * a.c.B, rows = (int64_t)Sq * nrep;
+    const DensePlan pl = dense_plan(rows, heads, prefill_keys_needed(a.Skv, Sq, a.causal_off), a.causal_off);
+    const int rwg = 256 / pl.kg;
+    const int64_t nblk = (rows + rwg - 1) / rwg;
+    a.kv_splits = pl.ks;
+    a.part = pl.ks > 1 ? (float*)(a.vtd + (int64_t)a.s_pad * kPD * heads) : nullptr;
+    const dim3 grid((unsigned)(nblk * heads * pl.ks));
     timer_before_launch(st);
-    hipLaunchKernelGGL((prefill_dense_kernel<kDenseQB>), dim3((unsigned)(nblk * heads * ks)), dim3(512), 0, st, a);
+    if (pl.kg == 1) hipLaunchKernelGGL((prefill_dense_kernel<kDenseQB, 1>), grid, dim3(512), 0, st, a);
+    else if (pl.kg == 2) hipLaunchKernelGGL((prefill_dense_kernel<kDenseQB, 2>), grid, dim3(512), 0, st, a);
+    else hipLaunchKernelGGL((prefill_dense_kernel<kDenseQB, 4>), grid, dim3(512), 0, st, a);
     timer_after_launch(st);
-    if (ks > 1) {
-        const int64_t rows = heads * Sq * nrep;
-        hipLaunchKernelGGL(prefill_merge_kernel, dim3((unsigned)((rows * 64 + 255) / 256)), dim3(256), 0, st, a);
+    if (pl.ks > 1) {
+        const dim3 mgrid((unsigned)((heads * rows * 32 + 255) / 256));
+        if (pl.ks <= 2) hipLaunchKernelGGL(prefill_merge_kernel<2>, mgrid, dim3(256), 0, st, a);
+        else if (pl.ks <= 4) hipLaunchKernelGGL(prefill_merge_kernel<4>, mgrid, dim3(256), 0, st, a);
+        else hipLaunchKernelGGL(prefill_merge_kernel<8>, mgrid, dim3(256), 0, st, a);
     }
     return hipGetLastError();
 }
