@@ -286,14 +286,15 @@ FQ_DEV void tail_state(const QueryArgs& q, const TailArgs& tail, int l, int b, i
 template <int D, int NREP, int NT>
 FQ_DEV void tail_state_lds(const uint16_t (*tk)[D], const uint16_t (*tv)[D], bool bf, int T, const float (*sq)[D],
                            float (*sp)[kTailMax], float* m_out, float* l_out, float (*acc_out)[D]) {
-    static_assert(D == 128 && NT % D == 0 && NT % 16 == 0, "tail layout");
+    static_assert((D == 128 || D == 64) && NT % D == 0, "tail layout");
     constexpr int NH = NT / D;                       // token groups in the p.v phase
+    constexpr int LPT = D / 8;                       // lanes per token in the q.k phase
     const int tid = threadIdx.x, lane = lane_id(), w = wave_id();
     auto cvt = [&](uint32_t bits) { return bf ? bf16_bits_to_f(bits & 0xFFFFu) : f16_bits_to_f(bits & 0xFFFFu); };
-    // logits: 16 lanes per token, lane j owns channels 8j .. 8j+7 (one 16-byte LDS read)
-    for (int i0 = 0; i0 < kTailMax * 16; i0 += NT) {
+    // logits: LPT lanes per token, lane j owns channels 8j .. 8j+7 (one 16-byte LDS read)
+    for (int i0 = 0; i0 < kTailMax * LPT; i0 += NT) {
         const int i = i0 + tid;
-        const int t = min(i >> 4, kTailMax - 1), j = i & 15;
+        const int t = min(i / LPT, kTailMax - 1), j = i % LPT;
         const uint4 raw = *(const uint4*)&tk[t][8 * j];
         const uint32_t wv[4] = {raw.x, raw.y, raw.z, raw.w};
         float kv[8];
@@ -305,7 +306,7 @@ FQ_DEV void tail_state_lds(const uint16_t (*tk)[D], const uint16_t (*tv)[D], boo
 #pragma unroll
             for (int c = 0; c < 8; ++c) v = fmaf(sq[r][8 * j + c], kv[c], v);
 #pragma unroll
-            for (int off = 1; off < 16; off <<= 1) v += __shfl_xor(v, off, 64);
+            for (int off = 1; off < LPT; off <<= 1) v += __shfl_xor(v, off, 64);
             if (j == 0 && t < T) sp[r][t] = v;
         }
     }
@@ -432,15 +433,15 @@ __global__ __launch_bounds__(kThreads) void merge_splits_kernel(QueryArgs q, Wor
 }
 
 // The same merge for few splits (<= SM) and no tail to fold in, as a latency
-// path: one wave per (group, query head), lane d holding channels d and
-// d + 64, every split's (m, l) and partial acc loaded in one round, then
+// path: one wave per (group, query head), lane d holding channels d and (D =
+// 128) d + 64, every split's (m, l) and partial acc loaded in one round, then
 // M = max_s m_s, w_s = exp2(m_s - M) (0 for an empty split), L = sum_s w_s l_s,
 // O = (sum_s w_s acc_s) / L, splits summed in ascending order.  ROT (or
 // q.rot): O rotated back by the wave butterflies, as store_outputs does.
-template <bool ROT, int SM>
+template <bool ROT, int SM, int D>
 __global__ __launch_bounds__(64) void merge_splits_wave_kernel(QueryArgs q, Workspace ws, int Hkv, int B,
                                                                 int splits) {
-    constexpr int D = 128;
+    static_assert(D == 128 || (D == 64 && !ROT), "two channels per lane, or one");
     const int g = blockIdx.x, r = blockIdx.y, nrep = q.nrep;
     const int h = g % Hkv, b = (g / Hkv) % B, l = g / (Hkv * B);
     const int lane = threadIdx.x;
@@ -452,7 +453,7 @@ __global__ __launch_bounds__(64) void merge_splits_wave_kernel(QueryArgs q, Work
         m[s] = ws.part_ml[pr * 2];
         lv[s] = ws.part_ml[pr * 2 + 1];
         a0[s] = ws.part_acc[pr * D + lane];
-        a1[s] = ws.part_acc[pr * D + lane + 64];
+        a1[s] = D == 128 ? ws.part_acc[pr * D + lane + 64] : 0.f;
     }
     float M = -INFINITY;
 #pragma unroll
@@ -469,7 +470,7 @@ __global__ __launch_bounds__(64) void merge_splits_wave_kernel(QueryArgs q, Work
         }
     }
     float v0 = L > 0.f ? A0 / L : 0.f, v1 = L > 0.f ? A1 / L : 0.f;
-    if (ROT || q.rot) {
+    if (D == 128 && (ROT || q.rot)) {
         const float inv = 1.0f / sqrtf((float)D);
         const float s0 = q.rot ? q.rot[lane] : 1.f, s1 = q.rot ? q.rot[lane + 64] : 1.f;
         wave_hadamard128(v0, v1);
@@ -479,25 +480,25 @@ __global__ __launch_bounds__(64) void merge_splits_wave_kernel(QueryArgs q, Work
     const int hq = h * nrep + r;
     const int64_t ob = l * q.o_s[0] + b * q.o_s[1] + hq * q.o_s[2];
     store_any(q.out, q.out_dtype, ob + lane * q.o_s[3], v0);
-    store_any(q.out, q.out_dtype, ob + (lane + 64) * q.o_s[3], v1);
+    if (D == 128) store_any(q.out, q.out_dtype, ob + (lane + 64) * q.o_s[3], v1);
     if (q.lse && lane == 0)
         q.lse[l * q.lse_s[0] + b * q.lse_s[1] + hq * q.lse_s[2]] = L > 0.f ? (M + log2f(L)) * kLn2 : -INFINITY;
 }
 
-// The split merge launch of the D = 128 matrix-core paths: the one-round wave
+// The split merge launch of the matrix-core paths: the one-round wave
 // merge for up to 32 splits without a tail, merge_splits_kernel otherwise.
-template <int NREP, bool ROT>
+template <int NREP, bool ROT, int D = 128>
 inline void launch_split_merge(const QueryArgs& q, const Workspace& ws, int Hkv, int B, int groups, int splits,
                                const TailArgs& tail, hipStream_t st) {
     if (tail.len == 0 && splits <= 32) {
         const dim3 grid(groups, NREP);
-        if (splits <= 8) hipLaunchKernelGGL((merge_splits_wave_kernel<ROT, 8>), grid, dim3(64), 0, st, q, ws, Hkv, B, splits);
-        else if (splits <= 16) hipLaunchKernelGGL((merge_splits_wave_kernel<ROT, 16>), grid, dim3(64), 0, st, q, ws, Hkv, B, splits);
-        else if (splits <= 24) hipLaunchKernelGGL((merge_splits_wave_kernel<ROT, 24>), grid, dim3(64), 0, st, q, ws, Hkv, B, splits);
-        else hipLaunchKernelGGL((merge_splits_wave_kernel<ROT, 32>), grid, dim3(64), 0, st, q, ws, Hkv, B, splits);
+        if (splits <= 8) hipLaunchKernelGGL((merge_splits_wave_kernel<ROT, 8, D>), grid, dim3(64), 0, st, q, ws, Hkv, B, splits);
+        else if (splits <= 16) hipLaunchKernelGGL((merge_splits_wave_kernel<ROT, 16, D>), grid, dim3(64), 0, st, q, ws, Hkv, B, splits);
+        else if (splits <= 24) hipLaunchKernelGGL((merge_splits_wave_kernel<ROT, 24, D>), grid, dim3(64), 0, st, q, ws, Hkv, B, splits);
+        else hipLaunchKernelGGL((merge_splits_wave_kernel<ROT, 32, D>), grid, dim3(64), 0, st, q, ws, Hkv, B, splits);
         return;
     }
-    hipLaunchKernelGGL((merge_splits_kernel<128, NREP, ROT>), dim3(groups), dim3(kThreads), 0, st, q, ws, Hkv, B, 0,
+    hipLaunchKernelGGL((merge_splits_kernel<D, NREP, ROT>), dim3(groups), dim3(kThreads), 0, st, q, ws, Hkv, B, 0,
                        splits, tail);
 }
 

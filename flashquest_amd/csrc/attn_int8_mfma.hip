@@ -55,8 +55,9 @@ struct Int8Params {
 
 // Per-wave LDS operands: q.k A digits of the current page [k-step][row][k-group,
 // swizzled][16 bytes]; p.v A of the current half page [row][k-group][16 bytes].
+template <int D>
 struct WaveLds8 {
-    uint8_t aqk[2][16][4][16];
+    uint8_t aqk[D / 64][16][4][16];
     uint8_t apv[16][4][16];
 };
 FQ_DEV int swz8(int row, int kg) { return kg ^ ((row >> 2) & 3); }
@@ -70,35 +71,40 @@ FQ_DEV uint32_t byte_of4(uint32_t y0, uint32_t y1, uint32_t y2, uint32_t y3) {
 
 // Half a page (tokens 32 hp .. 32 hp + 31): tiles T = 2 hp + t.
 struct HalfBuf {
-    uint4 kt[2][2];      // [t][k-step s]: K codes of token 16T + n16, bytes 64 s + 16 lg .. +15
-    uint2 vw[8];         // [2 ai + jj]: V codes of token 16 (2 hp + jj) + 4 ai + lg, bytes 8 n16 .. +7
+    uint4 kt[2][2];      // [t][k-step s]: K codes of token 16T + n16, bytes 64 s + 16 lg .. +15 (D = 64: s = 0)
+    uint2 vw[8];         // [2 ai + jj]: V codes of token 16 (2 hp + jj) + 4 ai + lg, bytes D/16 n16 .. (D = 64: x)
     uint32_t vs[2], vm[2];   // [t]: V scale / min (16-bit) of token 16T + n16
-    uint2 ks, km;        // K scale / min of the lane's channels 4 (L & 31) .. +3 (the page's)
+    uint2 ks, km;        // K scale / min of the lane's channels 4 (L % (D/4)) .. +3 (the page's)
 };
 
 struct Int8Rsrc {
     __amdgpu_buffer_rsrc_t k, v, vs, vm, ks, km;
 };
 
-// Dense rows (128-byte codes, 2-byte V metadata, 256-byte K metadata rows):
+// Dense rows (D-byte codes, 2-byte V metadata, 2 D-byte K metadata rows):
 // every offset is (lane part) + (page part) + an immediate.
+template <int D>
 FQ_DEV void load_half(HalfBuf& b, const Int8Rsrc& r, int p, int hp, int n16, int lg, int L) {
-    const int kbase = p * 64 * 128 + n16 * 128 + 16 * lg;
-    const int vbase = p * 64 * 128 + lg * 128 + 8 * n16;
+    const int kbase = p * 64 * D + n16 * D + 16 * lg;
+    const int vbase = p * 64 * D + lg * D + D / 16 * n16;
     const int mbase = (p * 64 + n16) * 2;
 #pragma unroll
     for (int t = 0; t < 2; ++t)
 #pragma unroll
-        for (int s = 0; s < 2; ++s) b.kt[t][s] = ld128(r.k, kbase + (32 * hp + 16 * t) * 128 + 64 * s);
+        for (int s = 0; s < D / 64; ++s) b.kt[t][s] = ld128(r.k, kbase + (32 * hp + 16 * t) * D + 64 * s);
 #pragma unroll
-    for (int i = 0; i < 8; ++i) b.vw[i] = ld64(r.v, vbase + (16 * (2 * hp + (i & 1)) + 4 * (i >> 1)) * 128);
+    for (int i = 0; i < 8; ++i) {
+        const int off = vbase + (16 * (2 * hp + (i & 1)) + 4 * (i >> 1)) * D;
+        if constexpr (D == 128) b.vw[i] = ld64(r.v, off);
+        else b.vw[i] = make_uint2(ld32(r.v, off), 0u);
+    }
 #pragma unroll
     for (int t = 0; t < 2; ++t) {
         b.vs[t] = ld16(r.vs, mbase + (32 * hp + 16 * t) * 2);
         b.vm[t] = ld16(r.vm, mbase + (32 * hp + 16 * t) * 2);
     }
-    b.ks = ld64(r.ks, p * 256 + 8 * (L & 31));
-    b.km = ld64(r.km, p * 256 + 8 * (L & 31));
+    b.ks = ld64(r.ks, p * 2 * D + 8 * (L % (D / 4)));
+    b.km = ld64(r.km, p * 2 * D + 8 * (L % (D / 4)));
 }
 
 // HCH (FUSED only): head chunks, sel.head_chunks virtual KV heads per cache KV
@@ -107,16 +113,22 @@ FQ_DEV void load_half(HalfBuf& b, const Int8Rsrc& r, int p, int hp, int n16, int
 // scores the summed query of all 2 NREP heads of the cache head, so every
 // chunk selects the same pages.  The chunks of a cache head are mapped to one
 // XCD so that the second one's page reads hit that XCD's L2.
-template <typename MT, int NREP, bool FUSED, bool HCH = false>
+//
+// D = 64: half the channels (one q.k step, four p.v tiles); its FUSED form
+// always selects from the scores of a scoring launch, as the INT4 kernel's.
+template <int D, typename MT, int NREP, bool FUSED, bool HCH = false>
 __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2)))
 void attn_int8_mfma_kernel(Int8Params a) {
-    constexpr int D = 128, NW = 8, NT = 512;
+    static_assert(D == 128 || D == 64, "head_dim");
+    constexpr int NW = 8, NT = 512;
+    constexpr int QKS = D / 64;                     // q.k k-steps; also the query heads a lane makes digits for
+    constexpr int NTL = D / 16;                     // p.v channel tiles
     static_assert(NREP <= 4, "query heads per KV head");
     static_assert(!HCH || FUSED, "head chunks run in the fused kernel");
     constexpr int NSLOT = FUSED ? NW + 1 : NW;      // the fused kernel's extra slot: the partial-page tail
     constexpr int TTOK = FUSED ? kTailMax : 1;
     __shared__ SplitLds<D, NREP, NSLOT> s_split;
-    __shared__ WaveLds8 s_wave[NW];
+    __shared__ WaveLds8<D> s_wave[NW];
     __shared__ int s_ent[kMaxWgPages];
     __shared__ float s_q[NREP][D];
 
@@ -132,7 +144,7 @@ void attn_int8_mfma_kernel(Int8Params a) {
     const bool chunk_sum = HCH && a.sel.mode == FQ_SELECT_PER_KV_HEAD_SUM;
     const int tid = threadIdx.x, L = lane_id(), w = __builtin_amdgcn_readfirstlane(wave_id());
     const int n16 = L & 15, lg = L >> 4;
-    WaveLds8& W = s_wave[w];
+    WaveLds8<D>& W = s_wave[w];
     const int S = c.S;
 
     // q: element tid of the group's heads, two branch-free 16-bit loads (the
@@ -150,11 +162,11 @@ void attn_int8_mfma_kernel(Int8Params a) {
     asm volatile("" : "+s"(hi_mask));
     uint32_t ql, qh, ql1 = 0u, qh1 = 0u;
     {
-        const char* qc = (const char*)q.q + (qb + (qi >> 7) * q.q_s[2] + (qi & 127) * q.q_s[3]) * esz;
+        const char* qc = (const char*)q.q + (qb + (qi / D) * q.q_s[2] + (qi % D) * q.q_s[3]) * esz;
         ql = *(const uint16_t*)qc;
         qh = *(const uint16_t*)(qc + esz - 2);
         if constexpr (HCH) {
-            const char* qc1 = (const char*)q.q + (qb + (qi1 >> 7) * q.q_s[2] + (qi1 & 127) * q.q_s[3]) * esz;
+            const char* qc1 = (const char*)q.q + (qb + (qi1 / D) * q.q_s[2] + (qi1 % D) * q.q_s[3]) * esz;
             ql1 = *(const uint16_t*)qc1;
             qh1 = *(const uint16_t*)(qc1 + esz - 2);
         }
@@ -163,13 +175,14 @@ void attn_int8_mfma_kernel(Int8Params a) {
     float ret_l = 0.f;
     ScoreRegs<NT> sr;
     ScoreRowRegs<NREP, NT> srow;        // kSelectOnly: the group's precomputed scores
-    const bool from_scores = FUSED && a.sel.enabled == kSelectOnly;
+    const bool from_scores = FUSED && (D == 64 || a.sel.enabled == kSelectOnly);
     const int score_rows = a.sel.mode == FQ_SELECT_PER_KV_HEAD_SUM ? 1 : NREP;
     // Partial-page tail (tail.in_kernel, split 0 of a group): its <= 64 raw
     // 16-bit K / V rows go to LDS with q.  The loads are unconditional: without
     // a tail the buffer is empty and they read 0.
     __shared__ uint16_t s_tk[TTOK][D], s_tv[TTOK][D];
     __shared__ float s_tp[NREP][TTOK];
+    constexpr int TCH = D / 8, TU = kTailMax * TCH / NT;     // 16-byte chunks of a tail row, per thread
     uint4 tkr[2], tvr[2];
     const int tail_T = FUSED && a.tail.in_kernel && split == 0 ? a.tail.len : 0;
     if constexpr (FUSED) {
@@ -183,15 +196,15 @@ void attn_int8_mfma_kernel(Int8Params a) {
         const auto rk = make_rsrc(tkb, tail_T > 0 ? 2 * (int64_t)(tail_T - 1) * t.ks[3] + 2 * D : 0);
         const auto rv = make_rsrc(tvb, tail_T > 0 ? 2 * (int64_t)(tail_T - 1) * t.vs[3] + 2 * D : 0);
 #pragma unroll
-        for (int u = 0; u < 2; ++u) {
-            const int i = tid + NT * u, tt = i >> 4, j = i & 15;       // token tt, bytes 16j .. 16j+15
+        for (int u = 0; u < TU; ++u) {
+            const int i = tid + NT * u, tt = i / TCH, j = i % TCH;     // token tt, bytes 16j .. 16j+15
             tkr[u] = ld128(rk, (int)(2 * tt * t.ks[3]) + 16 * j);
             tvr[u] = ld128(rv, (int)(2 * tt * t.vs[3]) + 16 * j);
         }
         if (from_scores)      // per_kv_head_sum with head chunks: the cache head's one summed row
             scores_load<NREP, NT>(srow, a.ws.scores + (int64_t)(chunk_sum ? g - (h - hk * HC) : g) * NREP * c.P,
                                   score_rows, c.P, tid);
-        else score_group_load<MT, NT>(sr, c, tid, l, b, hk);
+        else if constexpr (D == 128) score_group_load<MT, NT>(sr, c, tid, l, b, hk);
     }
     auto q_value = [&](uint32_t lo, uint32_t hi) {
         const uint32_t u = (lo & ~hi_mask) | ((hi << 16) & hi_mask);
@@ -201,15 +214,15 @@ void attn_int8_mfma_kernel(Int8Params a) {
     const float qv_raw = q_value(ql, qh);
 
     Int8Rsrc rs;
-    rs.k = make_rsrc(c.kp + l * c.kp_s[0] + b * c.kp_s[1] + hk * c.kp_s[2], (int64_t)S * 128);
-    rs.v = make_rsrc(c.vp + l * c.vp_s[0] + b * c.vp_s[1] + hk * c.vp_s[2], (int64_t)S * 128);
+    rs.k = make_rsrc(c.kp + l * c.kp_s[0] + b * c.kp_s[1] + hk * c.kp_s[2], (int64_t)S * D);
+    rs.v = make_rsrc(c.vp + l * c.vp_s[0] + b * c.vp_s[1] + hk * c.vp_s[2], (int64_t)S * D);
     rs.vs = make_rsrc((const uint16_t*)c.vsc + l * c.vsc_s[0] + b * c.vsc_s[1] + hk * c.vsc_s[2], (int64_t)S * 2);
     rs.vm = make_rsrc((const uint16_t*)c.vmn + l * c.vmn_s[0] + b * c.vmn_s[1] + hk * c.vmn_s[2], (int64_t)S * 2);
-    rs.ks = make_rsrc((const MT*)c.ksc + l * c.ksc_s[0] + b * c.ksc_s[1] + hk * c.ksc_s[2], (int64_t)c.P * 256);
-    rs.km = make_rsrc((const MT*)c.kmn + l * c.kmn_s[0] + b * c.kmn_s[1] + hk * c.kmn_s[2], (int64_t)c.P * 256);
+    rs.ks = make_rsrc((const MT*)c.ksc + l * c.ksc_s[0] + b * c.ksc_s[1] + hk * c.ksc_s[2], (int64_t)c.P * 2 * D);
+    rs.km = make_rsrc((const MT*)c.kmn + l * c.kmn_s[0] + b * c.kmn_s[1] + hk * c.kmn_s[2], (int64_t)c.P * 2 * D);
     auto issue_half = [&](HalfBuf& bf, int p, int hp) {
         __builtin_amdgcn_sched_barrier(0);
-        load_half(bf, rs, p, hp, n16, lg, L);
+        load_half<D>(bf, rs, p, hp, n16, lg, L);
         __builtin_amdgcn_sched_barrier(0);
     };
     HalfBuf b0, b1;
@@ -223,34 +236,36 @@ void attn_int8_mfma_kernel(Int8Params a) {
         if constexpr (HCH) {
             const float qv1 = q_value(ql1, qh1);
             if (tid < q_rows * D) {
-                const int r = (qi >> 7) - q_row0;
-                if ((unsigned)r < (unsigned)NREP) s_q[r][qi & 127] = qv_raw * q.qk_scale;
-                s_qraw[qi >> 7][qi & 127] = qv_raw;
+                const int r = (qi / D) - q_row0;
+                if ((unsigned)r < (unsigned)NREP) s_q[r][qi % D] = qv_raw * q.qk_scale;
+                s_qraw[qi / D][qi % D] = qv_raw;
             }
             if (tid + NT < q_rows * D) {
-                const int r = (qi1 >> 7) - q_row0;
-                if ((unsigned)r < (unsigned)NREP) s_q[r][qi1 & 127] = qv1 * q.qk_scale;
-                s_qraw[qi1 >> 7][qi1 & 127] = qv1;
+                const int r = (qi1 / D) - q_row0;
+                if ((unsigned)r < (unsigned)NREP) s_q[r][qi1 % D] = qv1 * q.qk_scale;
+                s_qraw[qi1 / D][qi1 % D] = qv1;
             }
         } else if (tid < NREP * D) {
-            s_q[qi >> 7][qi & 127] = qv_raw * q.qk_scale;
-            s_qraw[qi >> 7][qi & 127] = qv_raw;
+            s_q[qi / D][qi % D] = qv_raw * q.qk_scale;
+            s_qraw[qi / D][qi % D] = qv_raw;
         }
 #pragma unroll
-        for (int u = 0; u < 2; ++u) {
+        for (int u = 0; u < TU; ++u) {
             const int i = tid + NT * u;
-            *(uint4*)&s_tk[i >> 4][8 * (i & 15)] = tkr[u];
-            *(uint4*)&s_tv[i >> 4][8 * (i & 15)] = tvr[u];
+            *(uint4*)&s_tk[i / TCH][8 * (i % TCH)] = tkr[u];
+            *(uint4*)&s_tv[i / TCH][8 * (i % TCH)] = tvr[u];
         }
         __syncthreads();
         if (from_scores)     // uniform: a scoring launch wrote the group's scores
             scores_to_keys<NREP, NT>(srow, s_key, score_rows, c.P, tid);
-        else if (chunk_sum)
-            score_group_regs<MT, HCH ? 2 * NREP : NREP, NT, true>(sr, s_qraw, s_key, tid, c.P, 255.0f);
-        else if (a.sel.mode == FQ_SELECT_PER_KV_HEAD_SUM)
-            score_group_regs<MT, NREP, NT, true>(sr, s_qraw, s_key, tid, c.P, 255.0f);
-        else
-            score_group_regs<MT, NREP, NT, false>(sr, s_qraw, s_key, tid, c.P, 255.0f);
+        else if constexpr (D == 128) {
+            if (chunk_sum)
+                score_group_regs<MT, HCH ? 2 * NREP : NREP, NT, true>(sr, s_qraw, s_key, tid, c.P, 255.0f);
+            else if (a.sel.mode == FQ_SELECT_PER_KV_HEAD_SUM)
+                score_group_regs<MT, NREP, NT, true>(sr, s_qraw, s_key, tid, c.P, 255.0f);
+            else
+                score_group_regs<MT, NREP, NT, false>(sr, s_qraw, s_key, tid, c.P, 255.0f);
+        }
         const ForcedPages fp = forced_pages(c.P, a.sel.num_sinks, a.sel.window);
         if (S > 0 && split == 0 && w < fp.count) {       // split 0's first entries are the forced pages
             issue_half(b0, fp.page(w), 0);
@@ -269,17 +284,17 @@ void attn_int8_mfma_kernel(Int8Params a) {
         e0 = (int)((int64_t)n_sel * split / a.splits);
         e1 = (int)((int64_t)n_sel * (split + 1) / a.splits);
         for (int i = tid; i < e1 - e0; i += NT) s_ent[i] = a.ws.entries[(int64_t)g * c.P + e0 + i];
-        if (tid < NREP * D) s_q[qi >> 7][qi & 127] = qv_raw * q.qk_scale;
+        if (tid < NREP * D) s_q[qi / D][qi % D] = qv_raw * q.qk_scale;
         __syncthreads();
     }
     const int ent_base = FUSED ? e0 : 0;
     const int n_mine = S > 0 && w < e1 - e0 ? (e1 - e0 - w + NW - 1) / NW : 0;   // pages w, w + NW, ...
 
-    // A-operand values of this lane: channels c0 .. c0 + 3, heads r0, r0 + 1
-    const int c0 = 4 * (L & 31), r0 = 2 * (L >> 5);
-    float qv[2][4];
+    // A-operand values of this lane: channels c0 .. c0 + 3, heads r0, r0 + 1 (D = 64: r0)
+    const int c0 = 4 * (L % (D / 4)), r0 = QKS * (L / (D / 4));
+    float qv[QKS][4];
 #pragma unroll
-    for (int hh = 0; hh < 2; ++hh)
+    for (int hh = 0; hh < QKS; ++hh)
 #pragma unroll
         for (int j = 0; j < 4; ++j) qv[hh][j] = r0 + hh < NREP ? s_q[min(r0 + hh, NREP - 1)][c0 + j] : 0.f;
 
@@ -291,9 +306,9 @@ void attn_int8_mfma_kernel(Int8Params a) {
     for (int r = 0; r < NREP; ++r) m_run[r] = -INFINITY;
     float s_run = kBound ? 0.f : 1.f, inv_s = 1.f;
     float m_lane = 0.f;
-    v4f pacc[8];
+    v4f pacc[NTL];
 #pragma unroll
-    for (int t = 0; t < 8; ++t) pacc[t] = (v4f){0.f, 0.f, 0.f, 0.f};
+    for (int t = 0; t < NTL; ++t) pacc[t] = (v4f){0.f, 0.f, 0.f, 0.f};
     float l_acc = 0.f, bias = 0.f;
     float Cr = 0.f, unscale = 0.f;           // the current page's q.K_mn + 128 sum A (head lg), digit scale
 
@@ -315,13 +330,13 @@ void attn_int8_mfma_kernel(Int8Params a) {
             balance(k);
             // ---- the page's q.k A digits, q.K_mn and sum A per head
             const uint32_t sw[2] = {cb.ks.x, cb.ks.y}, mw[2] = {cb.km.x, cb.km.y};
-            float Av[2][4], cpart[2] = {0.f, 0.f}, apart[2] = {0.f, 0.f}, amax = 0.f;
+            float Av[QKS][4], cpart[2] = {0.f, 0.f}, apart[2] = {0.f, 0.f}, amax = 0.f;
 #pragma unroll
             for (int j = 0; j < 4; ++j) {
                 const float sf = half_to_f<MT>(sw[j >> 1] >> (16 * (j & 1)));
                 const float mf = half_to_f<MT>(mw[j >> 1] >> (16 * (j & 1)));
 #pragma unroll
-                for (int hh = 0; hh < 2; ++hh) {
+                for (int hh = 0; hh < QKS; ++hh) {
                     Av[hh][j] = qv[hh][j] * sf;
                     cpart[hh] = fmaf(qv[hh][j], mf, cpart[hh]);
                     apart[hh] += Av[hh][j];
@@ -332,7 +347,7 @@ void attn_int8_mfma_kernel(Int8Params a) {
             const float inv = sigma > 0.f ? kQkScale8 * __builtin_amdgcn_rcpf(sigma) : 0.f;
             const int s = c0 >> 6, kg = (c0 >> 4) & 3, bo = c0 & 15;
 #pragma unroll
-            for (int hh = 0; hh < 2; ++hh) {
+            for (int hh = 0; hh < QKS; ++hh) {
                 if (r0 + hh < NREP) {
                     uint32_t Y[4];
 #pragma unroll
@@ -343,27 +358,30 @@ void attn_int8_mfma_kernel(Int8Params a) {
                     *(uint32_t*)&W.aqk[s][row + 2][swz8(row + 2, kg)][bo] = byte_of4<0>(Y[0], Y[1], Y[2], Y[3]) ^ kFlip8;
                 }
                 float cs = fmaf(apart[hh], 128.0f, cpart[hh]);       // q.K_mn + 128 sum A over this lane's channels
-                cs += __shfl_xor(cs, 16, 64);
+                if constexpr (D == 128) cs += __shfl_xor(cs, 16, 64);
                 cpart[hh] = row_sum<16>(cs);
             }
-            const float x0 = __shfl(cpart[0], (lg >> 1) * 32, 64);
-            const float x1 = __shfl(cpart[1], (lg >> 1) * 32, 64);
-            Cr = (lg & 1) ? x1 : x0;
+            Cr = cpart[0];                   // D = 64: head lg is this lane group's own
+            if constexpr (D == 128) {
+                const float x0 = __shfl(cpart[0], (lg >> 1) * 32, 64);
+                const float x1 = __shfl(cpart[1], (lg >> 1) * 32, 64);
+                Cr = (lg & 1) ? x1 : x0;
+            }
             unscale = sigma * (1.0f / kQkScale8);
             __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
         }
         const v4i a0 = *(const v4i*)&W.aqk[0][n16][swz8(n16, lg)][0];
-        const v4i a1 = *(const v4i*)&W.aqk[1][n16][swz8(n16, lg)][0];
+        const v4i a1 = *(const v4i*)&W.aqk[QKS - 1][n16][swz8(n16, lg)][0];
         // ---- q.k of tiles T = 2 hp, 2 hp + 1
         float lg2[2], mp = -INFINITY;
 #pragma unroll
         for (int t = 0; t < 2; ++t) {
-            const uint4 k0 = cb.kt[t][0], k1 = cb.kt[t][1];
+            const uint4 k0 = cb.kt[t][0], k1 = cb.kt[t][QKS - 1];
             const v4i bk0 = {(int)(k0.x ^ kFlip8), (int)(k0.y ^ kFlip8), (int)(k0.z ^ kFlip8), (int)(k0.w ^ kFlip8)};
             const v4i bk1 = {(int)(k1.x ^ kFlip8), (int)(k1.y ^ kFlip8), (int)(k1.z ^ kFlip8), (int)(k1.w ^ kFlip8)};
             v4i acc = {0, 0, 0, 0};
             acc = __builtin_amdgcn_mfma_i32_16x16x64_i8(a0, bk0, acc, 0, 0, 0);
-            acc = __builtin_amdgcn_mfma_i32_16x16x64_i8(a1, bk1, acc, 0, 0, 0);
+            if constexpr (D == 128) acc = __builtin_amdgcn_mfma_i32_16x16x64_i8(a1, bk1, acc, 0, 0, 0);
             const float f = fmaf((float)acc[0], 65536.f, fmaf((float)acc[1], 256.f, (float)acc[2]));
             const float lgt = fmaf(f, unscale, Cr);
             const bool ok = lg < NREP && ((qm >> lg) & 1) && tok0 + 16 * t + n16 < S;
@@ -418,7 +436,7 @@ void attn_int8_mfma_kernel(Int8Params a) {
             for (int r = 0; r < 4; ++r) {
                 const float f = r < NREP ? am[r] * as : 0.f;
 #pragma unroll
-                for (int t = 0; t < 8; ++t) pacc[t][r] *= f;
+                for (int t = 0; t < NTL; ++t) pacc[t][r] *= f;
             }
         }
         // ---- p.v A: p * V_scale (/ s_run) in fp16; operand k = 8 kg + 2 ai + jj is
@@ -442,9 +460,9 @@ void attn_int8_mfma_kernel(Int8Params a) {
         }
         __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
         const v8h ap = *(const v8h*)&W.apv[n16][lg ^ ((n16 >> 2) & 3)][0];
-        // ---- p.v B: byte j of the lane's 8 channels for the step's 8 tokens, as fp16 subnormals
+        // ---- p.v B: byte j of the lane's NTL channels for the step's 8 tokens, as fp16 subnormals
 #pragma unroll
-        for (int j = 0; j < 8; ++j) {
+        for (int j = 0; j < NTL; ++j) {
             const uint32_t sel = 0x0C000C00u | ((4u + (j & 3)) << 16) | (uint32_t)(j & 3);
             uint32_t bw[4];
 #pragma unroll
@@ -484,10 +502,10 @@ void attn_int8_mfma_kernel(Int8Params a) {
         __builtin_amdgcn_s_setprio(0);
     }
 
-    // ---- wave state -> LDS (head r in lane group 0 component r; channel 8 n16 + j)
+    // ---- wave state -> LDS (head r in lane group 0 component r; channel NTL n16 + j)
     // the lo rows 4 + r (lane group 1) join the hi rows
 #pragma unroll
-    for (int j = 0; j < 8; ++j)
+    for (int j = 0; j < NTL; ++j)
 #pragma unroll
         for (int r = 0; r < NREP; ++r) pacc[j][r] += __shfl_xor(pacc[j][r], 16, 64);
     l_acc = row_sum<16>(l_acc);
@@ -499,7 +517,7 @@ void attn_int8_mfma_kernel(Int8Params a) {
         const float bb = __shfl(bias, 16 * r + n16, 64);
         if (lg == 0) {
 #pragma unroll
-            for (int j = 0; j < 8; ++j) s_split.acc[w][r][8 * n16 + j] = fmaf(pacc[j][r], pv_unscale, bb);
+            for (int j = 0; j < NTL; ++j) s_split.acc[w][r][NTL * n16 + j] = fmaf(pacc[j][r], pv_unscale, bb);
             if (n16 == 0) { s_split.m[w][r] = m_run[r]; s_split.l[w][r] = ll; }
         }
     }
@@ -512,20 +530,20 @@ void attn_int8_mfma_kernel(Int8Params a) {
                                                      a.splits > 1 || (a.tail.len > 0 && !a.tail.in_kernel), nslots);
 }
 
-template <typename MT, bool FUSED>
+template <int D, typename MT, bool FUSED>
 hipError_t launch_int8_nrep(const Int8Params& a, dim3 grid, hipStream_t st) {
     switch (a.q.nrep) {
 #define FQ_CASE(N)                                                                                      \
     case N:                                                                                             \
         timer_before_launch(st);                                                                        \
         if (FUSED && (N == 3 || N == 4) && a.sel.head_chunks > 1)                                       \
-            hipLaunchKernelGGL((attn_int8_mfma_kernel<MT, N, FUSED, FUSED && N >= 3>), grid, dim3(512), 0, \
+            hipLaunchKernelGGL((attn_int8_mfma_kernel<D, MT, N, FUSED, FUSED && N >= 3>), grid, dim3(512), 0, \
                                st, a);                                                                  \
         else                                                                                            \
-            hipLaunchKernelGGL((attn_int8_mfma_kernel<MT, N, FUSED>), grid, dim3(512), 0, st, a);       \
+            hipLaunchKernelGGL((attn_int8_mfma_kernel<D, MT, N, FUSED>), grid, dim3(512), 0, st, a);       \
         timer_after_launch(st);                                                                         \
         if (a.splits > 1 || (a.tail.len > 0 && !a.tail.in_kernel))                                      \
-            launch_split_merge<N, false>(a.q, a.ws, a.c.Hkv, a.c.B, grid.y, a.splits,                   \
+            launch_split_merge<N, false, D>(a.q, a.ws, a.c.Hkv, a.c.B, grid.y, a.splits,                   \
                                          a.tail.in_kernel ? TailArgs{} : a.tail, st);                    \
         break;
         FQ_CASE(1) FQ_CASE(2) FQ_CASE(3) FQ_CASE(4)
@@ -538,11 +556,11 @@ hipError_t launch_int8_nrep(const Int8Params& a, dim3 grid, hipStream_t st) {
 }  // namespace
 
 bool int8_mfma_supported(const Int4Cache& c, const QueryArgs& q, const AttnLaunch& al) {
-    if (c.bits != 8 || c.D != 128 || c.page != 64 || c.G != 1 || q.nrep > 4) return false;
+    if (c.bits != 8 || (c.D != 128 && c.D != 64) || c.page != 64 || c.G != 1 || q.nrep > 4) return false;
     if ((int64_t)al.s_max * kMaxWgPages < al.max_entries) return false;
-    // dense rows: 128-byte code rows, per-token V metadata, 128-channel K metadata rows
-    if (c.kp_s[3] != 128 || c.vp_s[3] != 128 || c.vsc_s[3] != 1 || c.vmn_s[3] != 1) return false;
-    if (c.ksc_s[3] != 128 || c.kmn_s[3] != 128) return false;
+    // dense rows: D-byte code rows, per-token V metadata, D-channel K metadata rows
+    if (c.kp_s[3] != c.D || c.vp_s[3] != c.D || c.vsc_s[3] != 1 || c.vmn_s[3] != 1) return false;
+    if (c.ksc_s[3] != c.D || c.kmn_s[3] != c.D) return false;
     for (int i = 0; i < 3; ++i) {
         if (c.kp_s[i] % 16 || c.vp_s[i] % 16 || c.ksc_s[i] % 8 || c.kmn_s[i] % 8) return false;
     }
@@ -576,14 +594,17 @@ hipError_t launch_attn_int8_mfma(const Int4Cache& c, const QueryArgs& q, const W
         a.sel = *sel;
         // split 0 of each group attends a 16-bit tail itself (16-byte aligned
         // rows, at least D apart); other tails are attended in the split merge
-        a.tail.in_kernel = mfma_tail_in_kernel(a.tail);
+        a.tail.in_kernel = mfma_tail_in_kernel(a.tail, c.D);
         // head chunks: a tail only inside the kernel (the split merge's tail
         // work indexes the cache by the virtual heads)
         if (a.sel.head_chunks > 1 && a.tail.len > 0 && !a.tail.in_kernel) return hipErrorInvalidValue;
     }
-    if (c.meta_dtype == FQ_BF16)
-        return fused ? launch_int8_nrep<bf16, true>(a, grid, st) : launch_int8_nrep<bf16, false>(a, grid, st);
-    return fused ? launch_int8_nrep<f16, true>(a, grid, st) : launch_int8_nrep<f16, false>(a, grid, st);
+    // head_dim 64: the tail inside the kernel or not at all (the split merge attends 128-channel tails)
+    if (c.D == 64 && a.tail.len > 0 && !a.tail.in_kernel) return hipErrorInvalidValue;
+#define FQ_W(D_, MT_) (fused ? launch_int8_nrep<D_, MT_, true>(a, grid, st) : launch_int8_nrep<D_, MT_, false>(a, grid, st))
+    if (c.D == 64) return c.meta_dtype == FQ_BF16 ? FQ_W(64, bf16) : FQ_W(64, f16);
+    return c.meta_dtype == FQ_BF16 ? FQ_W(128, bf16) : FQ_W(128, f16);
+#undef FQ_W
 }
 
 }  // namespace fq

@@ -1,7 +1,7 @@
 // Split-K sparse GQA decode attention over packed INT4 pages on the gfx950
 // matrix cores.  Same semantics as attn_int4.hip
 // (src/flashquest/kernel/sparse_int4_fwd.py:23-157); specialised for
-// head_dim 128, 64-token pages and up to 4 query heads per KV head.
+// head_dim 128 or 64, 64-token pages and up to 4 query heads per KV head.
 //
 // Why MFMA on a memory-bound GEMV: with 3 query heads per KV head every INT4
 // code feeds 3 multiply-adds for q.k and 3 for p.v, which is more fp32 VALU
@@ -56,8 +56,9 @@ struct MfmaParams {
 // A operands of one wave: [k-step][row][k-group, XOR-swizzled][16 bytes].
 // The k-group of row R is stored at position kg ^ ((R >> 2) & 3), which makes
 // the 16-byte operand reads (row = lane & 15, k-group = lane >> 4) conflict-free.
+template <int D>
 struct WaveLds {
-    uint8_t aqk[2][16][4][16];      // q.k: int8 digits, rows 4r + digit
+    uint8_t aqk[D / 64][16][4][16]; // q.k: int8 digits, rows 4r + digit
     uint8_t apv[2][16][4][16];      // p.v: fp16 hi parts, rows 4g + r (8 halves per k-group)
     uint8_t apl[2][16][4][16];      // p.v: fp16 lo parts, same layout
 };
@@ -79,14 +80,14 @@ constexpr uint32_t kDigitFlip = 0x80808080u;
 
 FQ_DEV void wave_lds_fence() { __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront"); }
 
-// Raw V metadata of one token: G halves (G = 4: 8 bytes, G = 1: 2 bytes).
+// Raw V metadata of one token: G halves (2 G bytes; G = 1, 2 or 4).
 struct VMetaRaw { uint2 v; };
 
 template <typename MT, int G>
 FQ_DEV void unpack_vmeta(const VMetaRaw& r, float (&out)[G]) {
     out[0] = half_to_f<MT>(r.v.x);
+    if constexpr (G >= 2) out[1] = half_to_f<MT>(r.v.x >> 16);
     if constexpr (G == 4) {
-        out[1] = half_to_f<MT>(r.v.x >> 16);
         out[2] = half_to_f<MT>(r.v.y);
         out[3] = half_to_f<MT>(r.v.y >> 16);
     }
@@ -106,28 +107,39 @@ FQ_DEV void load_vmeta(VMetaRaw (&m)[4], __amdgpu_buffer_rsrc_t r, int off) {
 #pragma unroll
     for (int T = 0; T < 4; ++T) {
         if constexpr (G == 4) m[T].v = ld64(r, off + T * 16 * 8);
+        else if constexpr (G == 2) m[T].v = make_uint2(ld32(r, off + T * 16 * 4), 0u);
         else m[T].v = make_uint2(ld16(r, off + T * 16 * 2), 0u);
     }
 }
 
 // Everything one page step reads.
 struct PageBuf {
-    uint4 kt[4];            // K codes: token 16T + n16, bytes 16*lg .. +15
+    uint4 kt[4];            // K codes: token 16T + n16, bytes 16*lg .. +15 (D = 64: 8*lg .. +7 in x, y)
     uint4 sv, mv;           // K scale / min: channels ch_base .. +7
-    uint32_t vw[16];        // V codes: token 16*(j&3) + 4*(j>>2) + lg, channels 8*n16 .. +7
+    uint32_t vw[16];        // V codes: token 16*(j&3) + 4*(j>>2) + lg, channels D/16*n16 .. (D = 64: the low 16 bits)
     VMetaRaw vs[4], vm[4];  // V scale / min of tokens 16T + n16
 };
 
-// koff: (token n16, byte 16*lg); voff: (token lg, byte 4*n16); moff: token n16's V
+// koff: (token n16, byte D/8*lg); voff: (token lg, byte D/32*n16); moff: token n16's V
 // metadata; soff: K scale / min channel ch_base.  All include the page part.
-template <int G>
+template <int D, int G>
 FQ_DEV void load_page(PageBuf& b, const SliceRsrc& r, int koff, int voff, int moff, int soff) {
 #pragma unroll
-    for (int T = 0; T < 4; ++T) b.kt[T] = ld128(r.k, koff + T * 16 * 64);
+    for (int T = 0; T < 4; ++T) {
+        if constexpr (D == 128) {
+            b.kt[T] = ld128(r.k, koff + T * 16 * 64);
+        } else {
+            const uint2 v = ld64(r.k, koff + T * 16 * 32);
+            b.kt[T] = make_uint4(v.x, v.y, 0u, 0u);
+        }
+    }
     b.sv = ld128(r.ks, soff);
     b.mv = ld128(r.km, soff);
 #pragma unroll
-    for (int j = 0; j < 16; ++j) b.vw[j] = ld32(r.v, voff + (16 * (j & 3) + 4 * (j >> 2)) * 64);
+    for (int j = 0; j < 16; ++j) {
+        const int t = 16 * (j & 3) + 4 * (j >> 2);
+        b.vw[j] = D == 128 ? ld32(r.v, voff + t * 64) : ld16(r.v, voff + t * 32);
+    }
     load_vmeta<G>(b.vs, r.vs, moff);
     load_vmeta<G>(b.vm, r.vm, moff);
 }
@@ -139,17 +151,30 @@ FQ_DEV void load_page(PageBuf& b, const SliceRsrc& r, int koff, int voff, int mo
 //
 // HCH (FUSED only): head chunks, sel.head_chunks virtual KV heads per cache
 // KV head (a separate instantiation, so the other kernels are unchanged).
-template <typename MT, int G, int NREP, int NW, bool FUSED, bool HCH = false>
+//
+// D = 64: the same page math with half the channels (one q.k step, four p.v
+// tiles).  Its FUSED form always selects from the scores of a scoring launch
+// (attend_from_scores): a page's 64-channel metadata is too little per
+// workgroup to be worth a second in-kernel scorer.  It replaces the VALU
+// kernel of attn_int4.hip, which is bound by its multiply-adds (59 us of a
+// 111 us step of 4 sequences x 16393 tokens, 32 / 8 heads, that also had to
+// attend the partial page in launches of its own; this way the step is 30 us,
+// most of it host time).
+template <int D, typename MT, int G, int NREP, int NW, bool FUSED, bool HCH = false>
 __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(2, 2)))
 void attn_int4_mfma_kernel(MfmaParams a) {
     static_assert(!FUSED || NW == 8, "in-kernel selection runs in the 8-wave kernel");
     static_assert(!HCH || FUSED, "head chunks run in the fused kernel");
-    constexpr int D = 128;
+    static_assert((D == 128 || D == 64) && (G == 1 || G == D / 32), "head_dim 128 / 64, per-token or 32-channel V groups");
     constexpr int NT = 64 * NW;
+    constexpr int QKS = D / 64;                     // q.k k-steps; also the query heads a lane makes digits for
+    constexpr int NTL = D / 16;                     // p.v channel tiles
+    constexpr int RB = D / 2;                       // bytes of a code row
+    constexpr bool kLoFree = 8 * G <= 16;           // p.v lo parts fit rows 4 G + .. of the hi parts' operand
     constexpr int NSLOT = FUSED ? NW + 1 : NW;      // the fused kernel's extra slot: the partial-page tail
     constexpr int TTOK = FUSED ? kTailMax : 1;
     __shared__ SplitLds<D, NREP, NSLOT> s_split;
-    __shared__ WaveLds s_wave[NW];
+    __shared__ WaveLds<D> s_wave[NW];
     __shared__ int s_ent[kMaxWgPages];
 
     const Int4Cache& c = a.c;
@@ -172,7 +197,7 @@ void attn_int4_mfma_kernel(MfmaParams a) {
     const bool chunk_sum = HCH && a.sel.mode == FQ_SELECT_PER_KV_HEAD_SUM;
     const int L = lane_id(), w = __builtin_amdgcn_readfirstlane(wave_id());
     const int n16 = L & 15, lg = L >> 4;
-    WaveLds& W = s_wave[w];
+    WaveLds<D>& W = s_wave[w];
     const int S = c.S;
 
     // Prologue: q (as prescaled fp32) and this split's page entries go to LDS.
@@ -204,8 +229,8 @@ void attn_int4_mfma_kernel(MfmaParams a) {
     uint32_t l0, h0, l1, h1;
     {
         const char* qc = (const char*)q.q;
-        const int64_t o0 = (qb + (i0 >> 7) * q.q_s[2] + (i0 & 127) * q.q_s[3]) * esz;
-        const int64_t o1 = (qb + (i1 >> 7) * q.q_s[2] + (i1 & 127) * q.q_s[3]) * esz;
+        const int64_t o0 = (qb + (i0 / D) * q.q_s[2] + (i0 % D) * q.q_s[3]) * esz;
+        const int64_t o1 = (qb + (i1 / D) * q.q_s[2] + (i1 % D) * q.q_s[3]) * esz;
         l0 = *(const uint16_t*)(qc + o0);
         h0 = *(const uint16_t*)(qc + o0 + esz - 2);
         l1 = *(const uint16_t*)(qc + o1);
@@ -217,9 +242,9 @@ void attn_int4_mfma_kernel(MfmaParams a) {
     // Needs 16-bit q with unit channel stride and 16-byte aligned rows; other
     // layouts (q_fast false: an empty buffer, the loads read 0) go through LDS.
     uint4 qsr[NREP];
-    const bool q_fast = FUSED && !chunk_sum && !q32 && !q.rot && q.q_s[3] == 1 && (q.q_s[2] & 7) == 0 &&
+    const bool q_fast = FUSED && D == 128 && !chunk_sum && !q32 && !q.rot && q.q_s[3] == 1 && (q.q_s[2] & 7) == 0 &&
                         (((uintptr_t)q.q + 2 * (uint64_t)qb) & 15) == 0;
-    if constexpr (FUSED) {
+    if constexpr (FUSED && D == 128) {
         const auto rq = make_rsrc((const char*)q.q + 2 * qb, q_fast ? 2 * ((int64_t)(NREP - 1) * q.q_s[2] + D) : 0);
 #pragma unroll
         for (int r = 0; r < NREP; ++r) qsr[r] = ld128(rq, (int)(2 * (r * q.q_s[2] + 8 * (tid & 15))));
@@ -228,8 +253,8 @@ void attn_int4_mfma_kernel(MfmaParams a) {
     // order, so one issued after the metadata loads would wait for all of them
     // and the scoring could not overlap the metadata's arrival.
     uint32_t rsg0 = 0u, rsg1 = 0u;
-    if constexpr (FUSED) {
-        const auto rr = make_rsrc(q.rot, q.rot && D == 128 ? 4 * D : 0);
+    if constexpr (FUSED && D == 128) {
+        const auto rr = make_rsrc(q.rot, q.rot ? 4 * D : 0);
         rsg0 = ld32(rr, 4 * L);
         rsg1 = ld32(rr, 4 * (L + 64));
     }
@@ -238,13 +263,14 @@ void attn_int4_mfma_kernel(MfmaParams a) {
     float ret_l = 0.f;
     ScoreRegs<NT> sr;
     ScoreRowRegs<NREP, NT> srow;        // kSelectOnly: the group's precomputed scores
-    const bool from_scores = FUSED && a.sel.enabled == kSelectOnly;
+    const bool from_scores = FUSED && (D == 64 || a.sel.enabled == kSelectOnly);
     const int score_rows = a.sel.mode == FQ_SELECT_PER_KV_HEAD_SUM ? 1 : NREP;
     // Partial-page tail (fused kernel, tail.in_kernel): its <= 64 raw 16-bit
     // K / V rows go to LDS with q, before scoring needs the metadata.  The
     // loads are unconditional: without a tail the buffer is empty and they read 0.
     __shared__ uint16_t s_tk[TTOK][D], s_tv[TTOK][D];
     __shared__ float s_tp[NREP][TTOK];
+    constexpr int TCH = D / 8, TU = kTailMax * TCH / 512;    // 16-byte chunks of a tail row, per thread
     uint4 tkr[2], tvr[2];
     const int tail_T = FUSED && a.tail.in_kernel && split == 0 ? a.tail.len : 0;   // split 0 of a group attends it
     if constexpr (FUSED) {
@@ -258,15 +284,15 @@ void attn_int4_mfma_kernel(MfmaParams a) {
         const auto rk = make_rsrc(tkb, tail_T > 0 ? 2 * (int64_t)(tail_T - 1) * t.ks[3] + 2 * D : 0);
         const auto rv = make_rsrc(tvb, tail_T > 0 ? 2 * (int64_t)(tail_T - 1) * t.vs[3] + 2 * D : 0);
 #pragma unroll
-        for (int u = 0; u < 2; ++u) {
-            const int i = tid + NT * u, tt = i >> 4, j = i & 15;       // token tt, bytes 16j .. 16j+15
+        for (int u = 0; u < TU; ++u) {
+            const int i = tid + NT * u, tt = i / TCH, j = i % TCH;     // token tt, bytes 16j .. 16j+15
             tkr[u] = ld128(rk, (int)(2 * tt * t.ks[3]) + 16 * j);
             tvr[u] = ld128(rv, (int)(2 * tt * t.vs[3]) + 16 * j);
         }
         if (from_scores)      // per_kv_head_sum with head chunks: the cache head's one summed row
             scores_load<NREP, NT>(srow, a.ws.scores + (int64_t)(chunk_sum ? g - (h - hk * HC) : g) * NREP * c.P,
                                   score_rows, c.P, tid);
-        else score_group_load<MT, NT>(sr, c, tid, l, b, hk);
+        else if constexpr (D == 128) score_group_load<MT, NT>(sr, c, tid, l, b, hk);
     }
     const bool qbf = q.q_dtype == FQ_BF16;
     auto q_float = [&](uint32_t u) {
@@ -285,23 +311,24 @@ void attn_int4_mfma_kernel(MfmaParams a) {
 
     // A-operand slot of this lane for the q.k digits: k-step qs_s, k-group qs_kg,
     // operand dword qs_jd; channels ch_base + 2b + par (b = 0..3); heads r0, r0+1.
-    const int Dq = L & 31, qs_s = Dq >> 4, qs_kg = (Dq >> 2) & 3, qs_jd = Dq & 3;
-    const int ch_base = 32 * qs_kg + 16 * qs_s + 8 * (qs_jd >> 1);
+    // (D = 64: one k-step, 16 lanes per head, head r0 alone.)
+    const int Dq = L & (16 * QKS - 1), qs_s = Dq >> 4, qs_kg = (Dq >> 2) & 3, qs_jd = Dq & 3;
+    const int ch_base = 16 * QKS * qs_kg + 16 * qs_s + 8 * (qs_jd >> 1);
     const int par = qs_jd & 1;
-    const int r0 = 2 * (L >> 5);
+    const int r0 = D == 128 ? 2 * (L >> 5) : L >> 4;
 
     SliceRsrc rs;
-    rs.k = make_rsrc(kb, (int64_t)S * 64);
-    rs.v = make_rsrc(vb, (int64_t)S * 64);
+    rs.k = make_rsrc(kb, (int64_t)S * RB);
+    rs.v = make_rsrc(vb, (int64_t)S * RB);
     rs.vs = make_rsrc(vsc, (int64_t)S * G * 2);
     rs.vm = make_rsrc(vmn, (int64_t)S * G * 2);
     rs.ks = make_rsrc(ksc, (int64_t)c.P * D * 2);
     rs.km = make_rsrc(kmn, (int64_t)c.P * D * 2);
-    const int koff0 = n16 * 64 + 16 * lg, voff0 = lg * 64 + 4 * n16, moff0 = n16 * G * 2, soff0 = ch_base * 2;
+    const int koff0 = n16 * RB + D / 8 * lg, voff0 = lg * RB + D / 32 * n16, moff0 = n16 * G * 2, soff0 = ch_base * 2;
     auto issue_page = [&](PageBuf& bf, int p) {
         // keep the scheduler from moving compute work in front of the loads
         __builtin_amdgcn_sched_barrier(0);
-        load_page<G>(bf, rs, koff0 + p * 4096, voff0 + p * 4096, moff0 + p * 64 * G * 2, soff0 + p * D * 2);
+        load_page<D, G>(bf, rs, koff0 + p * 64 * RB, voff0 + p * 64 * RB, moff0 + p * 64 * G * 2, soff0 + p * D * 2);
         __builtin_amdgcn_sched_barrier(0);
     };
     // Page buffers: one page in flight ahead of the one being computed.
@@ -321,32 +348,33 @@ void attn_int4_mfma_kernel(MfmaParams a) {
         {
             if (tid < q_rows * D) {
                 if constexpr (HCH) {
-                    const int r = (i0 >> 7) - q_row0;
-                    if ((unsigned)r < (unsigned)NREP) s_q[r][i0 & 127] = v0 * q.qk_scale;
+                    const int r = (i0 / D) - q_row0;
+                    if ((unsigned)r < (unsigned)NREP) s_q[r][i0 % D] = v0 * q.qk_scale;
                 } else {
-                    s_q[i0 >> 7][i0 & 127] = v0 * q.qk_scale;
+                    s_q[i0 / D][i0 % D] = v0 * q.qk_scale;
                 }
-                s_qraw[i0 >> 7][i0 & 127] = v0;
+                s_qraw[i0 / D][i0 % D] = v0;
             }
             if (tid + NT < q_rows * D) {
                 if constexpr (HCH) {
-                    const int r = (i1 >> 7) - q_row0;
-                    if ((unsigned)r < (unsigned)NREP) s_q[r][i1 & 127] = v1 * q.qk_scale;
+                    const int r = (i1 / D) - q_row0;
+                    if ((unsigned)r < (unsigned)NREP) s_q[r][i1 % D] = v1 * q.qk_scale;
                 } else {
-                    s_q[i1 >> 7][i1 & 127] = v1 * q.qk_scale;
+                    s_q[i1 / D][i1 % D] = v1 * q.qk_scale;
                 }
-                s_qraw[i1 >> 7][i1 & 127] = v1;
+                s_qraw[i1 / D][i1 % D] = v1;
             }
 #pragma unroll
-            for (int u = 0; u < 2; ++u) {
+            for (int u = 0; u < TU; ++u) {
                 const int i = tid + NT * u;
-                *(uint4*)&s_tk[i >> 4][8 * (i & 15)] = tkr[u];
-                *(uint4*)&s_tv[i >> 4][8 * (i & 15)] = tvr[u];
+                *(uint4*)&s_tk[i / TCH][8 * (i % TCH)] = tkr[u];
+                *(uint4*)&s_tv[i / TCH][8 * (i % TCH)] = tvr[u];
             }
             const bool sum = a.sel.mode == FQ_SELECT_PER_KV_HEAD_SUM;
             if (from_scores) {     // uniform: a scoring launch wrote the group's scores (never with q.rot)
                 scores_to_keys<NREP, NT>(srow, s_key, score_rows, c.P, tid);
-            } else if (q_fast) {      // uniform
+            } else if constexpr (D == 128) {
+            if (q_fast) {      // uniform
                 float qin[NREP][8];
 #pragma unroll
                 for (int r = 0; r < NREP; ++r) {
@@ -381,6 +409,7 @@ void attn_int4_mfma_kernel(MfmaParams a) {
                 } else if (sum) score_group_regs<MT, NREP, NT, true>(sr, s_qraw, s_key, tid, c.P);
                 else score_group_regs<MT, NREP, NT, false>(sr, s_qraw, s_key, tid, c.P);
             }
+            }
             const ForcedPages fp = forced_pages(c.P, a.sel.num_sinks, a.sel.window);
             if (S > 0 && split == 0 && w < fp.count) {       // split 0's first entries are the forced pages
                 issue_page(b0, fp.page(w));
@@ -408,17 +437,17 @@ void attn_int4_mfma_kernel(MfmaParams a) {
 #pragma unroll
         for (int u = 0; u < kEntPer; ++u)
             if (tid + u * NT < e1 - e0) s_ent[tid + u * NT] = ent[u];
-        if (tid < NREP * D) s_q[i0 >> 7][i0 & 127] = v0 * q.qk_scale;
-        if (tid + NT < NREP * D) s_q[i1 >> 7][i1 & 127] = v1 * q.qk_scale;
+        if (tid < NREP * D) s_q[i0 / D][i0 % D] = v0 * q.qk_scale;
+        if (tid + NT < NREP * D) s_q[i1 / D][i1 % D] = v1 * q.qk_scale;
         __syncthreads();
     }
     // Wave w takes entries w, w + NW, ... (a fixed assignment, so the fp32
     // accumulation order, and the result, do not depend on timing).
     const int n_mine = S > 0 && w < e1 - e0 ? (e1 - e0 - w + NW - 1) / NW : 0;   // pages w, w + NW, ...
 
-    float qv[2][4];
+    float qv[QKS][4];
 #pragma unroll
-    for (int hh = 0; hh < 2; ++hh)
+    for (int hh = 0; hh < QKS; ++hh)
 #pragma unroll
         for (int bb = 0; bb < 4; ++bb) qv[hh][bb] = r0 + hh < NREP ? s_q[min(r0 + hh, NREP - 1)][ch_base + 2 * bb + par] : 0.f;
 
@@ -437,9 +466,9 @@ void attn_int4_mfma_kernel(MfmaParams a) {
 #pragma unroll
     for (int gv = 0; gv < G; ++gv) { s_run[gv] = kBound ? 0.f : 1.f; inv_s[gv] = 1.f; }
     float m_lane = 0.f;                      // m_run[lg], or 0 while head lg has no logit yet
-    v4f pacc[8];                             // [tile]: component r = head, lane group lg = V group
+    v4f pacc[NTL];                           // [tile]: component r = head, lane group lg = V group
 #pragma unroll
-    for (int t = 0; t < 8; ++t) pacc[t] = (v4f){0.f, 0.f, 0.f, 0.f};
+    for (int t = 0; t < NTL; ++t) pacc[t] = (v4f){0.f, 0.f, 0.f, 0.f};
     float l_acc = 0.f, bias[G];              // head lg: sum p, sum p * V_mn[g] over this lane's tokens
 #pragma unroll
     for (int gv = 0; gv < G; ++gv) bias[gv] = 0.f;
@@ -469,13 +498,13 @@ void attn_int4_mfma_kernel(MfmaParams a) {
         // ---- q.k: digits of q * K_scale, then 2 MFMAs per 16-token tile
         const uint32_t sw[4] = {cb.sv.x, cb.sv.y, cb.sv.z, cb.sv.w};
         const uint32_t mw[4] = {cb.mv.x, cb.mv.y, cb.mv.z, cb.mv.w};
-        float A[2][4], cpart[2] = {0.f, 0.f}, amax = 0.f;
+        float A[QKS][4], cpart[2] = {0.f, 0.f}, amax = 0.f;
 #pragma unroll
         for (int bb = 0; bb < 4; ++bb) {
             const float sf = half_to_f<MT>(par ? sw[bb] >> 16 : sw[bb]);
             const float mf = half_to_f<MT>(par ? mw[bb] >> 16 : mw[bb]);
 #pragma unroll
-            for (int hh = 0; hh < 2; ++hh) {
+            for (int hh = 0; hh < QKS; ++hh) {
                 A[hh][bb] = qv[hh][bb] * sf;
                 cpart[hh] = fmaf(qv[hh][bb], mf, cpart[hh]);
                 amax = fmaxf(amax, fabsf(A[hh][bb]));
@@ -484,7 +513,7 @@ void attn_int4_mfma_kernel(MfmaParams a) {
         const float sigma = wave_max(amax);
         const float inv = sigma > 0.f ? kQkScale * __builtin_amdgcn_rcpf(sigma) : 0.f;
 #pragma unroll
-        for (int hh = 0; hh < 2; ++hh) {
+        for (int hh = 0; hh < QKS; ++hh) {
             if (r0 + hh < NREP) {
                 // Y = round(A * inv) + 0x808080, rounded by the fp32 add itself
                 uint32_t Y[4];
@@ -496,18 +525,20 @@ void attn_int4_mfma_kernel(MfmaParams a) {
                 dst[64 / 4] = byte_i<1>(Y[0], Y[1], Y[2], Y[3]) ^ kDigitFlip;      // row 4r+1: 256
                 dst[128 / 4] = byte_i<0>(Y[0], Y[1], Y[2], Y[3]) ^ kDigitFlip;     // row 4r+2: 1
             }
-            float cs = cpart[hh];            // sum over the 32 lanes of this half (heads r0 + hh)
-            cs += __shfl_xor(cs, 16, 64);
+            float cs = cpart[hh];            // sum over the 32 (D = 64: 16) lanes of head r0 + hh
+            if constexpr (D == 128) cs += __shfl_xor(cs, 16, 64);
             cpart[hh] = row_sum<16>(cs);
         }
-        // C for head lg lives in half lg >> 1, index lg & 1
-        const float c0 = __shfl(cpart[0], (lg >> 1) * 32, 64);
-        const float c1 = __shfl(cpart[1], (lg >> 1) * 32, 64);
-        const float Cr = (lg & 1) ? c1 : c0;
+        float Cr = cpart[0];                 // D = 64: head lg is this lane group's own
+        if constexpr (D == 128) {            // C for head lg lives in half lg >> 1, index lg & 1
+            const float c0 = __shfl(cpart[0], (lg >> 1) * 32, 64);
+            const float c1 = __shfl(cpart[1], (lg >> 1) * 32, 64);
+            Cr = (lg & 1) ? c1 : c0;
+        }
         const float unscale = sigma * (1.0f / kQkScale);
         wave_lds_fence();
         const v4i a0 = *(const v4i*)&W.aqk[0][n16][swz(n16, lg)][0];
-        const v4i a1 = *(const v4i*)&W.aqk[1][n16][swz(n16, lg)][0];
+        const v4i a1 = *(const v4i*)&W.aqk[QKS - 1][n16][swz(n16, lg)][0];
         float lg4[4], mp = -INFINITY;
 #pragma unroll
         for (int T = 0; T < 4; ++T) {
@@ -516,7 +547,7 @@ void attn_int4_mfma_kernel(MfmaParams a) {
             const v4i b1 = {(int)lo_nib(kt.z), (int)hi_nib(kt.z), (int)lo_nib(kt.w), (int)hi_nib(kt.w)};
             v4i acc = {0, 0, 0, 0};
             acc = __builtin_amdgcn_mfma_i32_16x16x64_i8(a0, b0, acc, 0, 0, 0);
-            acc = __builtin_amdgcn_mfma_i32_16x16x64_i8(a1, b1, acc, 0, 0, 0);
+            if constexpr (D == 128) acc = __builtin_amdgcn_mfma_i32_16x16x64_i8(a1, b1, acc, 0, 0, 0);
             const float f = fmaf((float)acc[0], 65536.f, fmaf((float)acc[1], 256.f, (float)acc[2]));
             const float lgt = fmaf(f, unscale, Cr);
             const bool ok = lg < NREP && ((qm >> lg) & 1) && tok0 + 16 * T + n16 < S;
@@ -577,7 +608,7 @@ void attn_int4_mfma_kernel(MfmaParams a) {
             float a_lg = as[0], am_lg = am[0];
             float ml = m_run[0];
 #pragma unroll
-            for (int gv = 1; gv < G; ++gv) a_lg = lg == gv ? as[gv] : a_lg;
+            for (int gv = 1; gv < G; ++gv) a_lg = (lg & (G - 1)) == gv ? as[gv] : a_lg;   // lo rows: lane groups G + g
 #pragma unroll
             for (int r = 1; r < NREP; ++r) {
                 am_lg = lg == r ? am[r] : am_lg;
@@ -591,7 +622,7 @@ void attn_int4_mfma_kernel(MfmaParams a) {
             for (int r = 0; r < 4; ++r) {
                 const float f = r < NREP ? am[r] * a_lg : 0.f;
 #pragma unroll
-                for (int t = 0; t < 8; ++t) pacc[t][r] *= f;
+                for (int t = 0; t < NTL; ++t) pacc[t][r] *= f;
             }
         }
 
@@ -623,8 +654,8 @@ void attn_int4_mfma_kernel(MfmaParams a) {
                     const h2v hv = __builtin_convertvector(av, h2v);
                     const h2v lv = __builtin_convertvector(av - __builtin_convertvector(hv, f2v), h2v);
                     *(uint32_t*)&W.apv[st][row][q][4 * (n16 >> 2)] = __builtin_bit_cast(uint32_t, hv);
-                    if constexpr (G == 1)        // rows 4..7 are free: lo in row 4 + r, same operand
-                        *(uint32_t*)&W.apv[st][row + 4][swz(row + 4, n16 & 3)][4 * (n16 >> 2)] =
+                    if constexpr (kLoFree)       // rows 4 G .. are free: lo in row 4 G + row, same operand
+                        *(uint32_t*)&W.apv[st][row + 4 * G][swz(row + 4 * G, n16 & 3)][4 * (n16 >> 2)] =
                             __builtin_bit_cast(uint32_t, lv);
                     else
                         *(uint32_t*)&W.apl[st][row][q][4 * (n16 >> 2)] = __builtin_bit_cast(uint32_t, lv);
@@ -634,8 +665,8 @@ void attn_int4_mfma_kernel(MfmaParams a) {
         wave_lds_fence();
         const v8h ap0 = *(const v8h*)&W.apv[0][n16][swz(n16, lg)][0];
         const v8h ap1 = *(const v8h*)&W.apv[1][n16][swz(n16, lg)][0];
-        v8h al0 = {}, al1 = {};          // used with G != 1 only
-        if constexpr (G != 1) {
+        v8h al0 = {}, al1 = {};          // used with every row taken (G = 4) only
+        if constexpr (!kLoFree) {
             al0 = *(const v8h*)&W.apl[0][n16][swz(n16, lg)][0];
             al1 = *(const v8h*)&W.apl[1][n16][swz(n16, lg)][0];
         }
@@ -647,7 +678,7 @@ void attn_int4_mfma_kernel(MfmaParams a) {
             nh[j] = hi_nib(cb.vw[j]);
         }
 #pragma unroll
-        for (int cc = 0; cc < 4; ++cc) {
+        for (int cc = 0; cc < D / 32; ++cc) {
             // bytes [cc of token j0, 0, cc of token j1, 0]
             const uint32_t sel = 0x0C000C00u | ((4u + cc) << 16) | (uint32_t)cc;
 #pragma unroll
@@ -664,7 +695,7 @@ void attn_int4_mfma_kernel(MfmaParams a) {
                 const v8h a = st ? ap1 : ap0, al = st ? al1 : al0;
                 pacc[2 * cc] = __builtin_amdgcn_mfma_f32_16x16x32_f16(a, blo, pacc[2 * cc], 0, 0, 0);
                 pacc[2 * cc + 1] = __builtin_amdgcn_mfma_f32_16x16x32_f16(a, bhi, pacc[2 * cc + 1], 0, 0, 0);
-                if constexpr (G != 1) {
+                if constexpr (!kLoFree) {
                     pacc[2 * cc] = __builtin_amdgcn_mfma_f32_16x16x32_f16(al, blo, pacc[2 * cc], 0, 0, 0);
                     pacc[2 * cc + 1] = __builtin_amdgcn_mfma_f32_16x16x32_f16(al, bhi, pacc[2 * cc + 1], 0, 0, 0);
                 }
@@ -697,16 +728,16 @@ void attn_int4_mfma_kernel(MfmaParams a) {
     }
 
     // ------------------------------------------------ wave state -> LDS
-    if constexpr (G == 1) {     // the lo rows 4 + r (lane group 1) join the hi rows
+    if constexpr (kLoFree) {    // the lo rows 4 G + .. (lane groups G + g) join the hi rows
 #pragma unroll
-        for (int t = 0; t < 8; ++t)
+        for (int t = 0; t < NTL; ++t)
 #pragma unroll
-            for (int r = 0; r < NREP; ++r) pacc[t][r] += __shfl_xor(pacc[t][r], 16, 64);
+            for (int r = 0; r < NREP; ++r) pacc[t][r] += __shfl_xor(pacc[t][r], 16 * G, 64);
     }
     l_acc = row_sum<16>(l_acc);
 #pragma unroll
     for (int gv = 0; gv < G; ++gv) bias[gv] = row_sum<16>(bias[gv]);
-    const int ug = G == 1 ? 0 : (n16 >> 2);      // channel group of this lane's columns
+    const int ug = n16 * G / 16;                 // channel group of this lane's columns
     float bsel = bias[0], ssel = s_run[0];
 #pragma unroll
     for (int gv = 1; gv < G; ++gv) {
@@ -720,8 +751,8 @@ void attn_int4_mfma_kernel(MfmaParams a) {
         const float bb = __shfl(bsel, src, 64);
         if (lg == ug) {
 #pragma unroll
-            for (int t = 0; t < 8; ++t) {
-                s_split.acc[w][r][8 * n16 + t] = fmaf(pacc[t][r], pv_unscale, bb);
+            for (int t = 0; t < NTL; ++t) {
+                s_split.acc[w][r][NTL * n16 + t] = fmaf(pacc[t][r], pv_unscale, bb);
             }
             if (n16 == 0) { s_split.m[w][r] = m_run[r]; s_split.l[w][r] = ll; }
         }
@@ -735,20 +766,20 @@ void attn_int4_mfma_kernel(MfmaParams a) {
                                                      a.splits > 1 || (a.tail.len > 0 && !a.tail.in_kernel), nslots);
 }
 
-template <typename MT, int G, int NW, bool FUSED>
+template <int D, typename MT, int G, int NW, bool FUSED>
 hipError_t launch_mfma_nrep(const MfmaParams& a, dim3 grid, hipStream_t st) {
     switch (a.q.nrep) {
 #define FQ_CASE(N)                                                                                     \
     case N:                                                                                            \
         timer_before_launch(st);                                                                       \
         if (FUSED && (N == 3 || N == 4) && a.sel.head_chunks > 1)                                      \
-            hipLaunchKernelGGL((attn_int4_mfma_kernel<MT, G, N, NW, FUSED, FUSED && N >= 3>), grid,       \
+            hipLaunchKernelGGL((attn_int4_mfma_kernel<D, MT, G, N, NW, FUSED, FUSED && N >= 3>), grid,    \
                                dim3(64 * NW), 0, st, a);                                               \
         else                                                                                           \
-            hipLaunchKernelGGL((attn_int4_mfma_kernel<MT, G, N, NW, FUSED>), grid, dim3(64 * NW), 0, st, a); \
+            hipLaunchKernelGGL((attn_int4_mfma_kernel<D, MT, G, N, NW, FUSED>), grid, dim3(64 * NW), 0, st, a); \
         timer_after_launch(st);                                                                        \
         if (a.splits > 1 || (a.tail.len > 0 && !a.tail.in_kernel))                                     \
-            launch_split_merge<N, false>(a.q, a.ws, a.c.Hkv, a.c.B, grid.y, a.splits,                  \
+            launch_split_merge<N, false, D>(a.q, a.ws, a.c.Hkv, a.c.B, grid.y, a.splits,                  \
                                          a.tail.in_kernel ? TailArgs{} : a.tail, st);                   \
         break;
         FQ_CASE(1) FQ_CASE(2) FQ_CASE(3) FQ_CASE(4)
@@ -788,17 +819,20 @@ int fused_splits(int groups, int max_entries, int s_max) {
 }  // namespace
 
 bool mfma_supported(const Int4Cache& c, const QueryArgs& q, const AttnLaunch& al) {
-    if (c.D != 128 || c.page != 64 || q.nrep > 4 || c.bits == 8) return false;
-    if (c.G != 1 && c.G != 4) return false;
+    if ((c.D != 128 && c.D != 64) || c.page != 64 || q.nrep > 4 || c.bits == 8) return false;
+    if (c.G != 1 && c.G != c.D / 32) return false;
     if ((int64_t)al.s_max * kMaxWgPages < al.max_entries) return false;
-    // contiguous 64-byte rows of codes, G-element rows of V metadata, 128-element
-    // rows of K metadata; 16-byte aligned code rows and 8-byte aligned metadata
-    if (c.kp_s[3] != 64 || c.vp_s[3] != 64 || c.vsc_s[3] != c.G || c.vmn_s[3] != c.G) return false;
-    if (c.ksc_s[3] != 128 || c.kmn_s[3] != 128) return false;
+    // contiguous D/2-byte rows of codes, G-element rows of V metadata, D-element
+    // rows of K metadata; 16-byte aligned slices of codes, 8-byte aligned metadata
+    if (c.kp_s[3] != c.D / 2 || c.vp_s[3] != c.D / 2 || c.vsc_s[3] != c.G || c.vmn_s[3] != c.G) return false;
+    if (c.ksc_s[3] != c.D || c.kmn_s[3] != c.D) return false;
     if (c.kp_s[2] % 16 || c.kp_s[1] % 16 || c.kp_s[0] % 16 || ((uintptr_t)c.kp & 15)) return false;
     if (c.vp_s[2] % 16 || c.vp_s[1] % 16 || c.vp_s[0] % 16 || ((uintptr_t)c.vp & 15)) return false;
     if (c.ksc_s[2] % 8 || c.ksc_s[1] % 8 || c.ksc_s[0] % 8 || ((uintptr_t)c.ksc & 15)) return false;
     if (c.kmn_s[2] % 8 || c.kmn_s[1] % 8 || c.kmn_s[0] % 8 || ((uintptr_t)c.kmn & 15)) return false;
+    if (c.G == 2 && (c.vsc_s[2] % 2 || c.vmn_s[2] % 2 || c.vsc_s[1] % 2 || c.vmn_s[1] % 2 || c.vsc_s[0] % 2 ||
+                     c.vmn_s[0] % 2 || ((uintptr_t)c.vsc & 3) || ((uintptr_t)c.vmn & 3)))
+        return false;
     if (c.G == 4 && (c.vsc_s[2] % 4 || c.vmn_s[2] % 4 || c.vsc_s[1] % 4 || c.vmn_s[1] % 4 || c.vsc_s[0] % 4 ||
                      c.vmn_s[0] % 4 || ((uintptr_t)c.vsc & 7) || ((uintptr_t)c.vmn & 7)))
         return false;
@@ -810,10 +844,10 @@ bool mfma_select_in_kernel(const Int4Cache& c, const QueryArgs& q, const AttnLau
            attention_splits_request() <= 0;
 }
 
-bool mfma_tail_in_kernel(const TailArgs& t) {
+bool mfma_tail_in_kernel(const TailArgs& t, int D) {
     const bool t16 = t.dtype == FQ_BF16 || t.dtype == FQ_F16;
     auto al16 = [](const int64_t* s) { return s[0] % 8 == 0 && s[1] % 8 == 0 && s[2] % 8 == 0 && s[3] % 8 == 0; };
-    return t.len > 0 && t16 && al16(t.ks) && al16(t.vs) && t.ks[3] >= 128 && t.vs[3] >= 128 &&
+    return t.len > 0 && t16 && al16(t.ks) && al16(t.vs) && t.ks[3] >= D && t.vs[3] >= D &&
            ((uintptr_t)t.k & 15) == 0 && ((uintptr_t)t.v & 15) == 0 &&
            2 * (int64_t)t.len * std::max(t.ks[3], t.vs[3]) < INT32_MAX;
 }
@@ -834,18 +868,24 @@ hipError_t launch_attn_int4_mfma(const Int4Cache& c, const QueryArgs& q, const W
         // least D apart): with one workgroup per group no merge launch follows,
         // with several, split 0 folds it into its partial and the merge has no
         // tail work left
-        a.tail.in_kernel = mfma_tail_in_kernel(a.tail);
+        a.tail.in_kernel = mfma_tail_in_kernel(a.tail, c.D);
         // head chunks: a tail only inside the kernel (the split merge's tail
         // work indexes the cache by the virtual heads)
         if (a.sel.head_chunks > 1 && a.tail.len > 0 && !a.tail.in_kernel) return hipErrorInvalidValue;
     }
+    // head_dim 64: the tail inside the kernel or not at all (the split merge attends 128-channel tails)
+    if (c.D == 64 && a.tail.len > 0 && !a.tail.in_kernel) return hipErrorInvalidValue;
     dim3 grid(a.splits, groups);
-#define FQ_W(MT_, G_)                                                                       \
-    (a.sel.enabled ? launch_mfma_nrep<MT_, G_, 8, true>(a, grid, st)                        \
-                   : sp.waves == 8 ? launch_mfma_nrep<MT_, G_, 8, false>(a, grid, st)       \
-                                   : launch_mfma_nrep<MT_, G_, 4, false>(a, grid, st))
-    if (c.meta_dtype == FQ_BF16) return c.G == 4 ? FQ_W(bf16, 4) : FQ_W(bf16, 1);
-    return c.G == 4 ? FQ_W(f16, 4) : FQ_W(f16, 1);
+#define FQ_W(D_, MT_, G_)                                                                       \
+    (a.sel.enabled ? launch_mfma_nrep<D_, MT_, G_, 8, true>(a, grid, st)                        \
+                   : sp.waves == 8 ? launch_mfma_nrep<D_, MT_, G_, 8, false>(a, grid, st)       \
+                                   : launch_mfma_nrep<D_, MT_, G_, 4, false>(a, grid, st))
+    if (c.D == 64) {
+        if (c.meta_dtype == FQ_BF16) return c.G == 2 ? FQ_W(64, bf16, 2) : FQ_W(64, bf16, 1);
+        return c.G == 2 ? FQ_W(64, f16, 2) : FQ_W(64, f16, 1);
+    }
+    if (c.meta_dtype == FQ_BF16) return c.G == 4 ? FQ_W(128, bf16, 4) : FQ_W(128, bf16, 1);
+    return c.G == 4 ? FQ_W(128, f16, 4) : FQ_W(128, f16, 1);
 #undef FQ_W
 }
 

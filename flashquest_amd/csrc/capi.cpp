@@ -428,8 +428,10 @@ static bool decode_selects_in_attention(const Int4Cache& c, const QueryArgs& q, 
 // Decode steps that split KV groups over several workgroups (too few groups
 // to fill the GPU) score each group once in a scoring launch over all CUs; the
 // attention workgroups then select from those scores (kSelectOnly) instead of
-// each re-scoring the group's pages.  INT4 and INT8, unrotated.
+// each re-scoring the group's pages.  INT4 and INT8, unrotated; with head_dim
+// 64 every such step (those kernels have no scorer of their own).
 static bool attend_from_scores(const Int4Cache& c, const QueryArgs& q, int bound) {
+    if (c.D == 64) return true;
     return c.L * c.B * c.Hkv < 192 && !q.rot && bound > kFusedSmallPages;
 }
 
@@ -445,7 +447,7 @@ static bool attend_from_scores(const Int4Cache& c, const QueryArgs& q, int bound
 static int mfma_head_chunks(Int4Cache& c, QueryArgs& q, int num_sinks, int window_pages, int k_max, int select_mode,
                             int s_max, const TailArgs* tail) {
     if ((c.bits != 4 && c.bits != 8) || q.rot || (q.nrep != 6 && q.nrep != 8)) return 1;
-    if (tail && tail->len > 0 && !mfma_tail_in_kernel(*tail)) return 1;
+    if (tail && tail->len > 0 && !mfma_tail_in_kernel(*tail, c.D)) return 1;
     Int4Cache c2 = c;
     QueryArgs q2 = q;
     c2.Hkv *= 2;
@@ -458,15 +460,19 @@ static int mfma_head_chunks(Int4Cache& c, QueryArgs& q, int num_sinks, int windo
     return 2;
 }
 
-static int quest_select(const fq_int4_cache* cache, const fq_query* query, const float* retention,
-                        int32_t num_sinks, int32_t window_pages, int32_t k_max, int32_t select_mode,
-                        float* scores_out, uint8_t* mask_out, void* workspace, size_t workspace_bytes_,
-                        fq_stream_t stream, int bits, bool mask_from_attention = false) {
-    Int4Cache c{};
-    QueryArgs q{};
-    Workspace ws{};
-    int st = attn_common(cache, query, workspace, workspace_bytes_, &c, &q, &ws, bits);
-    if (st) return st;
+// The parsed arguments of one decode step, shared by its two halves.
+struct DecodeStep {
+    Int4Cache c;
+    QueryArgs q;
+    Workspace ws;
+};
+
+static int quest_select(const DecodeStep& step, const float* retention, int32_t num_sinks, int32_t window_pages,
+                        int32_t k_max, int32_t select_mode, float* scores_out, uint8_t* mask_out, fq_stream_t stream,
+                        bool mask_from_attention = false) {
+    const Int4Cache& c = step.c;
+    const QueryArgs& q = step.q;
+    const Workspace& ws = step.ws;
     if (!retention) return fail(FQ_ERR_INVALID, "retention is NULL");
     if (select_mode != FQ_SELECT_PER_Q_HEAD && select_mode != FQ_SELECT_PER_KV_HEAD_SUM)
         return fail(FQ_ERR_INVALID, "select_mode=%d", select_mode);
@@ -499,6 +505,16 @@ static int quest_select(const fq_int4_cache* cache, const fq_query* query, const
                       "score+select");
 }
 
+static int quest_select(const fq_int4_cache* cache, const fq_query* query, const float* retention,
+                        int32_t num_sinks, int32_t window_pages, int32_t k_max, int32_t select_mode,
+                        float* scores_out, uint8_t* mask_out, void* workspace, size_t workspace_bytes_,
+                        fq_stream_t stream, int bits) {
+    DecodeStep s{};
+    const int st = attn_common(cache, query, workspace, workspace_bytes_, &s.c, &s.q, &s.ws, bits);
+    if (st) return st;
+    return quest_select(s, retention, num_sinks, window_pages, k_max, select_mode, scores_out, mask_out, stream);
+}
+
 int fq_quest_select_int4(const fq_int4_cache* cache, const fq_query* query, const float* retention,
                          int32_t num_sinks, int32_t window_pages, int32_t k_max, int32_t select_mode,
                          float* scores_out, uint8_t* mask_out, void* workspace, size_t workspace_bytes_,
@@ -507,15 +523,20 @@ int fq_quest_select_int4(const fq_int4_cache* cache, const fq_query* query, cons
                         workspace, workspace_bytes_, stream, 4);
 }
 
-static int quest_attend(const fq_int4_cache* cache, const fq_query* query, const float* retention, int32_t num_sinks,
-                        int32_t window_pages, int32_t k_max, int32_t select_mode, const TailArgs* tail,
-                        void* workspace, size_t workspace_bytes_, fq_stream_t stream, int bits = 4,
+// Whether the attention launch attends a partial-page tail: inside the
+// matrix-core kernel when it selects for itself, else (128 channels) in its
+// split merge.
+static bool tail_attended(const Int4Cache& c, const QueryArgs& q, const AttnLaunch& al, const TailArgs& t) {
+    if (!(c.bits == 8 ? int8_mfma_supported(c, q, al) : mfma_supported(c, q, al))) return false;
+    return c.D == 128 || (attn_selects_in_kernel(c, q, al) && mfma_tail_in_kernel(t, c.D));
+}
+
+static int quest_attend(const DecodeStep& step, const float* retention, int32_t num_sinks, int32_t window_pages,
+                        int32_t k_max, int32_t select_mode, const TailArgs* tail, fq_stream_t stream,
                         uint8_t* mask_out = nullptr) {
-    Int4Cache c{};
-    QueryArgs q{};
-    Workspace ws{};
-    int st = attn_common(cache, query, workspace, workspace_bytes_, &c, &q, &ws, bits);
-    if (st) return st;
+    Int4Cache c = step.c;
+    QueryArgs q = step.q;
+    const Workspace& ws = step.ws;
     if (!retention) return fail(FQ_ERR_INVALID, "retention is NULL");
     if (num_sinks < 0) num_sinks = 0;
     if (window_pages < 0) window_pages = 0;
@@ -523,7 +544,7 @@ static int quest_attend(const fq_int4_cache* cache, const fq_query* query, const
     const int chunks = mfma_head_chunks(c, q, num_sinks, window_pages, k_max, select_mode, ws.s_max, tail);
     const AttnLaunch al = choose_split(c.L * c.B * c.Hkv, quest_bound(c, q, num_sinks, window_pages, k_max,
                                                                       select_mode), ws.s_max);
-    if (tail && tail->len > 0 && !(bits == 8 ? int8_mfma_supported(c, q, al) : mfma_supported(c, q, al)))
+    if (tail && tail->len > 0 && !tail_attended(c, q, al, *tail))
         return fail(FQ_ERR_UNSUPPORTED, "the fused tail needs the matrix-core attention layout");
     SelectArgs sel{};
     if (q.rot && !attn_selects_in_kernel(c, q, al))
@@ -535,14 +556,16 @@ static int quest_attend(const fq_int4_cache* cache, const fq_query* query, const
         sel.head_chunks = chunks;
     }
     return hip_status(launch_attn_int4(c, q, ws, al, (hipStream_t)stream, &sel, tail),
-                      bits == 8 ? "sparse int8 attention" : "sparse int4 attention");
+                      c.bits == 8 ? "sparse int8 attention" : "sparse int4 attention");
 }
 
 int fq_quest_attend_int4(const fq_int4_cache* cache, const fq_query* query, const float* retention,
                          int32_t num_sinks, int32_t window_pages, int32_t k_max, int32_t select_mode,
                          void* workspace, size_t workspace_bytes_, fq_stream_t stream) {
-    return quest_attend(cache, query, retention, num_sinks, window_pages, k_max, select_mode, nullptr, workspace,
-                        workspace_bytes_, stream);
+    DecodeStep s{};
+    const int st = attn_common(cache, query, workspace, workspace_bytes_, &s.c, &s.q, &s.ws);
+    if (st) return st;
+    return quest_attend(s, retention, num_sinks, window_pages, k_max, select_mode, nullptr, stream);
 }
 
 // The partial-page tail of a decode step: validated here, attended by the
@@ -568,11 +591,22 @@ static int decode_with_tail(const fq_int4_cache* cache, const fq_query* query, c
     TailArgs t{};
     int st = check_tail(tail, cache, t);
     if (st) return st;
-    st = quest_select(cache, query, retention, num_sinks, window_pages, k_max, select_mode, nullptr, nullptr,
-                      workspace, workspace_bytes_, stream, bits);
+    DecodeStep s{};
+    st = attn_common(cache, query, workspace, workspace_bytes_, &s.c, &s.q, &s.ws, bits);
     if (st) return st;
-    return quest_attend(cache, query, retention, num_sinks, window_pages, k_max, select_mode, t.len > 0 ? &t : nullptr,
-                        workspace, workspace_bytes_, stream, bits);
+    if (t.len > 0) {       // refused before the selection is launched
+        Int4Cache c = s.c;
+        QueryArgs q = s.q;
+        const int sinks = std::max(num_sinks, 0), window = std::max(window_pages, 0), km = std::min(k_max, c.P);
+        mfma_head_chunks(c, q, sinks, window, km, select_mode, s.ws.s_max, &t);
+        const AttnLaunch al = choose_split(c.L * c.B * c.Hkv, quest_bound(c, q, sinks, window, km, select_mode),
+                                           s.ws.s_max);
+        if (!tail_attended(c, q, al, t))
+            return fail(FQ_ERR_UNSUPPORTED, "the fused tail needs the matrix-core attention layout");
+    }
+    st = quest_select(s, retention, num_sinks, window_pages, k_max, select_mode, nullptr, nullptr, stream);
+    if (st) return st;
+    return quest_attend(s, retention, num_sinks, window_pages, k_max, select_mode, t.len > 0 ? &t : nullptr, stream);
 }
 
 int fq_quest_decode_int4_tail(const fq_int4_cache* cache, const fq_query* query, const fq_tail* tail,
@@ -618,26 +652,31 @@ int fq_quest_fused_int8(const fq_int8_cache* cache, const fq_query* query, int32
     return quest_fused(cache, query, num_sinks, window_pages, k_max, select_mode, 8);
 }
 
+static int decode_step(const fq_int4_cache* cache, const fq_query* query, const float* retention, int32_t num_sinks,
+                       int32_t window_pages, int32_t k_max, int32_t select_mode, float* scores_out, uint8_t* mask_out,
+                       void* workspace, size_t workspace_bytes_, fq_stream_t stream, int bits) {
+    DecodeStep s{};
+    int st = attn_common(cache, query, workspace, workspace_bytes_, &s.c, &s.q, &s.ws, bits);
+    if (st) return st;
+    st = quest_select(s, retention, num_sinks, window_pages, k_max, select_mode, scores_out, mask_out, stream, true);
+    if (st) return st;
+    return quest_attend(s, retention, num_sinks, window_pages, k_max, select_mode, nullptr, stream, mask_out);
+}
+
 int fq_quest_decode_int4(const fq_int4_cache* cache, const fq_query* query, const float* retention,
                          int32_t num_sinks, int32_t window_pages, int32_t k_max, int32_t select_mode,
                          float* scores_out, uint8_t* mask_out, void* workspace, size_t workspace_bytes_,
                          fq_stream_t stream) {
-    int st = quest_select(cache, query, retention, num_sinks, window_pages, k_max, select_mode, scores_out, mask_out,
-                          workspace, workspace_bytes_, stream, 4, true);
-    if (st) return st;
-    return quest_attend(cache, query, retention, num_sinks, window_pages, k_max, select_mode, nullptr, workspace,
-                        workspace_bytes_, stream, 4, mask_out);
+    return decode_step(cache, query, retention, num_sinks, window_pages, k_max, select_mode, scores_out, mask_out,
+                       workspace, workspace_bytes_, stream, 4);
 }
 
 int fq_quest_decode_int8(const fq_int8_cache* cache, const fq_query* query, const float* retention,
                          int32_t num_sinks, int32_t window_pages, int32_t k_max, int32_t select_mode,
                          float* scores_out, uint8_t* mask_out, void* workspace, size_t workspace_bytes_,
                          fq_stream_t stream) {
-    int st = quest_select(cache, query, retention, num_sinks, window_pages, k_max, select_mode, scores_out, mask_out,
-                          workspace, workspace_bytes_, stream, 8, true);
-    if (st) return st;
-    return quest_attend(cache, query, retention, num_sinks, window_pages, k_max, select_mode, nullptr, workspace,
-                        workspace_bytes_, stream, 8, mask_out);
+    return decode_step(cache, query, retention, num_sinks, window_pages, k_max, select_mode, scores_out, mask_out,
+                       workspace, workspace_bytes_, stream, 8);
 }
 
 int fq_quest_select_int8(const fq_int8_cache* cache, const fq_query* query, const float* retention,

@@ -318,7 +318,7 @@ bool mfma_supported(const Int4Cache& c, const QueryArgs& q, const AttnLaunch& al
 bool mfma_select_in_kernel(const Int4Cache& c, const QueryArgs& q, const AttnLaunch& al);
 // The fused INT4 kernel attends a 16-bit partial-page tail itself (16-byte
 // aligned rows at least D apart).
-bool mfma_tail_in_kernel(const TailArgs& t);
+bool mfma_tail_in_kernel(const TailArgs& t, int D);
 // Page summary scores over the INT8 cache (summary.hip).
 struct SummaryArgs {
     const uint8_t* codes; int64_t c_s[4];          // (B, H_kv, S, D) bytes

@@ -57,7 +57,8 @@ _FUSED_TAIL_REFUSED = "the fused tail needs the matrix-core attention layout"
 def _tail_by_merge(run_sparse, Q3, O3, lse, K_tail, V_tail, sm_scale):
     """The reference's own partial-page sequence (llama_persistent_patch.py:
     232-245) for the shapes whose fused tail the library refuses (GQA ratios
-    above 4, head_dim 64, other page sizes): sparse attention over the
+    above 4, other page sizes, head_dim 64 with a float32 or unaligned tail or
+    past 512 pages): sparse attention over the
     completed pages into fp32 O and lse (run_sparse(O, lse)), then
     _bf16_dense_attn_with_lse over the tail (fp32 arithmetic, bf16 O, as
     there), then _merge_two_attentions (fp32, cast to O3's dtype)."""
