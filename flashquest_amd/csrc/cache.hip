@@ -7,11 +7,20 @@
 // One workgroup of 256 threads per (page, batch * head).  Thread t owns 8
 // channels (c8 = t % (D/8)) of tokens r, r + RPP, ... (r = t / (D/8)): every
 // load is 16 contiguous bytes and the D/8 threads of a token read one
-// contiguous row.  K: per-channel min/max over the page (lane shuffles, then
-// LDS across the 4 waves), scale arithmetic in the input dtype, codes by IEEE
-// fp32 division (the same operations as quant_k_kernel).  V: per-token,
+// contiguous row.  K: per-channel min/max over the page (lane swaps, then
+// LDS across the 4 waves), scale arithmetic in the input dtype, codes by
+// fp32 division (the values quant_k_kernel computes).  V: per-token,
 // per-group min/max over the group's lanes, fp32 arithmetic (as
 // quant_v_kernel).  Codes are stored 4 bytes (8 channels) per thread and token.
+//
+// A page has few bytes for its arithmetic: with an IEEE division per value
+// (about 12 instructions, some at a quarter of the rate) the kernel was bound by
+// its vector instructions and, in V, by one memory latency per token.  Every
+// load now goes out before the first use, reductions stay in the vector unit
+// (DPP, lane swaps) and the quotients come from one reciprocal per scale
+// (quot_code).  8192 tokens x 8 heads x 128 channels, INT4, back to back: K 12.6
+// -> 11.7 us, V 11.9 -> 10.7 us (21 MB each; what is left is one round of
+// workgroups: load latency, arithmetic and stores do not overlap).
 #include "fq_common.h"
 #include "turbo_quant.h"
 
@@ -71,12 +80,46 @@ FQ_DEV void load8(const TokSrc& s, int b, int h, int pos, int c8, float (&x)[8])
     }
 }
 
+// The codes of 8 values with their scales' reciprocals r = RN(1 / s):
+// rint(RN(d / s)) clamped, d = x - mn.  q0 = d r is within 1.5 ulp of d / s; one
+// residual correction brings it within one, and the second one rounds correctly
+// (Markstein: with y = RN(1 / b) and q within an ulp of a / b, RN(q + (a - b q) y)
+// is RN(a / b)), so ties round as the IEEE quotient's.  That holds while
+// nothing over- or underflows: quotients below 2^-100 round to 0 either way, and
+// scales above 1e30 (or NaN) take the division itself (quot_wide, per wave).
+// Scales are at least 1e-6.
 template <int BITS>
-FQ_DEV uint32_t codeq(float v, float mn, float s) {
-    float c = rintf(__fdiv_rn(v - mn, s));
-    c = fminf(fmaxf(c, 0.f), (float)((1 << BITS) - 1));
-    return (uint32_t)c;
+FQ_DEV uint32_t clamp_code(float q) {
+    return (uint32_t)fminf(fmaxf(rintf(q), 0.f), (float)((1 << BITS) - 1));
 }
+template <int BITS>
+FQ_DEV uint32_t quot_code(float d, float s, float r) {
+    const float q0 = d * r;
+    const float q1 = fmaf(fmaf(-q0, s, d), r, q0);
+    return clamp_code<BITS>(fmaf(fmaf(-q1, s, d), r, q1));
+}
+FQ_DEV bool quot_wide(bool ok) { return __builtin_amdgcn_ballot_w64(!ok) != 0; }   // any lane's scale out of range
+
+// min / max over the lanes with the same (lane & 15): rows 0..3 of the wave.
+template <bool MAX>
+FQ_DEV float mm(float a, float b) { return MAX ? fmaxf(a, b) : fminf(a, b); }
+template <bool MAX>
+FQ_DEV float across_rows(float v) {
+    const auto r = __builtin_amdgcn_permlane16_swap(__float_as_uint(v), __float_as_uint(v), false, false);
+    v = mm<MAX>(__uint_as_float(r[0]), __uint_as_float(r[1]));
+    const auto t = __builtin_amdgcn_permlane32_swap(__float_as_uint(v), __float_as_uint(v), false, false);
+    return mm<MAX>(__uint_as_float(t[0]), __uint_as_float(t[1]));
+}
+// min / max over each run of `n` lanes (1, 2, 4, 8 or 16; uniform).
+template <bool MAX>
+FQ_DEV float across_run(float v, int n) {
+    if (n > 1) v = mm<MAX>(v, dpp<kDppXor1>(v));
+    if (n > 2) v = mm<MAX>(v, dpp<kDppXor2>(v));
+    if (n > 4) v = mm<MAX>(v, dpp<kDppHalfMirror>(v));
+    if (n > 8) v = mm<MAX>(v, dpp<kDppMirror>(v));
+    return v;
+}
+constexpr int kDppRor8 = 0x128;      // lane i <- i ^ 8 within each 16
 
 // The 8 codes of a thread's channels: BITS 4 packs two per byte (4 bytes),
 // BITS 8 one per byte (8 bytes), at byte 8 * c8 * BITS / 8 of the row.
@@ -106,35 +149,37 @@ __global__ __launch_bounds__(kThreads) void page_quant_kernel(PageQuantParams a)
     const int c8 = tid % CPR, r = tid / CPR;
     const int bh = blockIdx.y, b = bh / a.H, h = bh % a.H;
     const int pg = blockIdx.x;
-    int pos[TPT];
+    // a partial last page: tokens past the end re-read the last one (the same
+    // page), which changes no minimum or maximum, and are not stored
+    int pos[TPT], lpos[TPT];
     bool ok[TPT];
 #pragma unroll
     for (int u = 0; u < TPT; ++u) {
         pos[u] = pg * kPage + r + RPP * u;
         ok[u] = pos[u] < a.n_tok;
+        lpos[u] = min(pos[u], a.n_tok - 1);
     }
 
     if (a.do_k) {
         float x[TPT][8];
         float mn[8], mx[8];
 #pragma unroll
+        for (int u = 0; u < TPT; ++u) load8(a.k, b, h, lpos[u], c8, x[u]);
+#pragma unroll
         for (int i = 0; i < 8; ++i) { mn[i] = INFINITY; mx[i] = -INFINITY; }
 #pragma unroll
-        for (int u = 0; u < TPT; ++u) {
-            if (ok[u]) {
-                load8(a.k, b, h, pos[u], c8, x[u]);
+        for (int u = 0; u < TPT; ++u)
 #pragma unroll
-                for (int i = 0; i < 8; ++i) { mn[i] = fminf(mn[i], x[u][i]); mx[i] = fmaxf(mx[i], x[u][i]); }
-            }
-        }
+            for (int i = 0; i < 8; ++i) { mn[i] = fminf(mn[i], x[u][i]); mx[i] = fmaxf(mx[i], x[u][i]); }
         // rows of this wave: lanes c8 + CPR * j
 #pragma unroll
-        for (int off = CPR; off < 64; off <<= 1) {
-#pragma unroll
-            for (int i = 0; i < 8; ++i) {
-                mn[i] = fminf(mn[i], __shfl_xor(mn[i], off, 64));
-                mx[i] = fmaxf(mx[i], __shfl_xor(mx[i], off, 64));
+        for (int i = 0; i < 8; ++i) {
+            if constexpr (CPR == 8) {
+                mn[i] = fminf(mn[i], dpp<kDppRor8>(mn[i]));
+                mx[i] = fmaxf(mx[i], dpp<kDppRor8>(mx[i]));
             }
+            mn[i] = across_rows<false>(mn[i]);
+            mx[i] = across_rows<true>(mx[i]);
         }
         __shared__ float s_red[kThreads / 64][CPR][16];
         const int w = tid >> 6;
@@ -174,12 +219,25 @@ __global__ __launch_bounds__(kThreads) void page_quant_kernel(PageQuantParams a)
                 make_uint4(mw[0], mw[1], mw[2], mw[3]);
         }
         if (a.k_codes) {
+            float rc[8];
+            bool fine = true;
+#pragma unroll
+            for (int i = 0; i < 8; ++i) {
+                rc[i] = __fdiv_rn(1.0f, sc[i]);
+                fine &= sc[i] <= 1e30f;
+            }
+            const bool wide = quot_wide(fine);
 #pragma unroll
             for (int u = 0; u < TPT; ++u) {
-                if (!ok[u]) continue;
                 uint32_t cd[8];
+                if (wide) {
 #pragma unroll
-                for (int i = 0; i < 8; ++i) cd[i] = codeq<BITS>(x[u][i], mn[i], sc[i]);
+                    for (int i = 0; i < 8; ++i) cd[i] = clamp_code<BITS>(__fdiv_rn(x[u][i] - mn[i], sc[i]));
+                } else {
+#pragma unroll
+                    for (int i = 0; i < 8; ++i) cd[i] = quot_code<BITS>(x[u][i] - mn[i], sc[i], rc[i]);
+                }
+                if (!ok[u]) continue;
                 store_codes<BITS>(a.kp + b * a.kp_s[0] + h * a.kp_s[1] + (int64_t)(a.tok_dst0 + pos[u]) * a.kp_s[2],
                                   c8, cd);
             }
@@ -189,33 +247,34 @@ __global__ __launch_bounds__(kThreads) void page_quant_kernel(PageQuantParams a)
     if (a.do_v) {
         const int lpg = a.v_group / 8;          // lanes per V group (a power of two <= CPR)
         const int g = (8 * c8) / a.v_group;
+        float x[TPT][8];
+#pragma unroll
+        for (int u = 0; u < TPT; ++u) load8(a.v, b, h, lpos[u], c8, x[u]);
 #pragma unroll
         for (int u = 0; u < TPT; ++u) {
-            // every lane of the row takes part in the shuffles; invalid tokens are not stored
-            float x[8];
-            if (ok[u]) load8(a.v, b, h, pos[u], c8, x);
-            else {
+            // every lane of the row takes part in the reductions; invalid tokens are not stored
+            float mn = x[u][0], mx = x[u][0];
 #pragma unroll
-                for (int i = 0; i < 8; ++i) x[i] = 0.f;
-            }
-            float mn = x[0], mx = x[0];
-#pragma unroll
-            for (int i = 1; i < 8; ++i) { mn = fminf(mn, x[i]); mx = fmaxf(mx, x[i]); }
-            for (int off = 1; off < lpg; off <<= 1) {
-                mn = fminf(mn, __shfl_xor(mn, off, 64));
-                mx = fmaxf(mx, __shfl_xor(mx, off, 64));
-            }
+            for (int i = 1; i < 8; ++i) { mn = fminf(mn, x[u][i]); mx = fmaxf(mx, x[u][i]); }
+            mn = across_run<false>(mn, lpg);
+            mx = across_run<true>(mx, lpg);
             // fp32 (kv_quant.py:189-205; INT8: 78-89)
             const float s = fmaxf((mx - mn) * (BITS == 8 ? kCacheInv255 : kCacheInv15), kCacheEps);
+            const float rc = __fdiv_rn(1.0f, s);
+            uint32_t cd[8];
+            if (quot_wide(s <= 1e30f)) {
+#pragma unroll
+                for (int i = 0; i < 8; ++i) cd[i] = clamp_code<BITS>(__fdiv_rn(x[u][i] - mn, s));
+            } else {
+#pragma unroll
+                for (int i = 0; i < 8; ++i) cd[i] = quot_code<BITS>(x[u][i] - mn, s, rc);
+            }
             if (!ok[u]) continue;
             const int64_t t = a.tok_dst0 + pos[u];
             if (c8 % lpg == 0) {
                 store_any(a.vs, a.meta_dtype, b * a.vs_s[0] + h * a.vs_s[1] + t * a.vs_s[2] + g, s);
                 store_any(a.vm, a.meta_dtype, b * a.vm_s[0] + h * a.vm_s[1] + t * a.vm_s[2] + g, mn);
             }
-            uint32_t cd[8];
-#pragma unroll
-            for (int i = 0; i < 8; ++i) cd[i] = codeq<BITS>(x[i], mn, s);
             store_codes<BITS>(a.vp + b * a.vp_s[0] + h * a.vp_s[1] + t * a.vp_s[2], c8, cd);
         }
     }
@@ -294,23 +353,25 @@ bool rows16(const void* p, const int64_t* s, int n, int esize) {
 
 }  // namespace
 
+// bits 4 / 8: a thread stores its 8 codes as 4 / 8 bytes, so that is the codes' alignment.
 bool page_quant_k_ok(int D, int page, int in_dtype, const void* k, const int64_t* k_s, const uint8_t* packed,
-                     const int64_t* p_s, const void* scale, const int64_t* s_s, const void* mn, const int64_t* m_s) {
+                     const int64_t* p_s, const void* scale, const int64_t* s_s, const void* mn, const int64_t* m_s,
+                     int bits) {
     if ((D != 64 && D != 128) || page != kPage) return false;
     const int es = in_dtype == FQ_F32 ? 4 : 2;
     if (k_s[3] != 1 || !rows16(k, k_s, 3, es)) return false;
-    if (p_s[3] != 1 || ((uintptr_t)packed & 3) || p_s[0] % 4 || p_s[1] % 4 || p_s[2] % 4) return false;
+    if (p_s[3] != 1 || ((uintptr_t)packed % bits) || p_s[0] % bits || p_s[1] % bits || p_s[2] % bits) return false;
     if (s_s[3] != 1 || m_s[3] != 1 || !rows16(scale, s_s, 3, 2) || !rows16(mn, m_s, 3, 2)) return false;
     return true;
 }
 
 bool page_quant_v_ok(int D, int group, int in_dtype, const void* v, const int64_t* v_s, const uint8_t* packed,
-                     const int64_t* p_s, const int64_t* s_s, const int64_t* m_s) {
+                     const int64_t* p_s, const int64_t* s_s, const int64_t* m_s, int bits) {
     if (D != 64 && D != 128) return false;
     if (group < 8 || group > D || (group & (group - 1))) return false;
     const int es = in_dtype == FQ_F32 ? 4 : 2;
     if (v_s[3] != 1 || !rows16(v, v_s, 3, es)) return false;
-    if (p_s[3] != 1 || ((uintptr_t)packed & 3) || p_s[0] % 4 || p_s[1] % 4 || p_s[2] % 4) return false;
+    if (p_s[3] != 1 || ((uintptr_t)packed % bits) || p_s[0] % bits || p_s[1] % bits || p_s[2] % bits) return false;
     if (D / group > 1 && (s_s[3] != 1 || m_s[3] != 1)) return false;
     return true;
 }
@@ -330,26 +391,26 @@ hipError_t launch_page_quant(const PageQuantParams& a, int D, hipStream_t st, in
 
 hipError_t launch_quant_k_pages(const void* k, int in_dtype, const int64_t* k_s, int B, int H, int S, int D,
                                 uint8_t* packed, const int64_t* p_s, void* scale, const int64_t* s_s, void* mn,
-                                const int64_t* m_s, int meta_dtype, hipStream_t st) {
+                                const int64_t* m_s, int meta_dtype, hipStream_t st, int bits) {
     PageQuantParams a{};
     a.k = TokSrc{nullptr, {0, 0, 0}, k, {k_s[0], k_s[1], k_s[2]}, 0, in_dtype};
     a.do_k = true; a.k_codes = true;
     a.B = B; a.H = H; a.n_tok = S; a.tok_dst0 = 0;
     for (int i = 0; i < 3; ++i) { a.kp_s[i] = p_s[i]; a.ks_s[i] = s_s[i]; a.km_s[i] = m_s[i]; }
     a.kp = packed; a.ks = scale; a.km = mn; a.meta_dtype = meta_dtype;
-    return launch_page_quant(a, D, st);
+    return launch_page_quant(a, D, st, bits);
 }
 
 hipError_t launch_quant_v_pages(const void* v, int in_dtype, const int64_t* v_s, int B, int H, int S, int D,
                                 int group, uint8_t* packed, const int64_t* p_s, void* scale, const int64_t* s_s,
-                                void* mn, const int64_t* m_s, int meta_dtype, hipStream_t st) {
+                                void* mn, const int64_t* m_s, int meta_dtype, hipStream_t st, int bits) {
     PageQuantParams a{};
     a.v = TokSrc{nullptr, {0, 0, 0}, v, {v_s[0], v_s[1], v_s[2]}, 0, in_dtype};
     a.do_v = true;
     a.B = B; a.H = H; a.n_tok = S; a.tok_dst0 = 0;
     for (int i = 0; i < 3; ++i) { a.vp_s[i] = p_s[i]; a.vs_s[i] = s_s[i]; a.vm_s[i] = m_s[i]; }
     a.vp = packed; a.vs = scale; a.vm = mn; a.v_group = group; a.meta_dtype = meta_dtype;
-    return launch_page_quant(a, D, st);
+    return launch_page_quant(a, D, st, bits);
 }
 
 // Stage the tokens that remain after the completed pages in the partial-page

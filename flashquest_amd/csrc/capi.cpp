@@ -792,6 +792,10 @@ int fq_quantize_k_int8(const void* k, int32_t in_dtype, const int64_t k_strides[
     if (D % 2) return fail(FQ_ERR_INVALID, "quantize_k requires even head_dim; got %d", D);
     if (page_size < 1) return fail(FQ_ERR_INVALID, "page_size must be >= 1");
     if (!is_float_dtype(in_dtype) || !is_half(meta_dtype)) return fail(FQ_ERR_INVALID, "dtype");
+    if (page_quant_k_ok(D, page_size, in_dtype, k, k_strides, codes, c_strides, scale, s_strides, mn, m_strides, 8))
+        return hip_status(launch_quant_k_pages(k, in_dtype, k_strides, B, H, S, D, codes, c_strides, scale, s_strides,
+                                               mn, m_strides, meta_dtype, (hipStream_t)stream, 8),
+                          "quantize k int8");
     return hip_status(launch_quant_k(k, in_dtype, k_strides, B, H, S, D, page_size, codes, c_strides, scale,
                                      s_strides, mn, m_strides, meta_dtype, (hipStream_t)stream, 8),
                       "quantize k int8");
@@ -803,6 +807,10 @@ int fq_quantize_v_int8(const void* v, int32_t in_dtype, const int64_t v_strides[
                        fq_stream_t stream) {
     if (D % 2) return fail(FQ_ERR_INVALID, "quantize_v requires even head_dim; got %d", D);
     if (!is_float_dtype(in_dtype) || !is_half(meta_dtype)) return fail(FQ_ERR_INVALID, "dtype");
+    if (page_quant_v_ok(D, D, in_dtype, v, v_strides, codes, c_strides, s_strides, m_strides, 8))
+        return hip_status(launch_quant_v_pages(v, in_dtype, v_strides, B, H, S, D, D, codes, c_strides, scale,
+                                               s_strides, mn, m_strides, meta_dtype, (hipStream_t)stream, 8),
+                          "quantize v int8");
     return hip_status(launch_quant_v(v, in_dtype, v_strides, B, H, S, D, D, codes, c_strides, scale, s_strides, mn,
                                      m_strides, meta_dtype, (hipStream_t)stream, 8),
                       "quantize v int8");
@@ -838,9 +846,9 @@ int fq_quantize_k_int4(const void* k, int32_t in_dtype, const int64_t k_strides[
     if (D % 2) return fail(FQ_ERR_INVALID, "quantize_k_int4 requires even head_dim; got %d", D);
     if (page_size < 1) return fail(FQ_ERR_INVALID, "page_size must be >= 1");
     if (!is_float_dtype(in_dtype) || !is_half(meta_dtype)) return fail(FQ_ERR_INVALID, "dtype");
-    if (page_quant_k_ok(D, page_size, in_dtype, k, k_strides, packed, p_strides, scale, s_strides, mn, m_strides))
+    if (page_quant_k_ok(D, page_size, in_dtype, k, k_strides, packed, p_strides, scale, s_strides, mn, m_strides, 4))
         return hip_status(launch_quant_k_pages(k, in_dtype, k_strides, B, H, S, D, packed, p_strides, scale, s_strides,
-                                               mn, m_strides, meta_dtype, (hipStream_t)stream),
+                                               mn, m_strides, meta_dtype, (hipStream_t)stream, 4),
                           "quantize k");
     return hip_status(launch_quant_k(k, in_dtype, k_strides, B, H, S, D, page_size, packed, p_strides, scale,
                                      s_strides, mn, m_strides, meta_dtype, (hipStream_t)stream),
@@ -854,9 +862,9 @@ int fq_quantize_v_int4(const void* v, int32_t in_dtype, const int64_t v_strides[
     if (D % 2) return fail(FQ_ERR_INVALID, "quantize_v_int4 requires even head_dim; got %d", D);
     if (group < 2 || group % 2 || D % group) return fail(FQ_ERR_INVALID, "bad V group %d for D=%d", group, D);
     if (!is_float_dtype(in_dtype) || !is_half(meta_dtype)) return fail(FQ_ERR_INVALID, "dtype");
-    if (page_quant_v_ok(D, group, in_dtype, v, v_strides, packed, p_strides, s_strides, m_strides))
+    if (page_quant_v_ok(D, group, in_dtype, v, v_strides, packed, p_strides, s_strides, m_strides, 4))
         return hip_status(launch_quant_v_pages(v, in_dtype, v_strides, B, H, S, D, group, packed, p_strides, scale,
-                                               s_strides, mn, m_strides, meta_dtype, (hipStream_t)stream),
+                                               s_strides, mn, m_strides, meta_dtype, (hipStream_t)stream, 4),
                           "quantize v");
     return hip_status(launch_quant_v(v, in_dtype, v_strides, B, H, S, D, group, packed, p_strides, scale,
                                      s_strides, mn, m_strides, meta_dtype, (hipStream_t)stream),
