@@ -288,6 +288,11 @@ def workspace(device: torch.device, nbytes: int, stream: int | None = None) -> t
     return buf
 
 
+def workspace_if_any(device: torch.device, stream: int) -> torch.Tensor | None:
+    """The scratch buffer of (device, stream) as it is, or None before the first workspace() there."""
+    return _ws.get((device.index, stream))
+
+
 class KernelTimer:
     """Times the sparse-attention kernels launched from this thread (HIP events
     around each launch, recorded by the library on the launch stream)."""

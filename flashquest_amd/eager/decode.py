@@ -12,6 +12,7 @@ import math
 
 import torch
 
+from .. import _host
 from .. import _lib as L
 from .. import _ops
 
@@ -49,6 +50,20 @@ def merge_two_attentions(O_a, lse_a, O_b, lse_b) -> torch.Tensor:
                                   out.stride(0), None, N, D, L.stream_handle(O_a.device)),
             "merge_two_attentions")
     return out.view(O_a.shape)
+
+
+def _native_decode(bits, Q, planes, H_kv, retention, head_pattern, num_sinks, window_pages, k_max_static, select_mode,
+                   page_size, sm_scale, return_lse, K_tail, V_tail):
+    """The step through the native host path: (O, lse), or None for the general way."""
+    host = _host.module()
+    H_q = Q.shape[-3]
+    if host is None or H_kv < 1 or H_q % H_kv:
+        return None
+    r, r_stride = _ops.retention_rows(retention, head_pattern, H_q, H_kv, Q.shape[0] if Q.dim() == 5 else 1, Q.device)
+    stream = L.stream_handle(Q.device)
+    return host.decode(bits, Q, planes, r, r_stride, int(num_sinks), int(window_pages),
+                       -1 if k_max_static is None else int(k_max_static), L.SELECT_MODES[select_mode], int(page_size),
+                       sm_scale, bool(return_lse), K_tail, V_tail, L.workspace_if_any(Q.device, stream), stream)
 
 
 _FUSED_TAIL_REFUSED = "the fused tail needs the matrix-core attention layout"
@@ -152,6 +167,12 @@ def quest_decode_int4(
     if D not in (64, 128):
         raise NotImplementedError(f"head_dim={D} not in (64, 128)")
     H_kv = K_scale.shape[-3]
+    if out is None and _rotation is None and not return_selection and not _direct:
+        res = _native_decode(4, Q, (K_packed, K_scale, K_mn, V_packed, V_scale, V_mn), H_kv, retention, head_pattern,
+                             num_sinks, window_pages, k_max_static, select_mode, page_size, sm_scale, return_lse,
+                             K_tail, V_tail)
+        if res is not None:
+            return res
     nrep = Q.shape[-3] // H_kv if Q.shape[-3] % H_kv == 0 else 0
     if (not _direct and _ops.wants_head_chunks(Q.shape[-3], H_kv, D, page_size) and _rotation is None
             and not _one_launch(4, Q, (K_packed, K_scale, K_mn, V_packed, V_scale, V_mn), nrep, page_size,
@@ -502,6 +523,12 @@ def quest_decode_int8(
     if D not in (64, 128):
         raise NotImplementedError(f"head_dim={D} not in (64, 128)")
     H_kv = K_scale.shape[-3]
+    if not return_selection and not _direct:
+        res = _native_decode(8, Q, (K_uint8, K_scale, K_mn, V_uint8, V_scale, V_mn), H_kv, retention, head_pattern,
+                             num_sinks, window_pages, k_max_static, select_mode, page_size, sm_scale, return_lse,
+                             K_tail, V_tail)
+        if res is not None:
+            return res
     nrep = Q.shape[-3] // H_kv if Q.shape[-3] % H_kv == 0 else 0
     if (not _direct and _ops.wants_head_chunks(Q.shape[-3], H_kv, D, page_size)
             and not _one_launch(8, Q, (K_uint8, K_scale, K_mn, V_uint8, V_scale, V_mn), nrep, page_size,
@@ -601,6 +628,12 @@ def quest_decode_turbo(
     if K_scale_raw.dtype != torch.bfloat16 or K_mn_raw.dtype != torch.bfloat16:
         raise AssertionError("K_scale_raw / K_mn_raw must be bf16")
     H_kv = K_msb.shape[-3]
+    if not return_selection and not _direct:
+        res = _native_decode(3, Q, (K_msb, K_lsb, K_scale_turbo, V_msb, V_lsb, V_scale_turbo, K_scale_raw, K_mn_raw),
+                             H_kv, retention, head_pattern, num_sinks, window_pages, k_max_static, select_mode,
+                             page_size, sm_scale, return_lse, None, None)
+        if res is not None:
+            return res
     nrep = Q.shape[-3] // H_kv if Q.shape[-3] % H_kv == 0 else 0
     if (not _direct and _ops.wants_head_chunks(Q.shape[-3], H_kv, D, page_size)
             and not _one_launch(3, Q, (K_msb, K_lsb, K_scale_turbo, V_msb, V_lsb, V_scale_turbo), nrep, page_size,

@@ -14,12 +14,22 @@ from __future__ import annotations
 
 import torch
 
+from .. import _host
 from .. import _lib as L
 
 # kv_quant.py:225-230 (identical K and V codebooks, K3-V3)
 K_TURBO_CODEBOOK = torch.tensor(
     [-2.1519, -1.3439, -0.7560, -0.2451, 0.2451, 0.7560, 1.3439, 2.1519], dtype=torch.float32)
 V_TURBO_CODEBOOK = K_TURBO_CODEBOOK.clone()
+
+
+def _native_quantize(is_v: bool, bits: int, X: torch.Tensor, unit: int, meta_dtype: torch.dtype):
+    """A quantiser that allocates its outputs, through the native host path
+    (unit: page size or V group); None for the general way."""
+    host = _host.module()
+    if host is None or not isinstance(unit, int):
+        return None
+    return host.quantize(int(is_v), bits, X, unit, L._DTYPES.get(meta_dtype, -1), L.stream_handle(X.device))
 
 
 def quantize_k(K: torch.Tensor, page_size: int, *, meta_dtype: torch.dtype = torch.bfloat16, out=None):
@@ -33,6 +43,9 @@ def quantize_k(K: torch.Tensor, page_size: int, *, meta_dtype: torch.dtype = tor
         raise ValueError(f"quantize_k requires even head_dim; got {D}")
     P = (S + page_size - 1) // page_size
     if out is None:
+        res = _native_quantize(False, 8, K, page_size, meta_dtype)
+        if res is not None:
+            return res
         codes = torch.empty(B, H, S, D, dtype=torch.uint8, device=K.device)
         scale = torch.empty(B, H, P, D, dtype=meta_dtype, device=K.device)
         mn = torch.empty(B, H, P, D, dtype=meta_dtype, device=K.device)
@@ -53,6 +66,9 @@ def quantize_v(V: torch.Tensor, *, meta_dtype: torch.dtype = torch.bfloat16, out
     if D % 2 != 0:
         raise ValueError(f"quantize_v requires even head_dim; got {D}")
     if out is None:
+        res = _native_quantize(True, 8, V, D, meta_dtype)
+        if res is not None:
+            return res
         codes = torch.empty(B, H, S, D, dtype=torch.uint8, device=V.device)
         scale = torch.empty(B, H, S, 1, dtype=meta_dtype, device=V.device)
         mn = torch.empty(B, H, S, 1, dtype=meta_dtype, device=V.device)
@@ -108,6 +124,9 @@ def quantize_k_int4(K: torch.Tensor, page_size: int, *, meta_dtype: torch.dtype 
         raise ValueError(f"quantize_k_int4 requires even head_dim; got {D}")
     P = (S + page_size - 1) // page_size
     if out is None:
+        res = _native_quantize(False, 4, K, page_size, meta_dtype)
+        if res is not None:
+            return res
         packed = torch.empty(B, H, S, D // 2, dtype=torch.uint8, device=K.device)
         scale = torch.empty(B, H, P, D, dtype=meta_dtype, device=K.device)
         mn = torch.empty(B, H, P, D, dtype=meta_dtype, device=K.device)
@@ -132,6 +151,9 @@ def quantize_v_int4(V: torch.Tensor, *, v_group: int | None = None,
     group = D if v_group is None else int(v_group)
     G = D // group
     if out is None:
+        res = _native_quantize(True, 4, V, group, meta_dtype)
+        if res is not None:
+            return res
         packed = torch.empty(B, H, S, D // 2, dtype=torch.uint8, device=V.device)
         scale = torch.empty(B, H, S, G, dtype=meta_dtype, device=V.device)
         mn = torch.empty(B, H, S, G, dtype=meta_dtype, device=V.device)

@@ -13,6 +13,7 @@ from __future__ import annotations
 
 import torch
 
+from .. import _host
 from .. import _lib as L
 from .. import _ops
 
@@ -52,6 +53,15 @@ def _prefill_call(fn_name: str, cache_desc, keep, q, K_tail, V_tail, causal_offs
     return out
 
 
+def _native_prefill(bits, q, planes, K_tail, V_tail, page_size, causal_offset, sm_scale):
+    """The call through the native host path, or None for the general way."""
+    host = _host.module() if q.is_cuda else None
+    if host is None:
+        return None
+    return host.prefill(bits, q, planes, K_tail, V_tail, int(page_size), int(causal_offset), sm_scale,
+                        L.stream_handle(q.device))
+
+
 def flash_attn_prefill_int4(q, K_packed, K_scale, K_mn, V_packed, V_scale, V_mn, K_tail=None, V_tail=None, *,
                             page_size: int = 64, causal_offset: int = 0, sm_scale: float | None = None):
     """Causal GQA attention of q (B, H_q, S_q, D) over one layer's packed INT4
@@ -59,6 +69,10 @@ def flash_attn_prefill_int4(q, K_packed, K_scale, K_mn, V_packed, V_scale, V_mn,
     (B, H_kv, T, D).  Query i attends keys j <= i + causal_offset
     (0 = torch's is_causal, as the reference's prefill call).  Returns bf16
     (B, H_q, S_q, D)."""
+    out = _native_prefill(4, q, (K_packed, K_scale, K_mn, V_packed, V_scale, V_mn), K_tail, V_tail, page_size,
+                          causal_offset, sm_scale)
+    if out is not None:
+        return out
     K_packed = _ops._ensure_inner_contiguous(K_packed, 8)   # one thread loads 8 code bytes
     c, keep = _ops.int4_cache(K_packed, K_scale, K_mn, V_packed, V_scale, V_mn, page_size)
     return _prefill_call("fq_prefill_int4", c, keep, q, K_tail, V_tail, causal_offset, sm_scale)
@@ -67,6 +81,10 @@ def flash_attn_prefill_int4(q, K_packed, K_scale, K_mn, V_packed, V_scale, V_mn,
 def flash_attn_prefill_int8(q, K_uint8, K_scale, K_mn, V_uint8, V_scale, V_mn, K_tail=None, V_tail=None, *,
                             page_size: int = 64, causal_offset: int = 0, sm_scale: float | None = None):
     """flash_attn_prefill_int4 over the INT8 cache (one code byte per channel)."""
+    out = _native_prefill(8, q, (K_uint8, K_scale, K_mn, V_uint8, V_scale, V_mn), K_tail, V_tail, page_size,
+                          causal_offset, sm_scale)
+    if out is not None:
+        return out
     K_uint8 = _ops._ensure_inner_contiguous(K_uint8, 16)
     c, keep = _ops.int8_cache(K_uint8, K_scale, K_mn, V_uint8, V_scale, V_mn, page_size)
     return _prefill_call("fq_prefill_int8", c, keep, q, K_tail, V_tail, causal_offset, sm_scale)

@@ -1,0 +1,97 @@
+"""The native host path gives what the general (ctypes) path gives, bit for bit,
+over the forms it takes, and leaves the others to it: layouts that need a copy,
+queries that are not contiguous, tensor subclasses."""
+import pytest
+import torch
+
+from flashquest_amd import _host
+from tests.cases import Int4Case, Int8Case
+
+pytestmark = pytest.mark.gpu
+
+
+def _both(monkeypatch, call):
+    assert _host.module() is not None, "the native host path is built with the library"
+    got = call()
+    with monkeypatch.context() as m:
+        m.setattr(_host, "_module", None)
+        want = call()
+    torch.cuda.synchronize()
+    for g, w in zip(got, want):
+        assert (g is None) == (w is None)
+        if g is not None:
+            assert type(g) is type(w) and g.shape == w.shape and g.stride() == w.stride() and g.dtype == w.dtype
+            assert torch.equal(g, w)
+
+
+def _planes(bits, room=0, layers=0):
+    case = (Int4Case if bits == 4 else Int8Case)(seed=5, B=2, Hq=6, Hkv=2, S=64 * 45)
+    keys = ("K_packed", "K_scale", "K_mn", "V_packed", "V_scale", "V_mn") if bits == 4 else \
+        ("K_uint8", "K_scale", "K_mn", "V_uint8", "V_scale", "V_mn")
+    d, out = case.device(), []
+    for k in keys:
+        t = torch.nn.functional.pad(d[k], (0, 0, 0, room))[:, :, :d[k].shape[2]]
+        out.append(torch.stack([t] * layers) if layers else t)
+    q = case.q_dev()
+    return (torch.stack([q] * layers) if layers else q), out
+
+
+class Sub(torch.Tensor):
+    pass
+
+
+@pytest.mark.parametrize("bits", [4, 8])
+@pytest.mark.parametrize("form", ["plain", "layers", "room", "tail", "no_lse", "q_strided", "q_subclass", "misaligned", "k_max"])
+def test_decode(monkeypatch, bits, form):
+    from flashquest_amd.eager.decode import quest_decode_int4, quest_decode_int8
+    q, planes = _planes(bits, room=3 if form == "room" else 0, layers=2 if form == "layers" else 0)
+    kw = dict(retention=0.3)
+    if form == "tail":
+        kw.update(K_tail=torch.randn(2, 2, 64, 128, device="cuda").bfloat16()[:, :, :11],
+                  V_tail=torch.randn(2, 2, 64, 128, device="cuda").bfloat16()[:, :, :11])
+    elif form == "no_lse":
+        kw["return_lse"] = False
+    elif form == "q_strided":
+        q = torch.stack([q, q], dim=-1)[..., 0]
+    elif form == "q_subclass":
+        q = q.as_subclass(Sub)
+    elif form == "misaligned":
+        flat = torch.empty(planes[0].numel() + 2, dtype=torch.uint8, device="cuda")
+        planes[0] = flat[2:].view(planes[0].shape).copy_(planes[0])
+    elif form == "k_max":
+        kw["k_max_static"] = 7
+    op = quest_decode_int4 if bits == 4 else quest_decode_int8
+    _both(monkeypatch, lambda: op(q, *planes, **kw))
+
+
+@pytest.mark.parametrize("bits", [4, 8])
+@pytest.mark.parametrize("tail,dtype", [(0, torch.bfloat16), (9, torch.bfloat16), (9, torch.float16)])
+def test_prefill(monkeypatch, bits, tail, dtype):
+    from flashquest_amd.kernel import flash_attn_prefill_int4, flash_attn_prefill_int8
+    _, planes = _planes(bits)
+    q = torch.randn(2, 6, 50, 128, device="cuda").to(dtype)
+    kt, vt = (torch.randn(2, 2, tail, 128, device="cuda").to(dtype) for _ in range(2))
+    op = flash_attn_prefill_int4 if bits == 4 else flash_attn_prefill_int8
+    _both(monkeypatch, lambda: (op(q, *planes, kt, vt, causal_offset=100),))
+
+
+@pytest.mark.parametrize("meta", [torch.bfloat16, torch.float16])
+def test_quantisers(monkeypatch, meta):
+    from flashquest_amd.kernel import quantize_k, quantize_k_int4, quantize_v, quantize_v_int4
+    x = torch.randn(2, 3, 130, 128, device="cuda").bfloat16()
+    for y in (x, x.transpose(0, 1), x[..., ::2]):
+        _both(monkeypatch, lambda: quantize_k_int4(y, 64, meta_dtype=meta) + quantize_v_int4(y, meta_dtype=meta) +
+              quantize_v_int4(y, v_group=32, meta_dtype=meta) + quantize_k(y, 64, meta_dtype=meta) +
+              quantize_v(y, meta_dtype=meta))
+
+
+def test_errors_are_the_general_paths():
+    from flashquest_amd.eager.decode import quest_decode_int4
+    from flashquest_amd.kernel import quantize_k_int4
+    q, planes = _planes(4)
+    with pytest.raises(ValueError):
+        quest_decode_int4(q, *planes, retention=1.5)
+    with pytest.raises(AssertionError):
+        quest_decode_int4(q, *planes[:2], planes[2].half(), *planes[3:], retention=0.3)
+    with pytest.raises(ValueError):
+        quantize_k_int4(torch.zeros(1, 1, 64, 63, device="cuda").bfloat16(), 64)
