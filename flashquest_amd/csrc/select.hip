@@ -365,26 +365,40 @@ __global__ __launch_bounds__(kThreads) void select_groups_rows_kernel(GroupSelec
 }
 
 // ---------------------------------------------------------------------------
-// The same selection for few groups (a single layer's decode step): one
-// 8-wave workgroup per group runs the in-LDS selection of the fused decode
-// (block_select_group), so the group's rows are searched by 8 waves instead of
-// one.  P <= 64 kSelC.  The list puts the forced pages first.
+// The same selection with an 8-wave workgroup per group, which runs the in-LDS
+// selection of the fused decode (block_select_group): the group's rows are
+// searched and listed by 8 waves instead of one.  For few groups (a single
+// layer's decode step) and for long contexts; P <= 64 C.  The list puts the
+// forced pages first.  A wave alone spends the time on its own LDS counts and
+// lists: scoring and selection of 224 groups x 2048 pages with 3 query heads each,
+// 95.0 -> 72.3 us per query head and 59.6 -> 55.7 from one summed row; 1024
+// pages 42.4 -> 40.6 per query head.
 // ---------------------------------------------------------------------------
-template <int NREP>
+template <int NREP, int C>
 __global__ __launch_bounds__(512) void select_groups_block_kernel(GroupSelectParams a) {
-    constexpr int NT = 512, NW = 8;
-    __shared__ uint32_t s_key[NREP * 64 * kSelC];
+    constexpr int NT = 512, NW = 8, KN = NREP * 64 * C / NT;
+    static_assert(64 * C % NT == 0, "a thread's pages are the same in every row");
+    __shared__ uint32_t s_key[NREP * 64 * C];
     __shared__ BlockSelectLds s_bsel;
-    __shared__ int s_ent[64 * kSelC];
+    __shared__ int s_ent[64 * C];
     const int g = blockIdx.x, tid = threadIdx.x, P = a.P;
     const int rows = a.mode == FQ_SELECT_PER_KV_HEAD_SUM ? 1 : NREP;
-    ScoreRowRegs<NREP, NT> srow;
-    scores_load<NREP, NT>(srow, a.ws.scores + (int64_t)g * NREP * P, rows, P, tid);
+    const float* sc = a.ws.scores + (int64_t)g * NREP * P;
+    float v[KN];
+#pragma unroll
+    for (int u = 0; u < KN; ++u) {        // every load before the first use
+        const int i = tid + u * NT, r = i / (64 * C), p = i % (64 * C);
+        v[u] = sc[min(r, rows - 1) * P + min(p, P - 1)];
+    }
     const float ret_l = group_retention(a, g)[min(lane_id(), NREP - 1)];     // lane r: head r's retention
-    scores_to_keys<NREP, NT>(srow, s_key, rows, P, tid);
+#pragma unroll
+    for (int u = 0; u < KN; ++u) {
+        const int i = tid + u * NT, r = i / (64 * C), p = i % (64 * C);
+        if (r < rows) s_key[i] = p < P ? sortable_key(v[u]) : 0u;
+    }
     __syncthreads();
-    const int n = block_select_group<kSelC, NW, NREP>(s_key, P, a.mode, ret_l, a.k_max, a.num_sinks, a.window, s_ent,
-                                                      s_bsel);
+    const int n = block_select_group<C, NW, NREP>(s_key, P, a.mode, ret_l, a.k_max, a.num_sinks, a.window, s_ent,
+                                                  s_bsel);
     int* entries = a.ws.entries + (int64_t)g * P;
     for (int i = tid; i < n; i += NT) entries[i] = s_ent[i];
     if (a.mask_out)       // uniform; the keys are no longer needed: their LDS is the scratch
@@ -505,10 +519,15 @@ hipError_t launch_score(const Int4Cache& c, const QueryArgs& q, int S_q, const i
     a.scores = scores;
     if (sc4_s) for (int i = 0; i < 4; ++i) a.sc_s[i] = sc4_s[i];
     const int G = c.L * c.B * c.Hkv;
-    // pages per chunk: about two workgroups per CU in one pass over the GPU,
-    // each streaming a whole number of passes of ppp pages
+    // pages per chunk, a whole number of passes of ppp pages: kPasses of them
+    // (what a workgroup keeps in flight at once), fewer where that leaves less
+    // than two workgroups per CU.  With longer chunks the workgroups run out of
+    // step and the last round of the CUs is partly empty: 2048 pages x 224
+    // groups scored and selected in 82 us with 688-page chunks, 66.6 / 63.5 /
+    // 59.6 us with 208 / 112 / 64; 1024 pages 50.8 -> 42.4 us with 64, and 50.7
+    // with 32.
     const int ppp = kThreads / (c.D / 8);
-    int target_chunks = (512 + G - 1) / G;
+    int target_chunks = std::max((512 + G - 1) / G, (c.P + kPasses * ppp - 1) / (kPasses * ppp));
     int ppc = (c.P + target_chunks - 1) / target_chunks;
     ppc = ((ppc + ppp - 1) / ppp) * ppp;
     if (ppc < ppp) ppc = ppp;
@@ -543,13 +562,19 @@ hipError_t launch_score(const Int4Cache& c, const QueryArgs& q, int S_q, const i
 #undef FQ_SCORE
     hipError_t e = hipGetLastError();
     if (e != hipSuccess || !ws || !select_groups) return e;
-    if (G < 192 && c.P <= 64 * kSelC && q.nrep <= 4) {     // few groups: a workgroup per group
-        switch (q.nrep) {
-            case 1: hipLaunchKernelGGL(select_groups_block_kernel<1>, dim3(G), dim3(512), 0, st, sp); break;
-            case 2: hipLaunchKernelGGL(select_groups_block_kernel<2>, dim3(G), dim3(512), 0, st, sp); break;
-            case 3: hipLaunchKernelGGL(select_groups_block_kernel<3>, dim3(G), dim3(512), 0, st, sp); break;
-            default: hipLaunchKernelGGL(select_groups_block_kernel<4>, dim3(G), dim3(512), 0, st, sp); break;
-        }
+#define FQ_BLOCK(C_)                                                                                                   \
+    switch (q.nrep) {                                                                                                  \
+        case 1: hipLaunchKernelGGL((select_groups_block_kernel<1, C_>), dim3(G), dim3(512), 0, st, sp); break;         \
+        case 2: hipLaunchKernelGGL((select_groups_block_kernel<2, C_>), dim3(G), dim3(512), 0, st, sp); break;         \
+        case 3: hipLaunchKernelGGL((select_groups_block_kernel<3, C_>), dim3(G), dim3(512), 0, st, sp); break;         \
+        default: hipLaunchKernelGGL((select_groups_block_kernel<4, C_>), dim3(G), dim3(512), 0, st, sp); break;        \
+    }
+    if (q.nrep <= 4 && c.P > 64 * 16 && c.P <= 64 * 32) {
+        FQ_BLOCK(32)
+    } else if (q.nrep <= 4 && c.P > 64 * kSelC && c.P <= 64 * 16) {
+        FQ_BLOCK(16)
+    } else if (q.nrep <= 4 && G < 192 && c.P <= 64 * kSelC) {     // few groups
+        FQ_BLOCK(kSelC)
     } else if (c.P > 64 * 8 && c.P <= 64 * 32 && q.nrep > 1 && select_mode == FQ_SELECT_PER_Q_HEAD) {
         if (c.P <= 64 * 16) hipLaunchKernelGGL(select_groups_rows_kernel<16>, dim3(G), dim3(kThreads), 0, st, sp);
         else hipLaunchKernelGGL(select_groups_rows_kernel<32>, dim3(G), dim3(kThreads), 0, st, sp);
@@ -558,6 +583,7 @@ hipError_t launch_score(const Int4Cache& c, const QueryArgs& q, int S_q, const i
     else if (c.P <= 64 * 16) hipLaunchKernelGGL(select_groups_wave_kernel<16>, dim3(G), dim3(64), 0, st, sp, G);
     else if (c.P <= 64 * 32) hipLaunchKernelGGL(select_groups_wave_kernel<32>, dim3(G), dim3(64), 0, st, sp, G);
     else hipLaunchKernelGGL(select_groups_kernel, dim3(G), dim3(kThreads), 0, st, sp);
+#undef FQ_BLOCK
     return hipGetLastError();
 }
 
