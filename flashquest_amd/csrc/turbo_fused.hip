@@ -21,8 +21,33 @@
 namespace fq {
 namespace {
 
-__device__ __constant__ float kTurboCodebookF[8] = {-2.1519f, -1.3439f, -0.7560f, -0.2451f,
-                                                    0.2451f, 0.7560f, 1.3439f, 2.1519f};
+// The codebook is whole in units of 1e-4 (+-2451, 7560, 13439, 21519; its fp32
+// values differ from those by their own rounding), and each value is 256 H + L
+// with two int8 digits: byte tables for v_perm, codes 0-3 and 4-7.
+constexpr int kTurboInt[8] = {-21519, -13439, -7560, -2451, 2451, 7560, 13439, 21519};
+constexpr float kTurboUnit = 1e-4f;
+constexpr int turbo_low(int v) { return v - 256 * ((v + 32768 + 128) / 256 - 128); }     // in [-128, 127]
+constexpr uint32_t turbo_table(bool high, int first) {
+    uint32_t t = 0;
+    for (int i = 0; i < 4; ++i) {
+        const int v = kTurboInt[first + i], d = high ? (v - turbo_low(v)) / 256 : turbo_low(v);
+        t |= (uint32_t)(d & 0xFF) << (8 * i);
+    }
+    return t;
+}
+constexpr uint32_t kCodeHi[2] = {turbo_table(true, 0), turbo_table(true, 4)};
+constexpr uint32_t kCodeLo[2] = {turbo_table(false, 0), turbo_table(false, 4)};
+static_assert(turbo_low(2451) == -109 && turbo_low(-13439) == -127 && turbo_low(21519) == 15, "codebook digits");
+
+constexpr float kFixScale = 8323071.0f;       // 2^23 - 2^16 - 1: |X| <= this has 3 balanced int8 digits
+constexpr uint32_t kDigitFlip3 = 0x80808080u;
+// Byte I of four values, packed (byte 0 from y0).
+template <int I>
+FQ_DEV uint32_t byte_of(uint32_t y0, uint32_t y1, uint32_t y2, uint32_t y3) {
+    constexpr uint32_t lo = 0x0C0C0000u | ((4u + I) << 8) | I;
+    constexpr uint32_t hi = ((4u + I) << 24) | ((uint32_t)I << 16) | 0x0C0Cu;
+    return __builtin_amdgcn_perm(y1, y0, lo) | __builtin_amdgcn_perm(y3, y2, hi);
+}
 
 struct TurboFusedParams {
     fq_turbo_cache c;
@@ -35,21 +60,22 @@ struct TurboFusedParams {
 
 typedef int v4i __attribute__((ext_vector_type(4)));
 typedef float v4f __attribute__((ext_vector_type(4)));
-typedef _Float16 v8h __attribute__((ext_vector_type(8)));
-typedef _Float16 h2v __attribute__((ext_vector_type(2)));
-typedef float f2v __attribute__((ext_vector_type(2)));
-
-// Everything one page step of a lane reads (lane = (n16 = lane & 15, lg = lane >> 4)):
-//   q.k (B operand: token 16T + n16, channels 32 lg .. 32 lg + 31):
-//     km[T]: K MSB dword (channel 32 lg + c at bit c), kl[T]: K LSB 8 bytes
-//     (channel 32 lg + c at bits 2c, 2c + 1), ks[T]: K scale of the token;
-//   p.v (B operand: channels 8 n16 .. 8 n16 + 7 of token 16 T + 4 ai + lg):
-//     vm[4T + ai]: V MSB byte, vl[4T + ai]: V LSB half; vs[T]: V scale of token 16T + n16.
+// One page as a lane loads it: bytes 16 lane .. + 15 of every KB of its planes
+// (k[0] / v[0]: the 64 MSB rows of 16 bytes; k[1], k[2] / v[1], v[2]: the 64 LSB
+// rows of 32), and the K and V scale of token `lane` (2-byte loads: rows of any
+// token count, and exact at a partial last page).
 struct TurboPage {
-    uint32_t km[4];
-    uint2 kl[4];
-    uint32_t ks[4], vs[4];
-    uint32_t vm[16], vl[16];
+    uint4 k[3], v[3];
+    uint32_t ks, vs;
+};
+
+// A wave's page in LDS, as its operands are read (lane = (n16 = lane & 15, lg = lane >> 4)):
+//   q.k: K row dwords of token 16 T + n16 (MSB dword lg, LSB dwords 2 lg, 2 lg + 1);
+//   p.v: V columns, transposed, of tokens 16 byte + 4 jd + lg: 64 (MSB) / 128 (LSB)
+//   bytes of padding per 16 tokens keep the four bytes' rows on different banks.
+struct TurboLds {
+    uint8_t k[3][1024];
+    uint8_t vm[1024 + 3 * 64], vl[2048 + 3 * 128];
 };
 
 struct TurboRsrc {
@@ -57,61 +83,82 @@ struct TurboRsrc {
     int km_t, kl_t, vm_t, vl_t, ks_t, vs_t;     // token strides in bytes
 };
 
-FQ_DEV uint32_t ld8(__amdgpu_buffer_rsrc_t r, int off) { return __builtin_amdgcn_raw_buffer_load_b8(r, off, 0, 0); }
-
-// Per-lane offsets of the page loads (page 0).  Token rows are dense (16-byte
-// MSB, 32-byte LSB rows, 2-byte scales), so every other offset of a page is
-// an immediate and a page costs one add per plane.
-struct TurboLaneOff {
-    int km, kl, ks, vm, vl, vs;
-};
-
-FQ_DEV void load_turbo_page(TurboPage& b, const TurboRsrc& r, const TurboLaneOff& o, int p) {
-    const int km = o.km + p * 64 * 16, kl = o.kl + p * 64 * 32, ks = o.ks + p * 64 * 2;
-    const int vm = o.vm + p * 64 * 16, vl = o.vl + p * 64 * 32, vs = o.vs + p * 64 * 2;
+// Token rows are dense (16-byte MSB, 32-byte LSB rows, 2-byte scales).
+FQ_DEV void load_turbo_page(TurboPage& b, const TurboRsrc& r, int lane, int p) {
+    const int row = 16 * lane + p * 1024, row2 = 16 * lane + p * 2048, sc = 2 * lane + p * 128;
+    b.k[0] = ld128(r.km, row);
+    b.k[1] = ld128(r.kl, row2);
+    b.k[2] = ld128(r.kl, row2 + 1024);
+    b.ks = ld16(r.ks, sc);
+    b.v[0] = ld128(r.vm, row);
+    b.v[1] = ld128(r.vl, row2);
+    b.v[2] = ld128(r.vl, row2 + 1024);
+    b.vs = ld16(r.vs, sc);
+}
+FQ_DEV void stage_turbo_page(TurboLds& s, const TurboPage& b, int lane) {
 #pragma unroll
-    for (int T = 0; T < 4; ++T) {
-        b.km[T] = ld32(r.km, km + 16 * T * 16);
-        b.kl[T] = ld64(r.kl, kl + 16 * T * 32);
-        b.ks[T] = ld16(r.ks, ks + 16 * T * 2);
-    }
-#pragma unroll
-    for (int i = 0; i < 16; ++i) {
-        const int t = 16 * (i >> 2) + 4 * (i & 3);
-        b.vm[i] = ld8(r.vm, vm + t * 16);
-        b.vl[i] = ld16(r.vl, vl + t * 32);
-    }
-#pragma unroll
-    for (int T = 0; T < 4; ++T) b.vs[T] = ld16(r.vs, vs + 16 * T * 2);
+    for (int u = 0; u < 3; ++u) *(uint4*)&s.k[u][16 * lane] = b.k[u];
+    *(uint4*)&s.vm[16 * lane + 64 * (lane >> 4)] = b.v[0];
+    *(uint4*)&s.vl[16 * lane + 128 * (lane >> 5)] = b.v[1];
+    *(uint4*)&s.vl[1024 + 16 * lane + 128 * (2 + (lane >> 5))] = b.v[2];
+}
+// out[T]: v of lane 16 T + (lane & 15), for every lane.
+FQ_DEV void spread_rows(uint32_t v, uint32_t (&out)[4]) {
+    const auto h = __builtin_amdgcn_permlane32_swap(v, v, false, false);       // rows 0 1 0 1, rows 2 3 2 3
+    const auto a = __builtin_amdgcn_permlane16_swap(h[0], h[0], false, false);
+    const auto c = __builtin_amdgcn_permlane16_swap(h[1], h[1], false, false);
+    out[0] = a[0]; out[1] = a[1]; out[2] = c[0]; out[3] = c[1];
 }
 
-// Both fp16 parts (hi = fp16(x), lo = fp16(x - hi)) of a float.
-FQ_DEV void split_f16(float x, _Float16& hi, _Float16& lo) {
-    hi = (_Float16)x;
-    lo = (_Float16)(x - (float)hi);
+// Transposing LDS reads (ds_read_b64_tr_b8 / _tr_b16).  In each group of 16
+// lanes: tr8, lanes 2r and 2r + 1 address the two halves of row r of an 8 x 16 byte
+// matrix and lane i gets column i, one byte per row; tr16, lanes 4r .. 4r + 3
+// address row r of a 4 x 16 matrix of 16-bit values and lane i gets column i.
+typedef int v2i __attribute__((ext_vector_type(2)));
+typedef short v4s __attribute__((ext_vector_type(4)));
+FQ_DEV uint2 read_tr8(const void* lds) {
+    const v2i r = __builtin_amdgcn_ds_read_tr8_b64_v2i32((__attribute__((address_space(3))) v2i*)lds);
+    return make_uint2((uint32_t)r[0], (uint32_t)r[1]);
+}
+FQ_DEV uint2 read_tr16(const void* lds) {
+    const v4s r = __builtin_amdgcn_ds_read_tr16_b64_v4i16((__attribute__((address_space(3))) v4s*)lds);
+    return __builtin_bit_cast(uint2, r);
 }
 
-// Sparse decode attention over the TurboQuant cache on the matrix cores.
+// The value of a head's four digit rows: weights 2^24, 2^16, 2^8, 1.
+FQ_DEV float digit_rows(const v4i& a) {
+    return fmaf((float)a[0], 16777216.f, fmaf((float)a[1], 65536.f, fmaf((float)a[2], 256.f, (float)a[3])));
+}
+
+// Sparse decode attention over the TurboQuant cache on the matrix cores
+// (v_mfma_i32_16x16x64_i8): both products contract 24-bit fixed-point values X
+// (three balanced int8 digits a2 a1 a0) with the codebook's two digits H L, all
+// int32 exact.  Query head r owns rows 4r .. 4r + 3, of weights 2^24, 2^16, 2^8
+// and 1: against H the A operand's rows are a2 a1 a0 0, against L they are 0 a2
+// a1 a0, into the same accumulator, so a lane ends with its head's four rows of
+// one column.  The codebook bytes come from 3-bit codes with one v_perm per
+// four codes and digit.
 //
-// q.k (v_mfma_f32_16x16x32_f16, 16 tokens x 32 channels per step): A rows
-// 4r + {0, 1} hold query head r's fp16 hi / lo parts (q = hi + lo to fp32
-// precision), B the codebook values of 8 channels of a token, once as fp16 hi
-// and once as fp16 lo parts, looked up two channels at a time from a 64-entry
-// LDS table (index lsb d0 | lsb d1 << 2 | msb d0 << 4 | msb d1 << 5); the fp32
-// sum of the four products is q . codebook to fp32 precision.  Logit = that
-// times the token's K scale (q is pre-scaled by sm_scale * log2 e / sqrt(D)
-// after the rotation).
+// q.k (16 tokens x 64 channels per step): X = q_rot of the head relative to its
+// largest |q_rot| (rotated, pre-scaled by sm_scale * log2 e / sqrt(D)), the same
+// operands for every page; logit = sum * the token's K scale.
 //
-// p.v (v_mfma_f32_16x16x32_f16, 32 tokens x 16 channels per step): A = p *
-// V_scale / s_run (s_run a running bound of the V scales) as fp16 hi parts in
-// rows r (query heads) and lo parts in rows 4 + r; B = the codebook values
-// built in registers, byte permutes assembling each token's 3-bit code and
-// looking it up in 8-entry tables with v_perm: once their fp16 hi parts, once
-// their fp16 lo parts (two matrix instructions per tile and step into one
-// accumulator).  Rows r then hold A_hi (c_hi + c_lo), rows 4 + r A_lo (c_hi +
-// c_lo), added at the end: each product p * V_scale * codebook to 2^-22
-// relative, fp32-level like the reference's fp32 p * v.  Column n16 of
+// p.v (64 tokens x 16 channels): X = p * V_scale / s_run (at most 1; s_run a
+// running bound of the V scales, p relative to the running maximum), so a
+// product carries 2^-24 of the largest one; the sums stay integers until a page
+// raises a reference, which moves them to fp32 and rescales.  Column n16 of
 // channel tile j is channel 8 n16 + j.
+//
+// A page comes in as six 16-byte row loads and two scales per lane (48 loads of 2 to
+// 4 bytes when each operand was gathered from memory) and is staged through LDS:
+// K is read back as row dwords, V's columns by transposing reads.
+//
+// What bounds it is the instruction issue (the codes' selectors and the tables'
+// v_perm): with fp16 hi + lo parts on both sides a page took 64 matrix
+// instructions, 64 16-byte LDS table reads that conflict and about 720 vector
+// instructions; now 32, none and about 600.  28 layers x 32768 tokens, 24 query
+// heads on 8, a quarter of the pages, per query head: 137 us before; 129 on int8
+// digits, 118 with V and 112 with K and V through LDS (446 MB: 4.0 TB/s).
 //
 // HCH (FUSED only): head chunks, sel.head_chunks virtual KV heads per cache KV
 // head (virtual head h = cache head hk * HC + chunk, NREP query heads each; q,
@@ -127,12 +174,12 @@ void attn_turbo_fused_kernel(TurboFusedParams a) {
     static_assert(!HCH || FUSED, "head chunks run in the fused kernel");
     __shared__ SplitLds<D, NREP, NW> s_split;
     __shared__ int s_ent[kMaxWgPages];
-    // q.k codebook table: entry e (lsb byte of 4 channels | their msb nibble << 8)
-    // holds the fp16 hi parts of the 4 channels' codebook values, then the lo parts
-    __shared__ uint4 s_lut[4096];
     __shared__ float s_qraw[HCH ? 2 * NREP : NREP][D];      // chunk_sum: every head of the cache head
     __shared__ float s_qrot[NREP][D];
-    __shared__ uint8_t s_apv[NW][2][16][4][16];     // p.v A operands per wave: [step][row][k-group, swizzled][16 bytes]
+    // p.v A digits per wave: [head][0, a2, a1, a0, 0][k-group, XOR head][16 bytes]; the H operand reads rows
+    // 1 .. 4 of a head, the L operand rows 0 .. 3
+    __shared__ uint32_t s_apv[NW][4][5][4][4];
+    __shared__ __attribute__((aligned(16))) TurboLds s_page[NW];      // each wave's current page
 
     const fq_turbo_cache& c = a.c;
     const QueryArgs& q = a.q;
@@ -193,35 +240,7 @@ void attn_turbo_fused_kernel(TurboFusedParams a) {
         return q32 ? __uint_as_float(u) : (q.q_dtype == FQ_BF16 ? fb : fh);
     };
     const float qv_raw = q_value(ql, qh);
-    {
-        // byte tables of the codebook's fp16 parts for v_perm: [part][low / high byte][codes 0-3 / 4-7]
-        uint32_t tb[2][2][2] = {};
-#pragma unroll
-        for (int v = 0; v < 8; ++v) {
-            _Float16 hi, lo;
-            split_f16(kTurboCodebookF[v], hi, lo);
-            const uint32_t bh = __builtin_bit_cast(uint16_t, hi), bl = __builtin_bit_cast(uint16_t, lo);
-            tb[0][0][v >> 2] |= (bh & 0xFFu) << (8 * (v & 3));
-            tb[0][1][v >> 2] |= (bh >> 8) << (8 * (v & 3));
-            tb[1][0][v >> 2] |= (bl & 0xFFu) << (8 * (v & 3));
-            tb[1][1][v >> 2] |= (bl >> 8) << (8 * (v & 3));
-        }
-        for (int e = tid; e < 4096; e += NT) {
-            // byte i of sel: code of channel i = msb bit i << 2 | lsb field i
-            const uint32_t lf = (e & 3) | ((e & 0xC) << 6) | ((e & 0x30) << 12) | ((e & 0xC0) << 18);
-            const uint32_t mf = ((e >> 8) & 1) | (((e >> 9) & 1) << 8) | (((e >> 10) & 1) << 16) | (((e >> 11) & 1) << 24);
-            const uint32_t sel = lf | (mf << 2);
-            uint32_t o[4];
-#pragma unroll
-            for (int part = 0; part < 2; ++part) {
-                const uint32_t lo8 = __builtin_amdgcn_perm(tb[part][0][1], tb[part][0][0], sel);
-                const uint32_t hi8 = __builtin_amdgcn_perm(tb[part][1][1], tb[part][1][0], sel);
-                o[2 * part] = __builtin_amdgcn_perm(hi8, lo8, 0x05010400u);
-                o[2 * part + 1] = __builtin_amdgcn_perm(hi8, lo8, 0x07030602u);
-            }
-            s_lut[e] = make_uint4(o[0], o[1], o[2], o[3]);
-        }
-    }
+    for (int i = tid; i < NW * 4 * 5 * 16; i += NT) (&s_apv[0][0][0][0][0])[i] = 0u;      // the zero rows, and heads past NREP
     if constexpr (HCH) {
         if (tid < q_rows * D) s_qraw[qi >> 7][qi & 127] = qv_raw;
         if (tid + NT < q_rows * D) s_qraw[qi1 >> 7][qi1 & 127] = q_value(ql1, qh1);
@@ -258,19 +277,12 @@ void attn_turbo_fused_kernel(TurboFusedParams a) {
         rs.ks = make_rsrc(ks, (int64_t)S * rs.ks_t);
         rs.vs = make_rsrc(vs, (int64_t)S * rs.vs_t);
     }
-    TurboLaneOff loff;
-    loff.km = n16 * 16 + 4 * lg;
-    loff.kl = n16 * 32 + 8 * lg;
-    loff.ks = n16 * 2;
-    loff.vm = lg * 16 + n16;
-    loff.vl = lg * 32 + 2 * n16;
-    loff.vs = n16 * 2;
     auto issue_page = [&](TurboPage& bf, int p) {
         __builtin_amdgcn_sched_barrier(0);
-        load_turbo_page(bf, rs, loff, p);
+        load_turbo_page(bf, rs, L, p);
         __builtin_amdgcn_sched_barrier(0);
     };
-    TurboPage b0, b1;
+    TurboPage nb;          // the page after the one in LDS
     bool first_issued = false;
 
     int e0, e1, ent_base = 0;          // this split's entries are s_ent[ent_base ..]
@@ -286,7 +298,7 @@ void attn_turbo_fused_kernel(TurboFusedParams a) {
         else score_group_regs<bf16, NREP, NT, false>(sr, s_qraw, s_key, tid, c.P);
         const ForcedPages fp = forced_pages(c.P, a.sel.num_sinks, a.sel.window);
         if (S > 0 && split == 0 && w < fp.count) {   // split 0's first entries are the forced pages
-            issue_page(b0, fp.page(w));
+            issue_page(nb, fp.page(w));
             first_issued = true;
         }
         __syncthreads();
@@ -307,37 +319,43 @@ void attn_turbo_fused_kernel(TurboFusedParams a) {
     }
     const int n_mine = S > 0 && w < e1 - e0 ? (e1 - e0 - w + NW - 1) / NW : 0;
 
-    // q.k A operands: row n16 = 4 r + part (part 0: hi, 1: lo, 2-3: zero); k-group
-    // lg of step kk = channels 32 lg + 4 kk .. + 3 against their codebook hi
-    // parts (k 0-3), then the same channels against the lo parts (k 4-7)
-    v8h aqk[8];
+    // q.k A operands: lane (row n16 = 4 r + i, k-group lg); k = 16 lg + 4 jd + byte of
+    // step s is channel 32 lg + 8 byte + 4 s + jd.  aqh: digits a2 a1 a0 0 in rows i,
+    // aql: 0 a2 a1 a0.  unscale: of head lg, the logits' factor (NaN where the
+    // head's query has a NaN or an infinity: those have no digits).
+    v4i aqh[2], aql[2];
+    float unscale;
     {
-        const int r = n16 >> 2, part = n16 & 3;
-#pragma unroll
-        for (int kk = 0; kk < 8; ++kk) {
-#pragma unroll
-            for (int i = 0; i < 4; ++i) {
-                const float x = r < NREP ? s_qrot[min(r, NREP - 1)][32 * lg + 4 * kk + i] : 0.f;
-                _Float16 hi, lo;
-                split_f16(x, hi, lo);
-                const _Float16 v = part == 0 ? hi : (part == 1 ? lo : (_Float16)0.f);
-                aqk[kk][i] = v;
-                aqk[kk][i + 4] = v;
-            }
+        const int r = min(n16 >> 2, NREP - 1), i = n16 & 3;
+        float am = 0.f, bad = 0.f;
+        for (int d = lg; d < D; d += 4) {                  // 4 lanes per row
+            am = fmaxf(am, fabsf(s_qrot[r][d]));
+            bad = fmaf(s_qrot[r][d], 0.f, bad);
         }
-    }
-    // the codebook's fp16 hi / lo parts as byte tables for v_perm:
-    // [part][low / high byte][codes 0-3 / 4-7]
-    uint32_t tbv[2][2][2] = {};
+        am = fmaxf(am, __shfl_xor(am, 16, 64));
+        am = fmaxf(am, __shfl_xor(am, 32, 64));
+        bad += __shfl_xor(bad, 16, 64);
+        bad += __shfl_xor(bad, 32, 64);
+        const float inv = am > 0.f ? kFixScale / am : 0.f;
+        const float un = fmaf(am, kTurboUnit / kFixScale, bad);
+        unscale = __shfl(un, 4 * min(lg, NREP - 1), 64);
+        const bool mine = (n16 >> 2) < NREP;
 #pragma unroll
-    for (int v = 0; v < 8; ++v) {
-        _Float16 hi, lo;
-        split_f16(kTurboCodebookF[v], hi, lo);
-        const uint32_t bh = __builtin_bit_cast(uint16_t, hi), bl = __builtin_bit_cast(uint16_t, lo);
-        tbv[0][0][v >> 2] |= (bh & 0xFFu) << (8 * (v & 3));
-        tbv[0][1][v >> 2] |= (bh >> 8) << (8 * (v & 3));
-        tbv[1][0][v >> 2] |= (bl & 0xFFu) << (8 * (v & 3));
-        tbv[1][1][v >> 2] |= (bl >> 8) << (8 * (v & 3));
+        for (int st = 0; st < 2; ++st)
+#pragma unroll
+            for (int jd = 0; jd < 4; ++jd) {
+                uint32_t Y[4];
+#pragma unroll
+                for (int by = 0; by < 4; ++by)        // X + 0x808080, rounded by the fp32 add itself
+                    Y[by] = (uint32_t)fmaf(s_qrot[r][32 * lg + 8 * by + 4 * st + jd], inv, 8421504.0f);
+                const uint32_t a2 = byte_of<2>(Y[0], Y[1], Y[2], Y[3]) ^ kDigitFlip3;
+                const uint32_t a1 = byte_of<1>(Y[0], Y[1], Y[2], Y[3]) ^ kDigitFlip3;
+                const uint32_t a0 = byte_of<0>(Y[0], Y[1], Y[2], Y[3]) ^ kDigitFlip3;
+                const uint32_t hi = i == 0 ? a2 : i == 1 ? a1 : i == 2 ? a0 : 0u;
+                const uint32_t lo = i == 0 ? 0u : i == 1 ? a2 : i == 2 ? a1 : a0;
+                aqh[st][jd] = mine ? (int)hi : 0;
+                aql[st][jd] = mine ? (int)lo : 0;
+            }
     }
 
     auto entry_of = [&](int k) { return __builtin_amdgcn_readfirstlane(s_ent[ent_base + w + NW * k]); };
@@ -345,13 +363,25 @@ void attn_turbo_fused_kernel(TurboFusedParams a) {
     float m_run[NREP];
 #pragma unroll
     for (int r = 0; r < NREP; ++r) m_run[r] = -INFINITY;
-    float s_run = 0.f, inv_s = 1.f;          // running bound of V scales (p * V_scale / s_run <= 1/2)
+    float s_run = 0.f, fix_s = 0.f;          // running bound of the V scales, kFixScale / s_run
     float m_lane = 0.f;                      // m_run[lg], or 0 while head lg has no logit yet
-    v4f pacc[8];                             // [channel tile]: component r = head r
+    v4i pacc[8];                             // [channel tile]: head lg's digit rows since the references last moved
+    float facc[8];                           // and what came before
 #pragma unroll
-    for (int t = 0; t < 8; ++t) pacc[t] = (v4f){0.f, 0.f, 0.f, 0.f};
-    float l_acc = 0.f;
+    for (int t = 0; t < 8; ++t) {
+        pacc[t] = (v4i){0, 0, 0, 0};
+        facc[t] = 0.f;
+    }
+    float l_acc = 0.f, bad_v = 0.f;          // bad_v: NaN once a p * V_scale is one or infinite (no digits either)
     auto& W = s_apv[w];
+    auto& WP = s_page[w];
+    // the lane's addresses: K rows (tile T 16 tokens on); the transposed reads' V rows: MSB read u, row r = 0..7 is
+    // token 16 (r & 3) + 4 (2 u + (r >> 2)) + lg, LSB read jd, row r = 0..3 token 16 r + 4 jd + lg
+    const uint8_t* const kmp = &WP.k[0][0] + 16 * n16 + 4 * lg;
+    const uint8_t* const klp = &WP.k[1][0] + 32 * n16 + 8 * lg;
+    const int trr = (n16 >> 1) & 3;
+    const uint8_t* const trm = WP.vm + (16 * trr + 4 * (n16 >> 3) + lg) * 16 + 64 * trr + 8 * (n16 & 1);
+    const uint8_t* const trl = WP.vl + (16 * (n16 >> 2) + lg) * 32 + 128 * (n16 >> 2) + 8 * (n16 & 3);
 
     // the idle partner-wave priority rule of the INT4 fused decode: two waves
     // share a SIMD; the one with more pages left (on a tie the younger) takes
@@ -364,43 +394,38 @@ void attn_turbo_fused_kernel(TurboFusedParams a) {
         else __builtin_amdgcn_s_setprio(0);
     };
 
-    auto compute = [&](const TurboPage& pb, int k) {
+    auto compute = [&](uint32_t scales, int k) {       // scales: K and V scale of token `lane`
         balance(k);
         const int ent = entry_of(k);
         const int p = ent & 0xFFFF, qm = ent >> 16;
         const int tok0 = p * 64;
-        // ---- q.k: the four 16-token tiles' accumulation chains interleaved
-        // (k-step outer), so four independent matrix instructions are in flight;
-        // each tile still accumulates its k-steps in order
+        uint32_t sc[4];
+        spread_rows(scales, sc);
+        // ---- q.k: tile T is tokens 16 T + n16
         float lg4[4], mp = -INFINITY;
-        v4f acc[4];
-#pragma unroll
-        for (int T = 0; T < 4; ++T) acc[T] = (v4f){0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-        for (int kk = 0; kk < 8; ++kk) {
-            // the k-step's four table reads go out together, then its four
-            // matrix instructions (one read in flight at a time otherwise)
-            uint4 e[4];
-#pragma unroll
-            for (int T = 0; T < 4; ++T) {
-                // table entry of channels 32 lg + 4 kk .. + 3: their LSB byte, MSB nibble
-                const uint32_t lw = (kk >> 2) ? pb.kl[T].y : pb.kl[T].x;
-                const int lsh = 8 * (kk & 3) - 4, msh = 4 * kk - 12;      // entry * 16, in bytes
-                const uint32_t a_l = (lsh >= 0 ? lw >> lsh : lw << -lsh) & 0xFF0u;
-                const uint32_t a_m = (msh >= 0 ? pb.km[T] >> msh : pb.km[T] << -msh) & 0xF000u;
-                e[T] = *(const uint4*)((const char*)s_lut + (a_l | a_m));
-            }
-            __builtin_amdgcn_sched_group_barrier(0x100, 4, 0);     // 4 LDS reads
-            __builtin_amdgcn_sched_group_barrier(0x008, 4, 0);     // then 4 matrix instructions
-#pragma unroll
-            for (int T = 0; T < 4; ++T) {
-                const v8h B = __builtin_bit_cast(v8h, (v4i){(int)e[T].x, (int)e[T].y, (int)e[T].z, (int)e[T].w});
-                acc[T] = __builtin_amdgcn_mfma_f32_16x16x32_f16(aqk[kk], B, acc[T], 0, 0, 0);
-            }
-        }
 #pragma unroll
         for (int T = 0; T < 4; ++T) {
-            const float lgt = (acc[T][0] + acc[T][1]) * bf16_bits_to_f(pb.ks[T] & 0xFFFFu);
+            // LSB bytes of channels 8 byte + 0..3 / 4..7
+            const uint2 kl = *(const uint2*)(klp + 512 * T);
+            const uint32_t km = *(const uint32_t*)(kmp + 256 * T);
+            const uint32_t le = __builtin_amdgcn_perm(kl.y, kl.x, 0x06040200u);
+            const uint32_t lo = __builtin_amdgcn_perm(kl.y, kl.x, 0x07050301u);
+            v4i acc = {0, 0, 0, 0};
+#pragma unroll
+            for (int st = 0; st < 2; ++st) {
+                v4i bh, bl;
+#pragma unroll
+                for (int jd = 0; jd < 4; ++jd) {
+                    const int i = 4 * st + jd;                 // byte: channel 8 byte + i, its MSB at bit i
+                    const uint32_t m = i >= 2 ? km >> (i - 2) : km << (2 - i);
+                    const uint32_t sel = (m & 0x04040404u) | (((st ? lo : le) >> (2 * jd)) & 0x03030303u);
+                    bh[jd] = (int)__builtin_amdgcn_perm(kCodeHi[1], kCodeHi[0], sel);
+                    bl[jd] = (int)__builtin_amdgcn_perm(kCodeLo[1], kCodeLo[0], sel);
+                }
+                acc = __builtin_amdgcn_mfma_i32_16x16x64_i8(aqh[st], bh, acc, 0, 0, 0);
+                acc = __builtin_amdgcn_mfma_i32_16x16x64_i8(aql[st], bl, acc, 0, 0, 0);
+            }
+            const float lgt = digit_rows(acc) * unscale * bf16_bits_to_f(sc[T] & 0xFFFFu);
             const bool ok = lg < NREP && ((qm >> lg) & 1) && tok0 + 16 * T + n16 < S;
             lg4[T] = ok ? lgt : -INFINITY;
             mp = fmaxf(mp, lg4[T]);
@@ -409,7 +434,7 @@ void attn_turbo_fused_kernel(TurboFusedParams a) {
         float vs_t[4], sp = 0.f;
 #pragma unroll
         for (int T = 0; T < 4; ++T) {
-            vs_t[T] = bf16_bits_to_f(pb.vs[T] & 0xFFFFu);
+            vs_t[T] = __uint_as_float(sc[T] & 0xFFFF0000u);
             sp = fmaxf(sp, vs_t[T]);
         }
         mp = row16_max(mp);
@@ -429,10 +454,10 @@ void attn_turbo_fused_kernel(TurboFusedParams a) {
                 am[r] = mn == m_run[r] ? 1.0f : exp2_fast(m_run[r] - mn);
                 m_run[r] = mn;
             }
-            const float sn = sp > s_run ? 2.0f * sp : s_run;
+            const float sn = fmaxf(sp, s_run);
             const float as = sn > 0.f ? s_run / sn : 1.0f;
             s_run = sn;
-            inv_s = sn > 0.f ? 1.0f / sn : 0.f;
+            fix_s = sn > 0.f ? kFixScale / sn : 0.f;
             float am_lg = am[0], ml = m_run[0];
 #pragma unroll
             for (int r = 1; r < NREP; ++r) {
@@ -441,109 +466,95 @@ void attn_turbo_fused_kernel(TurboFusedParams a) {
             }
             m_lane = ml == -INFINITY ? 0.f : ml;
             l_acc *= am_lg;
+            const float f = am_lg * as;
 #pragma unroll
-            for (int r = 0; r < 4; ++r) {
-                const float f = r < NREP ? am[r] * as : 0.f;
-#pragma unroll
-                for (int t = 0; t < 8; ++t) pacc[t][r] *= f;
+            for (int t = 0; t < 8; ++t) {
+                facc[t] = (facc[t] + digit_rows(pacc[t])) * f;
+                pacc[t] = (v4i){0, 0, 0, 0};
             }
         }
-        // ---- p.v A: p * V_scale / s_run (fp16); operand k = 8 kg + 2 ai + jj of
-        // step s is token 16 (2s + jj) + 4 ai + kg
-        float pr[4];
+        // ---- p.v A: the digits of p * V_scale / s_run; operand k = 16 kg + 4 jd + byte
+        // is token 16 byte + 4 jd + kg, so the lane's four tokens are one dword
+        uint32_t Y[4];
 #pragma unroll
         for (int T = 0; T < 4; ++T) {
-            pr[T] = exp2_fast(lg4[T] - m_lane);
-            l_acc += pr[T];
+            const float pr = exp2_fast(lg4[T] - m_lane);
+            l_acc += pr;
+            const float x = pr * vs_t[T];
+            bad_v = fmaf(x, 0.f, bad_v);
+            Y[T] = (uint32_t)fmaf(x, fix_s, 8421504.0f);
         }
-        if (lg < NREP) {       // rows lg (hi parts) and 4 + lg (lo parts), k-groups swizzled by row
-            const int kq = n16 & 3;
-#pragma unroll
-            for (int st = 0; st < 2; ++st) {
-                const f2v xv = {pr[2 * st] * vs_t[2 * st] * inv_s, pr[2 * st + 1] * vs_t[2 * st + 1] * inv_s};
-                const h2v hv = __builtin_convertvector(xv, h2v);
-                const h2v lv = __builtin_convertvector(xv - __builtin_convertvector(hv, f2v), h2v);
-                *(uint32_t*)&W[st][lg][kq][4 * (n16 >> 2)] = __builtin_bit_cast(uint32_t, hv);
-                *(uint32_t*)&W[st][4 + lg][kq ^ 1][4 * (n16 >> 2)] = __builtin_bit_cast(uint32_t, lv);
-            }
+        if (lg < NREP) {
+            uint32_t* dst = &W[lg][1][(n16 & 3) ^ lg][n16 >> 2];
+            dst[0] = byte_of<2>(Y[0], Y[1], Y[2], Y[3]) ^ kDigitFlip3;
+            dst[16] = byte_of<1>(Y[0], Y[1], Y[2], Y[3]) ^ kDigitFlip3;
+            dst[32] = byte_of<0>(Y[0], Y[1], Y[2], Y[3]) ^ kDigitFlip3;
         }
         __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
-        const int kr = lg ^ ((n16 >> 2) & 3);
-        const v8h ap0 = *(const v8h*)&W[0][n16][kr][0];
-        const v8h ap1 = *(const v8h*)&W[1][n16][kr][0];
-        // ---- p.v B: codes of channel 8 n16 + j for the step's 8 tokens, 4 at a time
+        const int hr = n16 >> 2;
+        const v4i aph = *(const v4i*)&W[hr][(n16 & 3) + 1][lg ^ hr][0];
+        const v4i apl = *(const v4i*)&W[hr][n16 & 3][lg ^ hr][0];
+        // ---- p.v B: codes of channel 8 n16 + j, dword jd = tokens 16 byte + 4 jd + lg
+        uint32_t m4[4], ll[4], lh[4];        // the 4 tokens' MSB bytes; LSB fields of channels 0-3 / 4-7
 #pragma unroll
-        for (int st = 0; st < 2; ++st) {
-            // per half hh: operand k = 4 hh + kk is token i = 4 (2 st + (kk & 1)) + 2 hh + (kk >> 1);
-            // m4: the 4 tokens' MSB bytes, ll / lh: their LSB fields of channels 0-3 / 4-7
-            uint32_t m4[2], ll[2], lh[2];
+        for (int u = 0; u < 2; ++u) {
+            const uint2 m = read_tr8(trm + 128 * u);
+            m4[2 * u] = m.x;
+            m4[2 * u + 1] = m.y;
+        }
 #pragma unroll
-            for (int hh = 0; hh < 2; ++hh) {
-                const int i0 = 8 * st + 2 * hh, i1 = i0 + 4, i2 = i0 + 1, i3 = i0 + 5;
-                m4[hh] = pb.vm[i0] | (pb.vm[i1] << 8) | (pb.vm[i2] << 16) | (pb.vm[i3] << 24);
-                const uint32_t x01 = __builtin_amdgcn_perm(pb.vl[i1], pb.vl[i0], 0x05010400u);
-                const uint32_t x23 = __builtin_amdgcn_perm(pb.vl[i3], pb.vl[i2], 0x05010400u);
-                ll[hh] = __builtin_amdgcn_perm(x23, x01, 0x05040100u);
-                lh[hh] = __builtin_amdgcn_perm(x23, x01, 0x07060302u);
+        for (int jd = 0; jd < 4; ++jd) {
+            const uint2 x = read_tr16(trl + 128 * jd);      // two tokens' LSB halves a dword
+            ll[jd] = __builtin_amdgcn_perm(x.y, x.x, 0x06040200u);
+            lh[jd] = __builtin_amdgcn_perm(x.y, x.x, 0x07050301u);
+        }
+#pragma unroll
+        for (int j = 0; j < 8; ++j) {
+            v4i bh, bl;
+#pragma unroll
+            for (int jd = 0; jd < 4; ++jd) {
+                const uint32_t m = j >= 2 ? m4[jd] >> (j - 2) : m4[jd] << (2 - j);
+                const uint32_t sel = (m & 0x04040404u) | (((j < 4 ? ll[jd] : lh[jd]) >> (2 * (j & 3))) & 0x03030303u);
+                bh[jd] = (int)__builtin_amdgcn_perm(kCodeHi[1], kCodeHi[0], sel);
+                bl[jd] = (int)__builtin_amdgcn_perm(kCodeLo[1], kCodeLo[0], sel);
             }
-            const v8h a = st ? ap1 : ap0;
-            v8h bl_prev;        // tile j - 1's lo-part operand: its matrix instruction follows tile j's
-#pragma unroll
-            for (int j = 0; j < 8; ++j) {
-                uint32_t bw[4], bwl[4];       // channel tile j: codebook hi / lo parts
-#pragma unroll
-                for (int hh = 0; hh < 2; ++hh) {
-                    const uint32_t lx = j < 4 ? ll[hh] : lh[hh];
-                    // byte k: msb bit j of token k at bit 2, its lsb field j below
-                    const uint32_t mj = j >= 2 ? m4[hh] >> (j - 2) : m4[hh] << (2 - j);
-                    const uint32_t sel = (mj & 0x04040404u) | ((lx >> (2 * (j & 3))) & 0x03030303u);
-                    const uint32_t lo = __builtin_amdgcn_perm(tbv[0][0][1], tbv[0][0][0], sel);
-                    const uint32_t hi = __builtin_amdgcn_perm(tbv[0][1][1], tbv[0][1][0], sel);
-                    bw[2 * hh] = __builtin_amdgcn_perm(hi, lo, 0x05010400u);
-                    bw[2 * hh + 1] = __builtin_amdgcn_perm(hi, lo, 0x07030602u);
-                    const uint32_t llo = __builtin_amdgcn_perm(tbv[1][0][1], tbv[1][0][0], sel);
-                    const uint32_t lhi = __builtin_amdgcn_perm(tbv[1][1][1], tbv[1][1][0], sel);
-                    bwl[2 * hh] = __builtin_amdgcn_perm(lhi, llo, 0x05010400u);
-                    bwl[2 * hh + 1] = __builtin_amdgcn_perm(lhi, llo, 0x07030602u);
-                }
-                const v8h bv = __builtin_bit_cast(v8h, (v4i){(int)bw[0], (int)bw[1], (int)bw[2], (int)bw[3]});
-                const v8h bl = __builtin_bit_cast(v8h, (v4i){(int)bwl[0], (int)bwl[1], (int)bwl[2], (int)bwl[3]});
-                pacc[j] = __builtin_amdgcn_mfma_f32_16x16x32_f16(a, bv, pacc[j], 0, 0, 0);
-                if (j > 0) pacc[j - 1] = __builtin_amdgcn_mfma_f32_16x16x32_f16(a, bl_prev, pacc[j - 1], 0, 0, 0);
-                bl_prev = bl;
-            }
-            pacc[7] = __builtin_amdgcn_mfma_f32_16x16x32_f16(a, bl_prev, pacc[7], 0, 0, 0);
+            pacc[j] = __builtin_amdgcn_mfma_i32_16x16x64_i8(aph, bh, pacc[j], 0, 0, 0);
+            pacc[j] = __builtin_amdgcn_mfma_i32_16x16x64_i8(apl, bl, pacc[j], 0, 0, 0);
         }
         __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
     };
 
+    // A page is loaded in whole rows (8 loads), one page ahead, and goes to LDS
+    // when the page before it is done; a wave's LDS accesses are in order, so its one
+    // page buffer needs no barrier.
     {
         s_left[w] = n_mine;
-        if (!first_issued) issue_page(b0, n_mine > 0 ? entry_of(0) & 0xFFFF : 0);
-        for (int k = 0; k < n_mine; k += 2) {
-            issue_page(b1, entry_of(min(k + 1, n_mine - 1)) & 0xFFFF);
-            compute(b0, k);
-            issue_page(b0, entry_of(min(k + 2, n_mine - 1)) & 0xFFFF);
-            if (k + 1 < n_mine) compute(b1, k + 1);
+        if (!first_issued) issue_page(nb, n_mine > 0 ? entry_of(0) & 0xFFFF : 0);
+        for (int k = 0; k < n_mine; ++k) {
+            stage_turbo_page(WP, nb, L);
+            const uint32_t scales = (nb.ks & 0xFFFFu) | (nb.vs << 16);
+            __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
+            issue_page(nb, entry_of(min(k + 1, n_mine - 1)) & 0xFFFF);
+            compute(scales, k);
         }
         __builtin_amdgcn_s_setprio(0);
     }
 
-    // ---- wave state -> LDS: head r's sums in lane group r (over the 16 token
-    // columns); outputs of channel 8 n16 + j in lane group 0, component r, plus
-    // the lo rows 4 + r in lane group 1
-#pragma unroll
-    for (int j = 0; j < 8; ++j)
-#pragma unroll
-        for (int r = 0; r < NREP; ++r) pacc[j][r] += __shfl_xor(pacc[j][r], 16, 64);
+    // ---- wave state -> LDS: head lg's sums (over its lane group's 16 token columns)
+    // and its outputs of channels 8 n16 + j, in units of s_run / kFixScale * 1e-4
     l_acc = row_sum<16>(l_acc);
+    bad_v = row_sum<16>(bad_v);
+    const float pv_unscale = s_run * (kTurboUnit / kFixScale);
+    if (lg < NREP) {
 #pragma unroll
-    for (int r = 0; r < NREP; ++r) {
-        const float ll = __shfl(l_acc, 16 * r + n16, 64);
-        if (lg == 0) {
+        for (int j = 0; j < 8; ++j)
+            s_split.acc[w][lg][8 * n16 + j] = fmaf(facc[j] + digit_rows(pacc[j]), pv_unscale, bad_v);
+        if (n16 == 0) {
+            float m = m_run[0];
 #pragma unroll
-            for (int j = 0; j < 8; ++j) s_split.acc[w][r][8 * n16 + j] = pacc[j][r] * s_run;
-            if (n16 == 0) { s_split.m[w][r] = m_run[r]; s_split.l[w][r] = ll; }
+            for (int r = 1; r < NREP; ++r) m = lg == r ? m_run[r] : m;
+            s_split.m[w][lg] = m;
+            s_split.l[w][lg] = l_acc;
         }
     }
     __syncthreads();
@@ -577,16 +588,15 @@ bool turbo_fused_supported(const fq_turbo_cache& c, const QueryArgs& q) {
     if (c.D != 128 || c.page_size != 64 || q.nrep > 4 || c.P > kMaxWgPages) return false;
     if (c.kmsb_strides[4] != 1 || c.klsb_strides[4] != 1 || c.vmsb_strides[4] != 1 || c.vlsb_strides[4] != 1)
         return false;
-    // dense token rows (16-byte MSB, 32-byte LSB rows, 2-byte scales); K: 4-byte
-    // MSB and 8-byte LSB words per lane; V: 2-byte LSB words
+    // dense token rows (16-byte MSB, 32-byte LSB rows, 2-byte scales), read in
+    // words of 4 bytes or more
     if (c.kmsb_strides[3] != 16 || c.klsb_strides[3] != 32 || c.vmsb_strides[3] != 16 || c.vlsb_strides[3] != 32)
         return false;
     if (c.kst_strides[3] != 1 || c.vst_strides[3] != 1) return false;
     for (int i = 0; i < 3; ++i) {
-        if (c.kmsb_strides[i] % 4 || c.klsb_strides[i] % 4 || c.vlsb_strides[i] % 2) return false;
+        if (c.kmsb_strides[i] % 4 || c.klsb_strides[i] % 4 || c.vmsb_strides[i] % 4 || c.vlsb_strides[i] % 4) return false;
     }
-    if ((uintptr_t)c.k_msb & 3) return false;
-    if (((uintptr_t)c.k_lsb & 3) || ((uintptr_t)c.v_lsb & 1)) return false;
+    if (((uintptr_t)c.k_msb | (uintptr_t)c.k_lsb | (uintptr_t)c.v_msb | (uintptr_t)c.v_lsb) & 3) return false;
     if (((uintptr_t)c.k_scale | (uintptr_t)c.v_scale) & 1) return false;
     return true;
 }
