@@ -14,51 +14,32 @@ FQ_DEV int k_for(float r, int P, int k_max) {
     return k;
 }
 
+constexpr int kTakeAll = 0x7FFFFFFF;        // wave_kth_hist: every key at the threshold is in
+template <int C>
+FQ_DEV uint32_t wave_kth_hist(const uint32_t (&key)[C], int k, uint32_t* hist, int& take);
+
 // Marks the k largest of keys (lane holds key[j] of page 64 j + lane; ties to the
-// lower page index) into qm |= bit.  The k-th largest key is found bit by bit
-// with wave-wide counts (ballots, scalar popcounts); ties are ranked by ballots.
-// The k-th largest of the wave's 64 C keys (k >= 1), found bit by bit: T keeps
-// the largest prefix that at least k keys reach.  Wave-uniform, no LDS.
-template <int C>
-FQ_DEV uint32_t wave_kth_largest(const uint32_t (&key)[C], int k) {
-    uint32_t T = 0;
-    for (int bitpos = 31; bitpos >= 0; --bitpos) {
-        const uint32_t cand = T | (1u << bitpos);
-        int cnt = 0;
-#pragma unroll
-        for (int j = 0; j < C; ++j) cnt += __popcll(__ballot(key[j] >= cand));
-        if (cnt >= k) T = cand;
-    }
-    return T;
-}
-
-template <int C>
-FQ_DEV uint32_t wave_kth_hist(const uint32_t (&key)[C], int k, uint32_t* hist, bool* exact = nullptr);
-
-// hist: 256 words of LDS used by this wave only (wave_kth_hist's digit counts).
+// lower page index) into qm |= bit.  hist: 256 words of LDS used by this wave only
+// (wave_kth_hist's digit counts).
 template <int C>
 FQ_DEV void wave_topk(const uint32_t (&key)[C], uint8_t (&qm)[C], int k, uint8_t bit, uint32_t* hist) {
     if (k <= 0) return;
-    bool exact;
-    const uint32_t T = wave_kth_hist<C>(key, k, hist, &exact);
-    if (exact) {         // exactly k keys >= T: no ties to rank
+    int take;
+    const uint32_t T = wave_kth_hist<C>(key, k, hist, take);
+    if (take == kTakeAll) {         // exactly k keys >= T: no ties to rank
 #pragma unroll
         for (int j = 0; j < C; ++j)
             if (key[j] >= T) qm[j] |= bit;
         return;
     }
     // T is the k-th largest key; keys above it are in, ties fill the rest by index
-    int gt = 0;
-#pragma unroll
-    for (int j = 0; j < C; ++j) gt += __popcll(__ballot(key[j] > T));
-    int take_eq = k - gt;
 #pragma unroll
     for (int j = 0; j < C; ++j) {
         if (key[j] > T) qm[j] |= bit;
         const uint64_t eq = __ballot(key[j] == T);
         const int rank = (int)lanes_below(eq);
-        if (key[j] == T && rank < take_eq) qm[j] |= bit;
-        take_eq -= __popcll(eq);
+        if (key[j] == T && rank < take) qm[j] |= bit;
+        take -= __popcll(eq);
     }
 }
 
@@ -196,22 +177,24 @@ FQ_DEV ForcedPages forced_pages(int P, int num_sinks, int window) {
 
 // Workgroup-wide selection for one KV group, same result as wave_select_group
 // (P <= 64 C pages, NW waves).  keys[r * 64 C + p] holds sortable_key of row
-// r's score of page p, and 0 (below every score) for p >= P.  Every wave loads
-// every key (C per lane per row); wave r finds row r's k-th largest key with
-// wave_kth_hist (no barrier inside; for one row only the last wave searches,
-// so its SIMD is not shared with a partner wave doing the same search, and
-// the last wave issues no forced-page loads before it); the thresholds meet
-// in LDS, and every
-// wave then ranks the ties and lists the pages.  Ties and forced pages follow
+// r's score of page p, and 0 (below every score) for p >= P.  Wave NW - 1 - r
+// finds row r's k-th largest key with wave_kth_hist (no barrier inside; up to 4
+// rows on different SIMDs, the waves that issued forced-page loads last); the
+// thresholds and how many ties they take meet in LDS.  Then wave w decides the
+// pages 64 j + lane with j = w (mod NW) alone, the counts meet in LDS, and each
+// wave writes its entries.  (Every wave ranking every page, as before, took
+// two thirds of the selection: 3.2 us a step with 3 query heads and 128 to 512
+// pages, now SELECT_NOTE.)  Ties and forced pages follow
 // wave_topk / wave_select_group; the entry list holds the forced pages first,
-// then the other selected pages, each part ascending; wave w writes the entries
-// of pages 64 j + lane with j = w (mod NW).  NROWS = 1: one top-k of the summed
-// row with the group's largest retention (per_kv_head_sum); NROWS = nrep: one
-// per query head.  ret_l: lane r holds query head r's retention.  All control
-// flow is wave-uniform.  Ends with a barrier; returns the list length in
+// then the other selected pages, each part ascending.  NROWS = 1: one top-k of
+// the summed row with the group's largest retention (per_kv_head_sum); NROWS =
+// nrep: one per query head.  ret_l: lane r holds query head r's retention.  All
+// control flow is wave-uniform.  Ends with a barrier; returns the list length in
 // every thread.
 struct alignas(16) BlockSelectLds {
     uint32_t T[4];          // k-th largest key per row
+    int take[4];            // how many of the keys equal to it are in
+    int cnt[64];            // entries of pages 64 j .. 64 j + 63
     uint32_t hist[8][256];  // wave_kth_hist: one 256-bin digit histogram per wave
 };
 
@@ -261,11 +244,12 @@ FQ_DEV uint32_t wave_max_u32(uint32_t v) {
 // words used by this wave only) and located by a wave prefix sum.  The bits
 // every key shares (the common prefix of the smallest and largest key) are
 // skipped, and the search stops once the keys reaching the current prefix are
-// exactly k (then T has exactly k keys >= T); otherwise T ends as the k-th
-// largest key -- the contract the callers rely on: keys above T, then ties at
+// exactly k (then T has exactly k keys >= T and take = kTakeAll); otherwise T
+// ends as the k-th largest key and take as the number of keys equal to it that
+// are in -- the contract the callers rely on: keys above T, then `take` ties at
 // T by page index, give the top k.  Wave-uniform; hist is left zeroed.
 template <int C>
-FQ_DEV uint32_t wave_kth_hist(const uint32_t (&key)[C], int k, uint32_t* hist, bool* exact) {
+FQ_DEV uint32_t wave_kth_hist(const uint32_t (&key)[C], int k, uint32_t* hist, int& take) {
     const int lane = lane_id();
     // lo: the smallest key above 0.  Key 0 marks a slot past the last page
     // (below every score, never among the top k <= P), so leaving it out of
@@ -276,8 +260,10 @@ FQ_DEV uint32_t wave_kth_hist(const uint32_t (&key)[C], int k, uint32_t* hist, b
     lo = wave_min_u32(lo);
     if (lo > hi) lo = hi;            // no key above 0
     hi = wave_max_u32(hi);
-    if (exact) *exact = false;
-    if (lo == hi) return hi;
+    if (lo == hi) {                  // every page's key the same
+        take = k;
+        return hi;
+    }
     int b = 31 - __clz(lo ^ hi);                    // bits above b are the same in every key
     uint32_t prefix = hi & ~((2u << b) - 1u);
     int need = k;                                   // keys still to take from those matching prefix above b
@@ -313,10 +299,13 @@ FQ_DEV uint32_t wave_kth_hist(const uint32_t (&key)[C], int k, uint32_t* hist, b
         prefix |= (uint32_t)(255 - 4 * ls - m_s) << shift;
         need -= ab_s;
         if (cd_s == need) {          // exactly k keys are >= prefix
-            if (exact) *exact = true;
+            take = kTakeAll;
             return prefix;
         }
-        if (shift == 0) return prefix;
+        if (shift == 0) {
+            take = need;
+            return prefix;
+        }
         b = shift - 1;
     }
 }
@@ -325,82 +314,77 @@ template <int C, int NW, int NROWS, int NREP>
 FQ_DEV int block_select_rows(const uint32_t* keys, int P, float ret_l, int k_max, int num_sinks, int window,
                              int* entries, BlockSelectLds& sl) {
     static_assert(NROWS <= NW && NROWS <= 4, "one wave per row; at most 4 rows");
+    static_assert(C <= 64, "one lane per count");
+    constexpr int CW = (C + NW - 1) / NW;        // 64-page chunks of one wave
     const int lane = lane_id(), w = __builtin_amdgcn_readfirstlane(wave_id());
     constexpr uint8_t kAll = (uint8_t)((1u << NREP) - 1u);
-    uint32_t key[NROWS][C];
-    int k[NROWS];
-    uint32_t T[NROWS];
-#pragma unroll
-    for (int r = 0; r < NROWS; ++r)
-#pragma unroll
-        for (int j = 0; j < C; ++j) key[r][j] = keys[r * 64 * C + 64 * j + lane];
-    float rmax = 0.f;
-#pragma unroll
-    for (int r = 0; r < NREP; ++r) rmax = fmaxf(rmax, __int_as_float(__builtin_amdgcn_readlane(__float_as_int(ret_l), r)));
-#pragma unroll
-    for (int r = 0; r < NROWS; ++r)
-        k[r] = k_for(NROWS == 1 ? rmax : __int_as_float(__builtin_amdgcn_readlane(__float_as_int(ret_l), r)), P, k_max);
-    bool exact = false;              // one row: exactly k keys >= T, no ties to rank
-    if constexpr (NROWS == 1) {      // one row: the last wave finds the threshold, shared through LDS
-        if (w == NW - 1) {
-            bool ex = false;
-            const uint32_t t = k[0] > 0 ? wave_kth_hist<C>(key[0], k[0], sl.hist[w], &ex) : 0u;
-            if (lane == 0) { sl.T[0] = t; sl.T[1] = ex ? 1u : 0u; }
-        }
-        lds_barrier();
-        T[0] = sl.T[0];
-        exact = sl.T[1] != 0u;
-    } else {                         // wave r finds row r's, shared through LDS
-#pragma unroll
-        for (int r = 0; r < NROWS; ++r) {
-            if (w == r) {
-                const uint32_t t = k[r] > 0 ? wave_kth_hist<C>(key[r], k[r], sl.hist[w]) : 0u;
-                if (lane == 0) sl.T[r] = t;
-            }
-        }
-        lds_barrier();
-#pragma unroll
-        for (int r = 0; r < NROWS; ++r) T[r] = sl.T[r];
-    }
-    // ties at T: the lowest page indices (wave_topk's rule); identical in every wave
-    uint8_t qm[C];
-#pragma unroll
-    for (int j = 0; j < C; ++j) qm[j] = 0;
-    if (exact) {         // uniform
-#pragma unroll
-        for (int j = 0; j < C; ++j) qm[j] = key[0][j] >= T[0] ? kAll : (uint8_t)0;
-    } else
 #pragma unroll
     for (int r = 0; r < NROWS; ++r) {
-        if (k[r] <= 0) continue;
-        const uint8_t bit = NROWS == 1 ? kAll : (uint8_t)(1u << r);
-        int gt = 0;
+        if (w == NW - 1 - r) {
+            float ret = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(ret_l), r));
+            if constexpr (NROWS == 1) {          // the group's largest
 #pragma unroll
-        for (int j = 0; j < C; ++j) gt += __popcll(__ballot(key[r][j] > T[r]));
-        int take_eq = k[r] - gt;
+                for (int i = 1; i < NREP; ++i)
+                    ret = fmaxf(ret, __int_as_float(__builtin_amdgcn_readlane(__float_as_int(ret_l), i)));
+                ret = fmaxf(ret, 0.f);
+            }
+            uint32_t key[C];
 #pragma unroll
-        for (int j = 0; j < C; ++j) {
-            const uint64_t eq = __ballot(key[r][j] == T[r]);
-            const bool in = key[r][j] > T[r] || (key[r][j] == T[r] && (int)lanes_below(eq) < take_eq);
-            qm[j] |= in ? bit : (uint8_t)0;
-            take_eq -= __popcll(eq);
+            for (int j = 0; j < C; ++j) key[j] = keys[r * 64 * C + 64 * j + lane];
+            const int k = k_for(ret, P, k_max);
+            int take = 0;
+            const uint32_t T = k > 0 ? wave_kth_hist<C>(key, k, sl.hist[w], take) : ~0u;     // k = 0: no key is in
+            if (lane == 0) { sl.T[r] = T; sl.take[r] = take; }
         }
     }
+    lds_barrier();
+    // the pages 64 j + lane of this wave's chunks: selected by which rows; the
+    // ties at a threshold are the lowest page indices (wave_topk's rule)
+    const ForcedPages fp = forced_pages(P, num_sinks, window);
+    uint8_t qm[CW];
+    bool in_list[CW];
+    uint64_t bal[CW];
+#pragma unroll
+    for (int u = 0; u < CW; ++u) {
+        const int j = w + NW * u;
+        qm[u] = 0;
+        in_list[u] = false;
+        bal[u] = 0;
+        if (j >= C) continue;                    // uniform
+#pragma unroll
+        for (int r = 0; r < NROWS; ++r) {
+            const uint8_t bit = NROWS == 1 ? kAll : (uint8_t)(1u << r);
+            const uint32_t T = (uint32_t)__builtin_amdgcn_readfirstlane((int)sl.T[r]);
+            int take = __builtin_amdgcn_readfirstlane(sl.take[r]);
+            const uint32_t key = keys[r * 64 * C + 64 * j + lane];
+            bool in = key > T;
+            if (take == kTakeAll) {
+                in = key >= T;
+            } else if (take > 0) {
+                for (int i = 0; i < j; ++i) take -= __popcll(__ballot(keys[r * 64 * C + 64 * i + lane] == T));
+                in = in || (key == T && (int)lanes_below(__ballot(key == T)) < take);
+            }
+            qm[u] |= in ? bit : (uint8_t)0;
+        }
+        const int i = 64 * j + lane;
+        in_list[u] = i < P && !fp.contains(i) && qm[u] != 0;
+        bal[u] = __ballot(in_list[u]);
+        if (lane == 0) sl.cnt[j] = __popcll(bal[u]);
+    }
+    lds_barrier();
     // The list: the forced pages first (ascending; forced_page() gives entry f
     // without the selection), then every other selected page ascending.
-    const ForcedPages fp = forced_pages(P, num_sinks, window);
-    int n = fp.count;
+    const int own = lane < C ? sl.cnt[lane] : 0;
+    const int before = fp.count + wave_incl_sum(own);      // lane j: the list's length after chunk j
+    const int n = __builtin_amdgcn_readlane(before, 63);
 #pragma unroll
-    for (int j = 0; j < C; ++j) {
+    for (int u = 0; u < CW; ++u) {
+        const int j = w + NW * u;
+        if (j >= C) continue;
         const int i = 64 * j + lane;
-        const bool forced = i < P && fp.contains(i);
-        const bool f = i < P && !forced && qm[j] != 0;
-        const uint64_t bal = __ballot(f);
-        if (j % NW == w) {
-            if (forced) entries[fp.index(i)] = i | ((int)kAll << 16);
-            if (f) entries[n + (int)lanes_below(bal)] = i | ((int)qm[j] << 16);
-        }
-        n += __popcll(bal);
+        const int at = __builtin_amdgcn_readlane(before, j) - __popcll(bal[u]);
+        if (i < P && fp.contains(i)) entries[fp.index(i)] = i | ((int)kAll << 16);
+        if (in_list[u]) entries[at + (int)lanes_below(bal[u])] = i | ((int)qm[u] << 16);
     }
     lds_barrier();
     return n;
