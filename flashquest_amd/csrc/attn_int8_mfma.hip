@@ -277,8 +277,9 @@ void attn_int8_mfma_kernel(Int8Params a) {
         if (a.sel.mask_out && split == 0)            // uniform: the caller asked for the selection
             block_write_mask<NT, NREP>(s_ent, total, c.P, (uint8_t*)s_key, a.sel.mask_out + (int64_t)g * NREP * c.P,
                                        tid);
-        e0 = (int)((int64_t)total * split / a.splits);
-        e1 = (int)((int64_t)total * (split + 1) / a.splits);
+        const int lead = a.tail.in_kernel ? kTailLead : 0;
+        e0 = split_begin(total, split, a.splits, lead);
+        e1 = split_begin(total, split + 1, a.splits, lead);
     } else {
         const int n_sel = a.ws.n_sel[g];
         e0 = (int)((int64_t)n_sel * split / a.splits);

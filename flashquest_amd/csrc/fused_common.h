@@ -25,6 +25,17 @@ FQ_DEV float row16_max(float v) {
     v = fmaxf(v, dpp<kDppXor1>(v));
     return fmaxf(v, dpp<kDppXor2>(v));
 }
+
+// Where split `split` of `splits` begins in a group's list of `total` entries
+// (the last ends at split_begin(splits)): balanced slices, split 0 `lead`
+// entries shorter than the others.  The partial-page tail is split 0's work:
+// attending 64 tokens takes it 2.6 us, as long as one page of each wave
+// (kTailLead entries), and with equal slices the whole step waited for it.
+constexpr int kTailLead = 8;
+FQ_DEV int split_begin(int total, int split, int splits, int lead) {
+    if (lead > 0) lead = splits > 1 ? min(lead, total / (splits - 1)) : 0;      // uniform
+    return max(0, (int)((int64_t)(total + lead) * split / splits) - lead);
+}
 FQ_DEV float lane_value(float v, int lane) { return __int_as_float(__builtin_amdgcn_readlane(__float_as_int(v), lane)); }
 
 
