@@ -429,10 +429,16 @@ static bool decode_selects_in_attention(const Int4Cache& c, const QueryArgs& q, 
 // to fill the GPU) score each group once in a scoring launch over all CUs; the
 // attention workgroups then select from those scores (kSelectOnly) instead of
 // each re-scoring the group's pages.  INT4 and INT8, unrotated; with head_dim
-// 64 every such step (those kernels have no scorer of their own).
+// 64 every such step (those kernels have no scorer of their own).  Up to
+// kSplitScorePages pages the redundant scoring in every split is cheaper than the
+// launch it saves: one layer of 8 groups, with the scoring launch and without, 64
+// pages 19.9 / 17.4 us, 128 pages 20.5 / 18.8, 160 pages 21.4 / 20.1, 192 pages
+// 21.5 / 21.0 (INT8 23.7 / 23.9), 256 pages 23.3 / 24.6; 128 groups, 160 pages 35.5
+// / 33.5.
+constexpr int kSplitScorePages = 160;
 static bool attend_from_scores(const Int4Cache& c, const QueryArgs& q, int bound) {
     if (c.D == 64) return true;
-    return c.L * c.B * c.Hkv < 192 && !q.rot && bound > kFusedSmallPages;
+    return c.L * c.B * c.Hkv < 192 && !q.rot && bound > kFusedSmallPages && c.P > kSplitScorePages;
 }
 
 // 6 or 8 query heads per KV head on the INT4 / INT8 matrix-core decode,
