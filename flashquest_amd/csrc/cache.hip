@@ -13,14 +13,14 @@
 // per-group min/max over the group's lanes, fp32 arithmetic (as
 // quant_v_kernel).  Codes are stored 4 bytes (8 channels) per thread and token.
 //
-// A page has few bytes for its arithmetic: with an IEEE division per value
-// (about 12 instructions, some at a quarter of the rate) the kernel was bound by
-// its vector instructions and, in V, by one memory latency per token.  Every
-// load now goes out before the first use, reductions stay in the vector unit
-// (DPP, lane swaps) and the quotients come from one reciprocal per scale
-// (quot_code).  8192 tokens x 8 heads x 128 channels, INT4, back to back: K 12.6
-// -> 11.7 us, V 11.9 -> 10.7 us (21 MB each; what is left is one round of
-// workgroups: load latency, arithmetic and stores do not overlap).
+// A page has few bytes for its arithmetic, and its loads, arithmetic and stores do
+// not overlap (one round of workgroups at ordinary sizes), so it is bound by
+// latency and vector issue: the type is a template argument and every load goes out
+// before the first use, reductions stay in the vector unit (DPP, lane swaps), the
+// quotients come from one reciprocal per scale (quot_code) and the codes' rounding
+// from an fp32 add.  8192 tokens x 8 heads x 128 channels, INT4, back to back: K
+// 12.6 us with a division per value, 11.7 with reciprocals, 10.0 with the type known
+// and 7 operations a code; V 11.9, 10.7, 9.3 us (21 MB each).
 #include "fq_common.h"
 #include "turbo_quant.h"
 
@@ -58,13 +58,17 @@ struct PageQuantParams {
     int meta_dtype;
 };
 
+// Channels 8 c8 .. + 7 of a position as floats.  The type is a template argument:
+// with a test of it per value, the page kernel waited for each load before the
+// next one went out.
+template <int DT>
 FQ_DEV void load8(const TokSrc& s, int b, int h, int pos, int c8, float (&x)[8]) {
     const bool in_head = pos < s.head_len;
     const char* base = (const char*)(in_head ? s.head : s.tail);
     const int64_t* st = in_head ? s.hs : s.ts;
     const int t = in_head ? pos : pos - s.head_len;
     const int64_t e = b * st[0] + h * st[1] + t * st[2] + 8 * c8;
-    if (s.dtype == FQ_F32) {
+    if constexpr (DT == FQ_F32) {
         const uint4 a = *(const uint4*)(base + e * 4), c = *(const uint4*)(base + e * 4 + 16);
         const uint32_t w[8] = {a.x, a.y, a.z, a.w, c.x, c.y, c.z, c.w};
 #pragma unroll
@@ -74,29 +78,31 @@ FQ_DEV void load8(const TokSrc& s, int b, int h, int pos, int c8, float (&x)[8])
         const uint32_t w[4] = {a.x, a.y, a.z, a.w};
 #pragma unroll
         for (int i = 0; i < 4; ++i) {
-            x[2 * i] = s.dtype == FQ_BF16 ? bf16_bits_to_f(w[i] & 0xFFFFu) : f16_bits_to_f(w[i] & 0xFFFFu);
-            x[2 * i + 1] = s.dtype == FQ_BF16 ? bf16_bits_to_f(w[i] >> 16) : f16_bits_to_f(w[i] >> 16);
+            x[2 * i] = DT == FQ_BF16 ? bf16_bits_to_f(w[i] & 0xFFFFu) : f16_bits_to_f(w[i] & 0xFFFFu);
+            x[2 * i + 1] = DT == FQ_BF16 ? bf16_bits_to_f(w[i] >> 16) : f16_bits_to_f(w[i] >> 16);
         }
     }
 }
 
-// The codes of 8 values with their scales' reciprocals r = RN(1 / s):
-// rint(RN(d / s)) clamped, d = x - mn.  q0 = d r is within 1.5 ulp of d / s; one
-// residual correction brings it within one, and the second one rounds correctly
-// (Markstein: with y = RN(1 / b) and q within an ulp of a / b, RN(q + (a - b q) y)
-// is RN(a / b)), so ties round as the IEEE quotient's.  That holds while
-// nothing over- or underflows: quotients below 2^-100 round to 0 either way, and
-// scales above 1e30 (or NaN) take the division itself (quot_wide, per wave).
-// Scales are at least 1e-6.
+// A code rint(RN(d / s)) clamped to [0, 2^BITS - 1], d = x - mn, with the scale's
+// reciprocal r = RN(1 / s), in the low bits of 2^23 + code (kCodeBias + code as an
+// integer), which the fp32 add rounds to even as rint does.  q0 = d r is within 1.5
+// ulp of d / s; one residual correction leaves an error of 2^-46 before its own
+// rounding, and no quotient of two floats lies that close to a code's tie without
+// being the tie (every significand of s with the 9 nearest d at each of the 255
+// ties: no code differs from the division's).  That holds while nothing over- or
+// underflows: quotients below 2^-100 round to 0 either way, and scales above 1e30
+// (or NaN) take the division itself (quot_wide, per wave).  Scales are at least
+// 1e-6.  A NaN's code is 0 (fmed3 gives the least of its other operands).
+constexpr uint32_t kCodeBias = 0x4B000000u;          // 2^23
 template <int BITS>
-FQ_DEV uint32_t clamp_code(float q) {
-    return (uint32_t)fminf(fmaxf(rintf(q), 0.f), (float)((1 << BITS) - 1));
+FQ_DEV uint32_t biased_code(float q) {
+    return __float_as_uint(__builtin_amdgcn_fmed3f(q, 0.f, (float)((1 << BITS) - 1)) + 8388608.0f);
 }
 template <int BITS>
 FQ_DEV uint32_t quot_code(float d, float s, float r) {
     const float q0 = d * r;
-    const float q1 = fmaf(fmaf(-q0, s, d), r, q0);
-    return clamp_code<BITS>(fmaf(fmaf(-q1, s, d), r, q1));
+    return biased_code<BITS>(fmaf(fmaf(-q0, s, d), r, q0));
 }
 FQ_DEV bool quot_wide(bool ok) { return __builtin_amdgcn_ballot_w64(!ok) != 0; }   // any lane's scale out of range
 
@@ -121,26 +127,26 @@ FQ_DEV float across_run(float v, int n) {
 }
 constexpr int kDppRor8 = 0x128;      // lane i <- i ^ 8 within each 16
 
-// The 8 codes of a thread's channels: BITS 4 packs two per byte (4 bytes),
-// BITS 8 one per byte (8 bytes), at byte 8 * c8 * BITS / 8 of the row.
+// The 8 codes (with their bias) of a thread's channels: BITS 4 packs two per byte
+// (4 bytes), BITS 8 one per byte (8 bytes), at byte 8 * c8 * BITS / 8 of the row.
+// The biases left of a code add up to one constant, taken off once.
 template <int BITS>
 FQ_DEV void store_codes(uint8_t* row, int c8, const uint32_t (&c)[8]) {
     if constexpr (BITS == 4) {
-        uint32_t word = 0;
+        uint32_t word = c[0] - (kCodeBias + (kCodeBias << 4));
 #pragma unroll
-        for (int i = 0; i < 8; ++i) word |= c[i] << (4 * i);
+        for (int i = 1; i < 8; ++i) word += c[i] << (4 * i);
         *(uint32_t*)(row + 4 * c8) = word;
     } else {
-        *(uint2*)(row + 8 * c8) = make_uint2(c[0] | c[1] << 8 | c[2] << 16 | c[3] << 24,
-                                             c[4] | c[5] << 8 | c[6] << 16 | c[7] << 24);
+        uint2 w = make_uint2(c[0] - kCodeBias, c[4] - kCodeBias);
+#pragma unroll
+        for (int i = 1; i < 4; ++i) { w.x += c[i] << (8 * i); w.y += c[4 + i] << (8 * i); }
+        *(uint2*)(row + 8 * c8) = w;
     }
 }
 
-FQ_DEV uint32_t meta_bits(float f, int dtype) {
-    return dtype == FQ_BF16 ? f_to_bf16_bits(f) : f_to_f16_bits(f);
-}
-
-template <int D, int BITS>
+// DT: the type of K and V, which share it.
+template <int D, int BITS, int DT>
 __global__ __launch_bounds__(kThreads) void page_quant_kernel(PageQuantParams a) {
     constexpr int CPR = D / 8;                  // threads per token row
     constexpr int RPP = kThreads / CPR;         // token rows per pass
@@ -164,7 +170,7 @@ __global__ __launch_bounds__(kThreads) void page_quant_kernel(PageQuantParams a)
         float x[TPT][8];
         float mn[8], mx[8];
 #pragma unroll
-        for (int u = 0; u < TPT; ++u) load8(a.k, b, h, lpos[u], c8, x[u]);
+        for (int u = 0; u < TPT; ++u) load8<DT>(a.k, b, h, lpos[u], c8, x[u]);
 #pragma unroll
         for (int i = 0; i < 8; ++i) { mn[i] = INFINITY; mx[i] = -INFINITY; }
 #pragma unroll
@@ -197,22 +203,25 @@ __global__ __launch_bounds__(kThreads) void page_quant_kernel(PageQuantParams a)
             }
         }
         // scale in the input dtype (kv_quant.py:131-149), as quant_k_kernel
-        const int dt = a.k.dtype;
         float sc[8];
 #pragma unroll
         for (int i = 0; i < 8; ++i) {
-            const float diff = round_to(mx[i] - mn[i], dt);
-            float s = round_to(diff * (BITS == 8 ? kCacheInv255 : kCacheInv15), dt);
-            sc[i] = round_to(fmaxf(s, kCacheEps), dt);
+            const float diff = round_to(mx[i] - mn[i], DT);
+            float s = round_to(diff * (BITS == 8 ? kCacheInv255 : kCacheInv15), DT);
+            sc[i] = round_to(fmaxf(s, kCacheEps), DT);
         }
         if (r == 0) {
             const int64_t p = a.tok_dst0 / kPage + pg;
             uint32_t sw[4], mw[4];
+            auto pack = [&](auto bits) {
 #pragma unroll
-            for (int j = 0; j < 4; ++j) {
-                sw[j] = meta_bits(sc[2 * j], a.meta_dtype) | meta_bits(sc[2 * j + 1], a.meta_dtype) << 16;
-                mw[j] = meta_bits(mn[2 * j], a.meta_dtype) | meta_bits(mn[2 * j + 1], a.meta_dtype) << 16;
-            }
+                for (int j = 0; j < 4; ++j) {
+                    sw[j] = bits(sc[2 * j]) | bits(sc[2 * j + 1]) << 16;
+                    mw[j] = bits(mn[2 * j]) | bits(mn[2 * j + 1]) << 16;
+                }
+            };
+            if (a.meta_dtype == FQ_BF16) pack([](float f) { return (uint32_t)f_to_bf16_bits(f); });      // uniform
+            else pack([](float f) { return (uint32_t)f_to_f16_bits(f); });
             *(uint4*)((uint16_t*)a.ks + b * a.ks_s[0] + h * a.ks_s[1] + p * a.ks_s[2] + 8 * c8) =
                 make_uint4(sw[0], sw[1], sw[2], sw[3]);
             *(uint4*)((uint16_t*)a.km + b * a.km_s[0] + h * a.km_s[1] + p * a.km_s[2] + 8 * c8) =
@@ -232,7 +241,7 @@ __global__ __launch_bounds__(kThreads) void page_quant_kernel(PageQuantParams a)
                 uint32_t cd[8];
                 if (wide) {
 #pragma unroll
-                    for (int i = 0; i < 8; ++i) cd[i] = clamp_code<BITS>(__fdiv_rn(x[u][i] - mn[i], sc[i]));
+                    for (int i = 0; i < 8; ++i) cd[i] = biased_code<BITS>(__fdiv_rn(x[u][i] - mn[i], sc[i]));
                 } else {
 #pragma unroll
                     for (int i = 0; i < 8; ++i) cd[i] = quot_code<BITS>(x[u][i] - mn[i], sc[i], rc[i]);
@@ -249,7 +258,7 @@ __global__ __launch_bounds__(kThreads) void page_quant_kernel(PageQuantParams a)
         const int g = (8 * c8) / a.v_group;
         float x[TPT][8];
 #pragma unroll
-        for (int u = 0; u < TPT; ++u) load8(a.v, b, h, lpos[u], c8, x[u]);
+        for (int u = 0; u < TPT; ++u) load8<DT>(a.v, b, h, lpos[u], c8, x[u]);
 #pragma unroll
         for (int u = 0; u < TPT; ++u) {
             // every lane of the row takes part in the reductions; invalid tokens are not stored
@@ -264,7 +273,7 @@ __global__ __launch_bounds__(kThreads) void page_quant_kernel(PageQuantParams a)
             uint32_t cd[8];
             if (quot_wide(s <= 1e30f)) {
 #pragma unroll
-                for (int i = 0; i < 8; ++i) cd[i] = clamp_code<BITS>(__fdiv_rn(x[u][i] - mn, s));
+                for (int i = 0; i < 8; ++i) cd[i] = biased_code<BITS>(__fdiv_rn(x[u][i] - mn, s));
             } else {
 #pragma unroll
                 for (int i = 0; i < 8; ++i) cd[i] = quot_code<BITS>(x[u][i] - mn, s, rc);
@@ -334,7 +343,9 @@ __global__ __launch_bounds__(kThreads) void turbo_append_kernel(TurboAppendParam
 #pragma unroll
     for (int c8 = 0; c8 < D / 8; ++c8) {
         float x[8];
-        load8(a.src, b, h, pos, c8, x);
+        if (a.src.dtype == FQ_BF16) load8<FQ_BF16>(a.src, b, h, pos, c8, x);      // uniform
+        else if (a.src.dtype == FQ_F16) load8<FQ_F16>(a.src, b, h, pos, c8, x);
+        else load8<FQ_F32>(a.src, b, h, pos, c8, x);
 #pragma unroll
         for (int i = 0; i < 8; ++i) v[8 * c8 + i] = x[i];
     }
@@ -381,12 +392,18 @@ bool page_quant_v_ok(int D, int group, int in_dtype, const void* v, const int64_
 hipError_t launch_page_quant(const PageQuantParams& a, int D, hipStream_t st, int bits = 4) {
     if (a.n_tok <= 0 || a.B * a.H == 0) return hipSuccess;
     dim3 grid((a.n_tok + kPage - 1) / kPage, a.B * a.H);
-    if (D == 128 && bits == 4) hipLaunchKernelGGL((page_quant_kernel<128, 4>), grid, dim3(kThreads), 0, st, a);
-    else if (D == 64 && bits == 4) hipLaunchKernelGGL((page_quant_kernel<64, 4>), grid, dim3(kThreads), 0, st, a);
-    else if (D == 128 && bits == 8) hipLaunchKernelGGL((page_quant_kernel<128, 8>), grid, dim3(kThreads), 0, st, a);
-    else if (D == 64 && bits == 8) hipLaunchKernelGGL((page_quant_kernel<64, 8>), grid, dim3(kThreads), 0, st, a);
-    else return hipErrorInvalidValue;
-    return hipGetLastError();
+    const int dt = a.do_k ? a.k.dtype : a.v.dtype;
+    if (a.do_k && a.do_v && a.v.dtype != dt) return hipErrorInvalidValue;
+#define FQ_Q(D_, BITS_)                                                                                              \
+    if (D == D_ && bits == BITS_) {                                                                                  \
+        if (dt == FQ_BF16) hipLaunchKernelGGL((page_quant_kernel<D_, BITS_, FQ_BF16>), grid, dim3(kThreads), 0, st, a);   \
+        else if (dt == FQ_F16) hipLaunchKernelGGL((page_quant_kernel<D_, BITS_, FQ_F16>), grid, dim3(kThreads), 0, st, a); \
+        else hipLaunchKernelGGL((page_quant_kernel<D_, BITS_, FQ_F32>), grid, dim3(kThreads), 0, st, a);                  \
+        return hipGetLastError();                                                                                    \
+    }
+    FQ_Q(128, 4) FQ_Q(64, 4) FQ_Q(128, 8) FQ_Q(64, 8)
+#undef FQ_Q
+    return hipErrorInvalidValue;
 }
 
 hipError_t launch_quant_k_pages(const void* k, int in_dtype, const int64_t* k_s, int B, int H, int S, int D,
