@@ -808,8 +808,9 @@ MfmaSplit mfma_splits(int groups, int max_entries, int s_max, int request) {
 
 // The fused decode: one workgroup of 8 waves per KV group when the groups
 // fill the GPU; otherwise every group is split over enough workgroups for one
-// per CU, each scoring and selecting the group's pages itself (the same list
-// in every split) and attending a balanced slice of it, at least 8 pages.
+// per CU, each selecting the group's pages itself (the same list in every split,
+// from its own scores or a scoring launch's) and attending a balanced slice of it
+// (split_begin), at least 8 pages.
 int fused_splits(int groups, int max_entries, int s_max) {
     if (groups >= 192 || max_entries <= kFusedSmallPages) return 1;
     int s = (256 + groups - 1) / std::max(groups, 1);

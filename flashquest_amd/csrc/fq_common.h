@@ -19,7 +19,8 @@ constexpr int kNoPage = 0x7FFF;
 // A decode step whose lists hold at most this many pages per KV group runs as
 // one launch with one workgroup per group (it scores, selects and attends
 // itself: a few pages per wave) even when the groups do not fill the GPU;
-// longer lists split each group over workgroups behind a scoring launch.
+// longer lists split each group over workgroups (behind a scoring launch where
+// scoring the group in each of them would cost more).
 constexpr int kFusedSmallPages = 40;
 constexpr int kMaxRows = 16;       // query rows per KV group in scoring (n_rep * S_q)
 constexpr float kLog2e = 1.4426950408889634f;

@@ -371,8 +371,8 @@ __global__ __launch_bounds__(kThreads) void select_groups_rows_kernel(GroupSelec
 // layer's decode step) and for long contexts; P <= 64 C.  The list puts the
 // forced pages first.  A wave alone spends the time on its own LDS counts and
 // lists: scoring and selection of 224 groups x 2048 pages with 3 query heads each,
-// 95.0 -> 72.3 us per query head and 59.6 -> 55.7 from one summed row; 1024
-// pages 42.4 -> 40.6 per query head.
+// 95.0 -> 65.3 us per query head and 59.6 -> 55.3 from one summed row; 1024
+// pages 42.4 -> 37.7 per query head.
 // ---------------------------------------------------------------------------
 template <int NREP, int C>
 __global__ __launch_bounds__(512) void select_groups_block_kernel(GroupSelectParams a) {
