@@ -114,12 +114,14 @@ FQ_DEV void load_half(HalfBuf& b, const Int8Rsrc& r, int p, int hp, int n16, int
 // chunk selects the same pages.  The chunks of a cache head are mapped to one
 // XCD so that the second one's page reads hit that XCD's L2.
 //
-// D = 64: half the channels (one q.k step, four p.v tiles); its FUSED form
+// D = 64: half the channels (one q.k step, four p.v tiles), and both products in
+// wider fixed point (fused_common.h, wide_scale); its FUSED form
 // always selects from the scores of a scoring launch, as the INT4 kernel's.
 template <int D, typename MT, int NREP, bool FUSED, bool HCH = false>
 __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2)))
 void attn_int8_mfma_kernel(Int8Params a) {
     static_assert(D == 128 || D == 64, "head_dim");
+    static_assert((int64_t)kMaxWgPages / 8 * 64 * 128 * 128 < INT32_MAX, "a wave's int32 sums (64 channels)");
     constexpr int NW = 8, NT = 512;
     constexpr int QKS = D / 64;                     // q.k k-steps; also the query heads a lane makes digits for
     constexpr int NTL = D / 16;                     // p.v channel tiles
@@ -301,15 +303,22 @@ void attn_int8_mfma_kernel(Int8Params a) {
 
     auto entry_of = [&](int k) { return __builtin_amdgcn_readfirstlane(s_ent[ent_base + w + NW * k]); };
 
-    constexpr bool kBound = std::is_same<MT, bf16>::value;
+    constexpr bool kWide = D == 64;          // as the INT4 kernel's
+    constexpr bool kBound = kWide || std::is_same<MT, bf16>::value;
     float m_run[NREP];
 #pragma unroll
     for (int r = 0; r < NREP; ++r) m_run[r] = -INFINITY;
     float s_run = kBound ? 0.f : 1.f, inv_s = 1.f;
     float m_lane = 0.f;
     v4f pacc[NTL];
+    v4i iacc[NTL];          // kWide: head lg's digit rows since the references last moved,
+    float facc[NTL];        // and what came before
 #pragma unroll
-    for (int t = 0; t < NTL; ++t) pacc[t] = (v4f){0.f, 0.f, 0.f, 0.f};
+    for (int t = 0; t < NTL; ++t) {
+        pacc[t] = (v4f){0.f, 0.f, 0.f, 0.f};
+        iacc[t] = (v4i){0, 0, 0, 0};
+        facc[t] = 0.f;
+    }
     float l_acc = 0.f, bias = 0.f;
     float Cr = 0.f, unscale = 0.f;           // the current page's q.K_mn + 128 sum A (head lg), digit scale
 
@@ -344,12 +353,30 @@ void attn_int8_mfma_kernel(Int8Params a) {
                     amax = fmaxf(amax, fabsf(Av[hh][j]));
                 }
             }
-            const float sigma = wave_max(amax);
-            const float inv = sigma > 0.f ? kQkScale8 * __builtin_amdgcn_rcpf(sigma) : 0.f;
             const int s = c0 >> 6, kg = (c0 >> 4) & 3, bo = c0 & 15;
+            if constexpr (kWide) {           // 16 lanes per head: the lane's own head's references
+                const WideScale ws = wide_scale(row16_max(amax));
+                unscale = ws.unscale;
+                if (r0 < NREP) {
+                    uint32_t Y[4];
 #pragma unroll
-            for (int hh = 0; hh < QKS; ++hh) {
-                if (r0 + hh < NREP) {
+                    for (int j = 0; j < 4; ++j) {
+                        Y[j] = wide_digits(Av[0][j], ws.scale);
+                        cpart[0] = fmaf(Av[0][j], 0.f, cpart[0]);        // an infinite or NaN A has no digits
+                    }
+                    const int row = 4 * r0;
+                    *(uint32_t*)&W.aqk[s][row][swz8(row, kg)][bo] = byte_of4<3>(Y[0], Y[1], Y[2], Y[3]) ^ kFlip8;
+                    *(uint32_t*)&W.aqk[s][row + 1][swz8(row + 1, kg)][bo] = byte_of4<2>(Y[0], Y[1], Y[2], Y[3]) ^ kFlip8;
+                    *(uint32_t*)&W.aqk[s][row + 2][swz8(row + 2, kg)][bo] = byte_of4<1>(Y[0], Y[1], Y[2], Y[3]) ^ kFlip8;
+                    *(uint32_t*)&W.aqk[s][row + 3][swz8(row + 3, kg)][bo] = byte_of4<0>(Y[0], Y[1], Y[2], Y[3]) ^ kFlip8;
+                }
+            } else {
+                const float sigma = wave_max(amax);
+                const float inv = sigma > 0.f ? kQkScale8 * __builtin_amdgcn_rcpf(sigma) : 0.f;
+                unscale = sigma * (1.0f / kQkScale8);
+#pragma unroll
+                for (int hh = 0; hh < QKS; ++hh) {
+                    if (r0 + hh >= NREP) continue;
                     uint32_t Y[4];
 #pragma unroll
                     for (int j = 0; j < 4; ++j) Y[j] = (uint32_t)fmaf(Av[hh][j], inv, 8421504.0f);
@@ -358,6 +385,9 @@ void attn_int8_mfma_kernel(Int8Params a) {
                     *(uint32_t*)&W.aqk[s][row + 1][swz8(row + 1, kg)][bo] = byte_of4<1>(Y[0], Y[1], Y[2], Y[3]) ^ kFlip8;
                     *(uint32_t*)&W.aqk[s][row + 2][swz8(row + 2, kg)][bo] = byte_of4<0>(Y[0], Y[1], Y[2], Y[3]) ^ kFlip8;
                 }
+            }
+#pragma unroll
+            for (int hh = 0; hh < QKS; ++hh) {
                 float cs = fmaf(apart[hh], 128.0f, cpart[hh]);       // q.K_mn + 128 sum A over this lane's channels
                 if constexpr (D == 128) cs += __shfl_xor(cs, 16, 64);
                 cpart[hh] = row_sum<16>(cs);
@@ -368,7 +398,6 @@ void attn_int8_mfma_kernel(Int8Params a) {
                 const float x1 = __shfl(cpart[1], (lg >> 1) * 32, 64);
                 Cr = (lg & 1) ? x1 : x0;
             }
-            unscale = sigma * (1.0f / kQkScale8);
             __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
         }
         const v4i a0 = *(const v4i*)&W.aqk[0][n16][swz8(n16, lg)][0];
@@ -383,7 +412,8 @@ void attn_int8_mfma_kernel(Int8Params a) {
             v4i acc = {0, 0, 0, 0};
             acc = __builtin_amdgcn_mfma_i32_16x16x64_i8(a0, bk0, acc, 0, 0, 0);
             if constexpr (D == 128) acc = __builtin_amdgcn_mfma_i32_16x16x64_i8(a1, bk1, acc, 0, 0, 0);
-            const float f = fmaf((float)acc[0], 65536.f, fmaf((float)acc[1], 256.f, (float)acc[2]));
+            const float f = kWide ? digit_rows(acc)
+                                  : fmaf((float)acc[0], 65536.f, fmaf((float)acc[1], 256.f, (float)acc[2]));
             const float lgt = fmaf(f, unscale, Cr);
             const bool ok = lg < NREP && ((qm >> lg) & 1) && tok0 + 16 * t + n16 < S;
             lg2[t] = ok ? lgt : -INFINITY;
@@ -395,7 +425,7 @@ void attn_int8_mfma_kernel(Int8Params a) {
         for (int t = 0; t < 2; ++t) {
             vs_t[t] = half_to_f<MT>(cb.vs[t]);
             vm_t[t] = half_to_f<MT>(cb.vm[t]);
-            sp = fmaxf(sp, vs_t[t]);
+            sp = fmaxf(sp, kWide ? fabsf(vs_t[t]) : vs_t[t]);
         }
         mp = row16_max(mp);
         bool grow = false;
@@ -419,10 +449,10 @@ void attn_int8_mfma_kernel(Int8Params a) {
             }
             float as = 1.0f;
             if constexpr (kBound) {
-                const float sn = sp > s_run ? 2.0f * sp : s_run;
+                const float sn = sp > s_run ? (kWide ? wide_bound(sp) : 2.0f * sp) : s_run;
                 as = sn > 0.f ? s_run / sn : 1.0f;
                 s_run = sn;
-                inv_s = sn > 0.f ? 1.0f / sn : 0.f;
+                inv_s = sn > 0.f ? (kWide ? kWideOne : 1.0f) / sn : 0.f;
             }
             float am_lg = am[0], ml = m_run[0];
 #pragma unroll
@@ -433,11 +463,20 @@ void attn_int8_mfma_kernel(Int8Params a) {
             m_lane = ml == -INFINITY ? 0.f : ml;
             l_acc *= am_lg;
             bias *= am_lg;
+            if constexpr (kWide) {
+                const float f = am_lg * as;
 #pragma unroll
-            for (int r = 0; r < 4; ++r) {
-                const float f = r < NREP ? am[r] * as : 0.f;
+                for (int t = 0; t < NTL; ++t) {
+                    facc[t] = (facc[t] + digit_rows(iacc[t])) * f;
+                    iacc[t] = (v4i){0, 0, 0, 0};
+                }
+            } else {
 #pragma unroll
-                for (int t = 0; t < NTL; ++t) pacc[t][r] *= f;
+                for (int r = 0; r < 4; ++r) {
+                    const float f = r < NREP ? am[r] * as : 0.f;
+#pragma unroll
+                    for (int t = 0; t < NTL; ++t) pacc[t][r] *= f;
+                }
             }
         }
         // ---- p.v A: p * V_scale (/ s_run) in fp16; operand k = 8 kg + 2 ai + jj is
@@ -447,7 +486,42 @@ void attn_int8_mfma_kernel(Int8Params a) {
         for (int t = 0; t < 2; ++t) {
             pr[t] = exp2_fast(lg2[t] - m_lane);
             l_acc += pr[t];
-            bias = fmaf(pr[t], vm_t[t], bias);
+            // kWide's codes are code - 128
+            bias = fmaf(pr[t], kWide ? fmaf(vs_t[t], 128.f, vm_t[t]) : vm_t[t], bias);
+        }
+        if constexpr (kWide) {
+            // A: the digits of p * V_scale / s_run in rows 4 head + digit, operand k as
+            // below, one byte each: the lane's two tokens are two bytes of a row
+            uint32_t Y[2];
+#pragma unroll
+            for (int t = 0; t < 2; ++t) {
+                const float x = pr[t] * vs_t[t];
+                bias = fmaf(x, 0.f, bias);           // an infinite or NaN product has no digits
+                Y[t] = wide_digits(x, inv_s) ^ kFlip8;
+            }
+            if (lg < NREP) {
+                uint8_t* dst = &W.apv[4 * lg][(n16 & 3) ^ lg][2 * (n16 >> 2)];
+#pragma unroll
+                for (int d = 0; d < 4; ++d)
+                    *(uint16_t*)(dst + 64 * d) = (uint16_t)(((Y[0] >> (24 - 8 * d)) & 255u) |
+                                                            (((Y[1] >> (24 - 8 * d)) & 255u) << 8));
+            }
+            __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
+            const int64_t ad = *(const int64_t*)&W.apv[n16][lg ^ ((n16 >> 2) & 3)][0];
+#pragma unroll
+            for (int j = 0; j < NTL; ++j) {
+                uint32_t bw[2];
+#pragma unroll
+                for (int i = 0; i < 2; ++i) {
+                    const uint32_t sel = 0x0C0C0400u + 0x0101u * j;
+                    const uint32_t t01 = __builtin_amdgcn_perm(cb.vw[4 * i + 1].x, cb.vw[4 * i].x, sel);
+                    const uint32_t t23 = __builtin_amdgcn_perm(cb.vw[4 * i + 3].x, cb.vw[4 * i + 2].x, sel);
+                    bw[i] = (t01 | (t23 << 16)) ^ kFlip8;
+                }
+                iacc[j] = __builtin_amdgcn_mfma_i32_16x16x32_i8(ad, (int64_t)((uint64_t)bw[1] << 32 | bw[0]), iacc[j], 0, 0, 0);
+            }
+            __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
+            return;
         }
         if (lg < NREP) {
             float x0 = pr[0] * vs_t[0], x1 = pr[1] * vs_t[1];
@@ -505,13 +579,29 @@ void attn_int8_mfma_kernel(Int8Params a) {
 
     // ---- wave state -> LDS (head r in lane group 0 component r; channel NTL n16 + j)
     // the lo rows 4 + r (lane group 1) join the hi rows
+    if constexpr (!kWide) {
 #pragma unroll
-    for (int j = 0; j < NTL; ++j)
+        for (int j = 0; j < NTL; ++j)
 #pragma unroll
-        for (int r = 0; r < NREP; ++r) pacc[j][r] += __shfl_xor(pacc[j][r], 16, 64);
+            for (int r = 0; r < NREP; ++r) pacc[j][r] += __shfl_xor(pacc[j][r], 16, 64);
+    }
     l_acc = row_sum<16>(l_acc);
     bias = row_sum<16>(bias);
-    const float pv_unscale = s_run * kSubnormal8;
+    const float pv_unscale = s_run * (kWide ? 1.0f / kWideOne : kSubnormal8);
+    if constexpr (kWide) {      // head lg's outputs of the lane's channels
+        if (lg < NREP) {
+#pragma unroll
+            for (int j = 0; j < NTL; ++j)
+                s_split.acc[w][lg][NTL * n16 + j] = fmaf(facc[j] + digit_rows(iacc[j]), pv_unscale, bias);
+            if (n16 == 0) {
+                float m = m_run[0];
+#pragma unroll
+                for (int r = 1; r < NREP; ++r) m = lg == r ? m_run[r] : m;
+                s_split.m[w][lg] = m;
+                s_split.l[w][lg] = l_acc;
+            }
+        }
+    } else
 #pragma unroll
     for (int r = 0; r < NREP; ++r) {
         const float ll = __shfl(l_acc, 16 * r + n16, 64);

@@ -152,25 +152,25 @@ FQ_DEV void load_page(PageBuf& b, const SliceRsrc& r, int koff, int voff, int mo
 // HCH (FUSED only): head chunks, sel.head_chunks virtual KV heads per cache
 // KV head (a separate instantiation, so the other kernels are unchanged).
 //
-// D = 64: the same page math with half the channels (one q.k step, four p.v
-// tiles).  Its FUSED form always selects from the scores of a scoring launch
+// D = 64: half the channels (one q.k step, four p.v tiles), and both products in
+// wider fixed point (fused_common.h, wide_scale).  Its FUSED form always selects from the scores of a scoring launch
 // (attend_from_scores): a page's 64-channel metadata is too little per
 // workgroup to be worth a second in-kernel scorer.  It replaces the VALU
 // kernel of attn_int4.hip, which is bound by its multiply-adds (59 us of a
 // 111 us step of 4 sequences x 16393 tokens, 32 / 8 heads, that also had to
-// attend the partial page in launches of its own; this way the step is 30 us,
-// most of it host time).
+// attend the partial page in launches of its own; this way the step is 22 us).
 template <int D, typename MT, int G, int NREP, int NW, bool FUSED, bool HCH = false>
 __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(2, 2)))
 void attn_int4_mfma_kernel(MfmaParams a) {
     static_assert(!FUSED || NW == 8, "in-kernel selection runs in the 8-wave kernel");
     static_assert(!HCH || FUSED, "head chunks run in the fused kernel");
+    static_assert((int64_t)kMaxWgPages / NW * 64 * 128 * 128 < INT32_MAX, "a wave's int32 sums (64 channels)");
     static_assert((D == 128 || D == 64) && (G == 1 || G == D / 32), "head_dim 128 / 64, per-token or 32-channel V groups");
     constexpr int NT = 64 * NW;
     constexpr int QKS = D / 64;                     // q.k k-steps; also the query heads a lane makes digits for
     constexpr int NTL = D / 16;                     // p.v channel tiles
     constexpr int RB = D / 2;                       // bytes of a code row
-    constexpr bool kLoFree = 8 * G <= 16;           // p.v lo parts fit rows 4 G + .. of the hi parts' operand
+    constexpr bool kWide = D == 64;                 // operands and products in 31-bit fixed point (wide_scale)
     constexpr int NSLOT = FUSED ? NW + 1 : NW;      // the fused kernel's extra slot: the partial-page tail
     constexpr int TTOK = FUSED ? kTailMax : 1;
     __shared__ SplitLds<D, NREP, NSLOT> s_split;
@@ -459,8 +459,9 @@ void attn_int4_mfma_kernel(MfmaParams a) {
     auto issue = [&](PageBuf& bf, int k) { issue_page(bf, k < n_mine ? entry_of(k) & 0xFFFF : kNoPage); };
 
     // running references (wave-uniform) and accumulators.  With fp16 metadata
-    // p * V_scale <= 65504 needs no bound; bf16 metadata is divided by s_run.
-    constexpr bool kBound = std::is_same<MT, bf16>::value;
+    // p * V_scale <= 65504 needs no bound; bf16 metadata is divided by s_run, and so
+    // is any with kWide, by a power of two.
+    constexpr bool kBound = kWide || std::is_same<MT, bf16>::value;
     float m_run[NREP], s_run[G], inv_s[G];
 #pragma unroll
     for (int r = 0; r < NREP; ++r) m_run[r] = -INFINITY;
@@ -468,8 +469,16 @@ void attn_int4_mfma_kernel(MfmaParams a) {
     for (int gv = 0; gv < G; ++gv) { s_run[gv] = kBound ? 0.f : 1.f; inv_s[gv] = 1.f; }
     float m_lane = 0.f;                      // m_run[lg], or 0 while head lg has no logit yet
     v4f pacc[NTL];                           // [tile]: component r = head, lane group lg = V group
+    // kWide: [V group][tile], head lg's digit rows since the references last moved, and what came before
+    constexpr int WG = kWide ? G : 1;
+    v4i iacc[WG][NTL];
+    float facc[WG][NTL];
 #pragma unroll
-    for (int t = 0; t < NTL; ++t) pacc[t] = (v4f){0.f, 0.f, 0.f, 0.f};
+    for (int t = 0; t < NTL; ++t) {
+        pacc[t] = (v4f){0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+        for (int gv = 0; gv < WG; ++gv) { iacc[gv][t] = (v4i){0, 0, 0, 0}; facc[gv][t] = 0.f; }
+    }
     float l_acc = 0.f, bias[G];              // head lg: sum p, sum p * V_mn[g] over this lane's tokens
 #pragma unroll
     for (int gv = 0; gv < G; ++gv) bias[gv] = 0.f;
@@ -511,11 +520,31 @@ void attn_int4_mfma_kernel(MfmaParams a) {
                 amax = fmaxf(amax, fabsf(A[hh][bb]));
             }
         }
-        const float sigma = wave_max(amax);
-        const float inv = sigma > 0.f ? kQkScale * __builtin_amdgcn_rcpf(sigma) : 0.f;
+        float unscale;
+        if constexpr (kWide) {               // 16 lanes per head: the lane's own head's references
+            const WideScale ws = wide_scale(row16_max(amax));
+            unscale = ws.unscale;
+            if (r0 < NREP) {
+                uint32_t Y[4];
 #pragma unroll
-        for (int hh = 0; hh < QKS; ++hh) {
-            if (r0 + hh < NREP) {
+                for (int bb = 0; bb < 4; ++bb) {
+                    Y[bb] = wide_digits(A[0][bb], ws.scale);
+                    cpart[0] = fmaf(A[0][bb], 0.f, cpart[0]);    // an infinite or NaN A has no digits
+                }
+                const int row = 4 * r0;
+                uint32_t* dst = (uint32_t*)&W.aqk[qs_s][row][swz(row, qs_kg)][4 * qs_jd];
+                dst[0] = byte_i<3>(Y[0], Y[1], Y[2], Y[3]) ^ kDigitFlip;           // row 4r: weight 2^24
+                dst[64 / 4] = byte_i<2>(Y[0], Y[1], Y[2], Y[3]) ^ kDigitFlip;      // row 4r+1: 65536
+                dst[128 / 4] = byte_i<1>(Y[0], Y[1], Y[2], Y[3]) ^ kDigitFlip;     // row 4r+2: 256
+                dst[192 / 4] = byte_i<0>(Y[0], Y[1], Y[2], Y[3]) ^ kDigitFlip;     // row 4r+3: 1
+            }
+        } else {
+            const float sigma = wave_max(amax);
+            const float inv = sigma > 0.f ? kQkScale * __builtin_amdgcn_rcpf(sigma) : 0.f;
+            unscale = sigma * (1.0f / kQkScale);
+#pragma unroll
+            for (int hh = 0; hh < QKS; ++hh) {
+                if (r0 + hh >= NREP) continue;
                 // Y = round(A * inv) + 0x808080, rounded by the fp32 add itself
                 uint32_t Y[4];
 #pragma unroll
@@ -526,6 +555,9 @@ void attn_int4_mfma_kernel(MfmaParams a) {
                 dst[64 / 4] = byte_i<1>(Y[0], Y[1], Y[2], Y[3]) ^ kDigitFlip;      // row 4r+1: 256
                 dst[128 / 4] = byte_i<0>(Y[0], Y[1], Y[2], Y[3]) ^ kDigitFlip;     // row 4r+2: 1
             }
+        }
+#pragma unroll
+        for (int hh = 0; hh < QKS; ++hh) {
             float cs = cpart[hh];            // sum over the 32 (D = 64: 16) lanes of head r0 + hh
             if constexpr (D == 128) cs += __shfl_xor(cs, 16, 64);
             cpart[hh] = row_sum<16>(cs);
@@ -536,7 +568,6 @@ void attn_int4_mfma_kernel(MfmaParams a) {
             const float c1 = __shfl(cpart[1], (lg >> 1) * 32, 64);
             Cr = (lg & 1) ? c1 : c0;
         }
-        const float unscale = sigma * (1.0f / kQkScale);
         wave_lds_fence();
         const v4i a0 = *(const v4i*)&W.aqk[0][n16][swz(n16, lg)][0];
         const v4i a1 = *(const v4i*)&W.aqk[QKS - 1][n16][swz(n16, lg)][0];
@@ -549,7 +580,8 @@ void attn_int4_mfma_kernel(MfmaParams a) {
             v4i acc = {0, 0, 0, 0};
             acc = __builtin_amdgcn_mfma_i32_16x16x64_i8(a0, b0, acc, 0, 0, 0);
             if constexpr (D == 128) acc = __builtin_amdgcn_mfma_i32_16x16x64_i8(a1, b1, acc, 0, 0, 0);
-            const float f = fmaf((float)acc[0], 65536.f, fmaf((float)acc[1], 256.f, (float)acc[2]));
+            const float f = kWide ? digit_rows(acc)
+                                  : fmaf((float)acc[0], 65536.f, fmaf((float)acc[1], 256.f, (float)acc[2]));
             const float lgt = fmaf(f, unscale, Cr);
             const bool ok = lg < NREP && ((qm >> lg) & 1) && tok0 + 16 * T + n16 < S;
             lg4[T] = ok ? lgt : -INFINITY;
@@ -578,7 +610,7 @@ void attn_int4_mfma_kernel(MfmaParams a) {
                 float v = vs_t[T][0];
 #pragma unroll
                 for (int gv = 1; gv < G; ++gv) v = lg == gv ? vs_t[T][gv] : v;
-                sp = fmaxf(sp, v);
+                sp = fmaxf(sp, kWide ? fabsf(v) : v);
             }
             sp = row16_max(sp);
 #pragma unroll
@@ -600,16 +632,18 @@ void attn_int4_mfma_kernel(MfmaParams a) {
                 as[gv] = 1.0f;
                 if constexpr (kBound) {
                     // A = p * V_scale / s_run <= 1/2: bound set with a factor-2 headroom
-                    const float sn = sp_g[gv] > s_run[gv] ? 2.0f * sp_g[gv] : s_run[gv];
+                    // (kWide: the next power of two, so that neither division rounds)
+                    const float up = kWide ? wide_bound(sp_g[gv]) : 2.0f * sp_g[gv];
+                    const float sn = sp_g[gv] > s_run[gv] ? up : s_run[gv];
                     as[gv] = sn > 0.f ? s_run[gv] / sn : 1.0f;
                     s_run[gv] = sn;
-                    inv_s[gv] = sn > 0.f ? 1.0f / sn : 0.f;
+                    inv_s[gv] = sn > 0.f ? (kWide ? kWideOne : 1.0f) / sn : 0.f;
                 }
             }
             float a_lg = as[0], am_lg = am[0];
             float ml = m_run[0];
 #pragma unroll
-            for (int gv = 1; gv < G; ++gv) a_lg = (lg & (G - 1)) == gv ? as[gv] : a_lg;   // lo rows: lane groups G + g
+            for (int gv = 1; gv < G; ++gv) a_lg = lg == gv ? as[gv] : a_lg;
 #pragma unroll
             for (int r = 1; r < NREP; ++r) {
                 am_lg = lg == r ? am[r] : am_lg;
@@ -619,11 +653,23 @@ void attn_int4_mfma_kernel(MfmaParams a) {
             l_acc *= am_lg;
 #pragma unroll
             for (int gv = 0; gv < G; ++gv) bias[gv] *= am_lg;
+            if constexpr (kWide) {
 #pragma unroll
-            for (int r = 0; r < 4; ++r) {
-                const float f = r < NREP ? am[r] * a_lg : 0.f;
+                for (int gv = 0; gv < G; ++gv) {
+                    const float f = am_lg * as[gv];
 #pragma unroll
-                for (int t = 0; t < NTL; ++t) pacc[t][r] *= f;
+                    for (int t = 0; t < NTL; ++t) {
+                        facc[gv][t] = (facc[gv][t] + digit_rows(iacc[gv][t])) * f;
+                        iacc[gv][t] = (v4i){0, 0, 0, 0};
+                    }
+                }
+            } else {
+#pragma unroll
+                for (int r = 0; r < 4; ++r) {
+                    const float f = r < NREP ? am[r] * a_lg : 0.f;
+#pragma unroll
+                    for (int t = 0; t < NTL; ++t) pacc[t][r] *= f;
+                }
             }
         }
 
@@ -633,6 +679,59 @@ void attn_int4_mfma_kernel(MfmaParams a) {
         for (int T = 0; T < 4; ++T) {
             pr[T] = exp2_fast(lg4[T] - m_lane);      // exp2(-inf) = 0 for masked tokens
             l_acc += pr[T];
+        }
+        if constexpr (kWide) {
+            // A: the digits of p * V_scale / s_run in rows 4 head + digit; operand k =
+            // 16 kg + 4 jd + byte is token 16 byte + 4 jd + kg, so the lane's four tokens
+            // are one dword per digit
+#pragma unroll
+            for (int gv = 0; gv < G; ++gv) {
+                uint32_t Y[4];
+#pragma unroll
+                for (int T = 0; T < 4; ++T) {
+                    const float x = pr[T] * vs_t[T][gv];
+                    // the operand below is code - 8: less for the two sums to cancel
+                    bias[gv] = fmaf(pr[T], fmaf(vs_t[T][gv], 8.f, vm_t[T][gv]), bias[gv]);
+                    bias[gv] = fmaf(x, 0.f, bias[gv]);       // an infinite or NaN product has no digits
+                    Y[T] = wide_digits(x, inv_s[gv]);
+                }
+                if (lg < NREP) {
+                    uint32_t* dst = (uint32_t*)&W.apv[gv][4 * lg][(n16 & 3) ^ lg][4 * (n16 >> 2)];
+                    dst[0] = byte_i<3>(Y[0], Y[1], Y[2], Y[3]) ^ kDigitFlip;
+                    dst[64 / 4] = byte_i<2>(Y[0], Y[1], Y[2], Y[3]) ^ kDigitFlip;
+                    dst[128 / 4] = byte_i<1>(Y[0], Y[1], Y[2], Y[3]) ^ kDigitFlip;
+                    dst[192 / 4] = byte_i<0>(Y[0], Y[1], Y[2], Y[3]) ^ kDigitFlip;
+                }
+            }
+            wave_lds_fence();
+            v4i ad[G];
+#pragma unroll
+            for (int gv = 0; gv < G; ++gv) ad[gv] = *(const v4i*)&W.apv[gv][n16][swz(n16, lg)][0];
+            // B: dword jd = 16 (code - 8) of one channel of tokens 16 byte + 4 jd + lg
+            uint32_t nl[8], nh[8];           // two tokens' 4 codes in two registers
+#pragma unroll
+            for (int j = 0; j < 8; ++j) {
+                const uint32_t v2 = cb.vw[2 * j] | (cb.vw[2 * j + 1] << 16);
+                nl[j] = ((v2 << 4) & 0xF0F0F0F0u) ^ kDigitFlip;
+                nh[j] = (v2 & 0xF0F0F0F0u) ^ kDigitFlip;
+            }
+#pragma unroll
+            for (int cc = 0; cc < NTL / 2; ++cc) {
+                const uint32_t sel = 0x06040200u + 0x01010101u * cc;
+                v4i bl, bh;
+#pragma unroll
+                for (int jd = 0; jd < 4; ++jd) {
+                    bl[jd] = (int)__builtin_amdgcn_perm(nl[2 * jd + 1], nl[2 * jd], sel);
+                    bh[jd] = (int)__builtin_amdgcn_perm(nh[2 * jd + 1], nh[2 * jd], sel);
+                }
+#pragma unroll
+                for (int gv = 0; gv < G; ++gv) {     // every group's products; a column keeps its own group's
+                    iacc[gv][2 * cc] = __builtin_amdgcn_mfma_i32_16x16x64_i8(ad[gv], bl, iacc[gv][2 * cc], 0, 0, 0);
+                    iacc[gv][2 * cc + 1] = __builtin_amdgcn_mfma_i32_16x16x64_i8(ad[gv], bh, iacc[gv][2 * cc + 1], 0, 0, 0);
+                }
+            }
+            wave_lds_fence();
+            return;
         }
         // Operand k = 8*kg + 2*ai + jj of step s carries token 16*(2s + jj) + 4*ai + kg
         // (the order of the V dwords below): token 16T + n16 is step T>>1, kg = n16&3,
@@ -655,8 +754,8 @@ void attn_int4_mfma_kernel(MfmaParams a) {
                     const h2v hv = __builtin_convertvector(av, h2v);
                     const h2v lv = __builtin_convertvector(av - __builtin_convertvector(hv, f2v), h2v);
                     *(uint32_t*)&W.apv[st][row][q][4 * (n16 >> 2)] = __builtin_bit_cast(uint32_t, hv);
-                    if constexpr (kLoFree)       // rows 4 G .. are free: lo in row 4 G + row, same operand
-                        *(uint32_t*)&W.apv[st][row + 4 * G][swz(row + 4 * G, n16 & 3)][4 * (n16 >> 2)] =
+                    if constexpr (G == 1)        // rows 4..7 are free: lo in row 4 + r, same operand
+                        *(uint32_t*)&W.apv[st][row + 4][swz(row + 4, n16 & 3)][4 * (n16 >> 2)] =
                             __builtin_bit_cast(uint32_t, lv);
                     else
                         *(uint32_t*)&W.apl[st][row][q][4 * (n16 >> 2)] = __builtin_bit_cast(uint32_t, lv);
@@ -666,8 +765,8 @@ void attn_int4_mfma_kernel(MfmaParams a) {
         wave_lds_fence();
         const v8h ap0 = *(const v8h*)&W.apv[0][n16][swz(n16, lg)][0];
         const v8h ap1 = *(const v8h*)&W.apv[1][n16][swz(n16, lg)][0];
-        v8h al0 = {}, al1 = {};          // used with every row taken (G = 4) only
-        if constexpr (!kLoFree) {
+        v8h al0 = {}, al1 = {};          // used with G != 1 only
+        if constexpr (G != 1) {
             al0 = *(const v8h*)&W.apl[0][n16][swz(n16, lg)][0];
             al1 = *(const v8h*)&W.apl[1][n16][swz(n16, lg)][0];
         }
@@ -696,7 +795,7 @@ void attn_int4_mfma_kernel(MfmaParams a) {
                 const v8h a = st ? ap1 : ap0, al = st ? al1 : al0;
                 pacc[2 * cc] = __builtin_amdgcn_mfma_f32_16x16x32_f16(a, blo, pacc[2 * cc], 0, 0, 0);
                 pacc[2 * cc + 1] = __builtin_amdgcn_mfma_f32_16x16x32_f16(a, bhi, pacc[2 * cc + 1], 0, 0, 0);
-                if constexpr (!kLoFree) {
+                if constexpr (G != 1) {
                     pacc[2 * cc] = __builtin_amdgcn_mfma_f32_16x16x32_f16(al, blo, pacc[2 * cc], 0, 0, 0);
                     pacc[2 * cc + 1] = __builtin_amdgcn_mfma_f32_16x16x32_f16(al, bhi, pacc[2 * cc + 1], 0, 0, 0);
                 }
@@ -729,11 +828,11 @@ void attn_int4_mfma_kernel(MfmaParams a) {
     }
 
     // ------------------------------------------------ wave state -> LDS
-    if constexpr (kLoFree) {    // the lo rows 4 G + .. (lane groups G + g) join the hi rows
+    if constexpr (G == 1 && !kWide) {     // the lo rows 4 + r (lane group 1) join the hi rows
 #pragma unroll
         for (int t = 0; t < NTL; ++t)
 #pragma unroll
-            for (int r = 0; r < NREP; ++r) pacc[t][r] += __shfl_xor(pacc[t][r], 16 * G, 64);
+            for (int r = 0; r < NREP; ++r) pacc[t][r] += __shfl_xor(pacc[t][r], 16, 64);
     }
     l_acc = row_sum<16>(l_acc);
 #pragma unroll
@@ -744,7 +843,25 @@ void attn_int4_mfma_kernel(MfmaParams a) {
     for (int gv = 1; gv < G; ++gv) {
         if (ug == gv) { bsel = bias[gv]; ssel = s_run[gv]; }
     }
-    const float pv_unscale = ssel * kSubnormal;
+    const float pv_unscale = ssel * (kWide ? 0.0625f / kWideOne : kSubnormal);
+    if constexpr (kWide) {      // head lg's outputs of the lane's channels, from their own group's sums
+        if (lg < NREP) {
+#pragma unroll
+            for (int t = 0; t < NTL; ++t) {
+                float v = facc[0][t] + digit_rows(iacc[0][t]);
+#pragma unroll
+                for (int gv = 1; gv < G; ++gv) v = ug == gv ? facc[gv][t] + digit_rows(iacc[gv][t]) : v;
+                s_split.acc[w][lg][NTL * n16 + t] = fmaf(v, pv_unscale, bsel);
+            }
+            if (n16 == 0) {
+                float m = m_run[0];
+#pragma unroll
+                for (int r = 1; r < NREP; ++r) m = lg == r ? m_run[r] : m;
+                s_split.m[w][lg] = m;
+                s_split.l[w][lg] = l_acc;
+            }
+        }
+    } else
 #pragma unroll
     for (int r = 0; r < NREP; ++r) {
         const int src = 16 * r + n16;

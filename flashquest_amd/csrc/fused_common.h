@@ -39,6 +39,42 @@ FQ_DEV int split_begin(int total, int split, int splits, int lead) {
 FQ_DEV float lane_value(float v, int lane) { return __int_as_float(__builtin_amdgcn_readlane(__float_as_int(v), lane)); }
 
 
+// The value of a head's four digit rows: weights 2^24, 2^16, 2^8, 1.
+template <typename V4>
+FQ_DEV float digit_rows(const V4& a) {
+    return fmaf((float)a[0], 16777216.f, fmaf((float)a[1], 65536.f, fmaf((float)a[2], 256.f, (float)a[3])));
+}
+
+// 64-channel heads (attn_mfma.hip, attn_int8_mfma.hip) contract both products in
+// 31-bit fixed point, four balanced int8 digits a value, int32 sums exact:
+//   q.k : q * K_scale, relative to the largest of its own head and page
+//   p.v : p * V_scale, relative to s_run, the power of two at or above every
+//         |V_scale| the wave has met (p <= 1); the sums move to fp32 and are rescaled
+//         when a reference moves.
+// The scales are powers of two, so a value is exact down to 2^-7 of the largest and
+// good to 2^-31 of it below: no less than the fp32 operands of the VALU kernel these
+// heads ran on (attn_int4.hip).  Error against 64 bits relative to |O|, float32
+// queries over 8192 tokens, V of any size and spread: 3e-7 to 1.3e-6 (that kernel:
+// 4e-7 to 1.4e-6).  The 128-channel form, 24 bits per page and fp16 hi + lo pairs
+// against codes as fp16 subnormals, gives 1e-4 to 5e-4 here with INT4 codes (the
+// matrix unit aligns the subnormals' products by their exponent), 5e-6 to 9e-2 with
+// INT8.  Its time is the same but for V in 32-channel groups, whose products run
+// once per group (16 sequences x 16393 tokens, 32 / 8 heads: 36.1 us for 36.6
+// without groups, 39.8 for 36.8 with them).
+constexpr float kWideOne = 1073741824.0f;       // 2^30
+struct WideScale { float scale, unscale; };
+// amax * scale in [2^29, 2^30); an amax below 2^-97 is taken for 2^-97.
+FQ_DEV WideScale wide_scale(float amax) {
+    const uint32_t e = min(max(__float_as_uint(amax) >> 23, 30u), 254u);
+    return {__uint_as_float((283u - e) << 23), __uint_as_float((e - 29u) << 23)};
+}
+// The digits of a * scale, |a * scale| <= 2^30, as bytes + 128 (the highest is byte 3).
+FQ_DEV uint32_t wide_digits(float a, float scale) { return (uint32_t)(int)rintf(a * scale) + 0x80808080u; }
+// The power of two at or above s >= 0, at least 2^-96 (kWideOne over it is finite).
+FQ_DEV float wide_bound(float s) {
+    return fmaxf(__uint_as_float((__float_as_uint(s) + 0x7FFFFFu) & 0xFF800000u), 1.2621774e-29f);
+}
+
 FQ_DEV __amdgpu_buffer_rsrc_t make_rsrc(const void* base, int64_t bytes) {
     const int n = bytes > 0x7FFFFFFF ? 0x7FFFFFFF : (int)bytes;
     return __builtin_amdgcn_make_buffer_rsrc(const_cast<void*>(base), (short)0, n, 0x00020000);

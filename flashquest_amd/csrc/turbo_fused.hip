@@ -125,11 +125,6 @@ FQ_DEV uint2 read_tr16(const void* lds) {
     return __builtin_bit_cast(uint2, r);
 }
 
-// The value of a head's four digit rows: weights 2^24, 2^16, 2^8, 1.
-FQ_DEV float digit_rows(const v4i& a) {
-    return fmaf((float)a[0], 16777216.f, fmaf((float)a[1], 65536.f, fmaf((float)a[2], 256.f, (float)a[3])));
-}
-
 // Sparse decode attention over the TurboQuant cache on the matrix cores
 // (v_mfma_i32_16x16x64_i8): both products contract 24-bit fixed-point values X
 // (three balanced int8 digits a2 a1 a0) with the codebook's two digits H L, all

@@ -97,3 +97,74 @@ def test_layers_strides_and_masks(bits):
         om, lm = op(Q[l], *[views[i][l] for i in (0, 1, 2, 3, 4, 5)], selection_mask=mask[l].unsqueeze(2))
         assert max_err(om[:, :, 0], ref["O"]) <= decode_tol(ref["O"], "bf16")
         assert max_err(lm[:, :, 0], ref["lse"]) <= 1e-4
+
+
+def _dequant64(host, bits, page=64):
+    """The cache's keys and values in 64 bits."""
+    kc, ks, km, vc, vs, vm = host
+    if bits == 4:
+        kc, vc = O.unpack_int4(kc), O.unpack_int4(vc)
+    at = np.arange(kc.shape[2]) // page
+    G = vs.shape[-1]
+    wide = lambda x: np.repeat(x.astype(np.float64), vc.shape[-1] // G, axis=-1)
+    return kc * ks.astype(np.float64)[:, :, at] + km.astype(np.float64)[:, :, at], vc * wide(vs) + wide(vm)
+
+
+@pytest.mark.parametrize("bits,meta,vgroup", [(4, "f16", None), (4, "f16", 32), (4, "bf16", None), (4, "bf16", 32),
+                                              (8, "bf16", None), (8, "f16", None)])
+@pytest.mark.parametrize("form", ["plain", "v_1e-2", "v_1e-3", "v_four_decades", "v_one_large_row", "q_two_decades"])
+def test_operands_as_close_as_fp32(bits, meta, vgroup, form):
+    """float32 queries against 64 bits, the error relative to |O| of each head, every page selected.
+
+    The logits (log2 domain) stay below 32, where half an fp32 ulp is 2^-20: the
+    rounded query, the sum of the products, the one with the page minimum and the
+    difference to the maximum are four such roundings, each at most 2^-20 ln 2 of
+    its token's weight.  They differ from token to token; a head whose weight lies
+    on a single token keeps none of it (the normaliser has the same factor).  The
+    sums of p v and of p then add 8 roundings of 2^-24.  Operands of 22 bits,
+    p * V_scale held against a fixed or distant bound, or products summed with
+    16-bit alignment are 6e-6 to 9e-2 here.
+    """
+    bound = 4 * 2.0 ** -20 * np.log(2) + 8 * 2.0 ** -24
+    rng = np.random.default_rng(len(form) + bits)
+    B, Hkv, nrep, S, D = 1, 2, 4, 64 * 40 + 21, 64
+    K = 2 * rng.standard_normal((B, Hkv, S, D)).astype(np.float32)
+    V = rng.standard_normal((B, Hkv, S, D)).astype(np.float32)
+    Q = rng.standard_normal((B, Hkv * nrep, D)).astype(np.float32)
+    if form.startswith("v_1e"):
+        V *= np.float32(form[2:])
+    elif form == "v_four_decades":
+        V *= (10.0 ** -rng.uniform(0, 4, (B, Hkv, S, 1))).astype(np.float32)
+    elif form == "v_one_large_row":
+        V[:, :, S // 3] *= 300
+    elif form == "q_two_decades":
+        Q *= (10.0 ** -rng.uniform(0, 2, (B, Hkv * nrep, 1))).astype(np.float32)
+    dt = torch.float16 if meta == "f16" else torch.bfloat16
+    up = lambda a: torch.from_numpy(a).to("cuda:0")
+    if bits == 4:
+        host = (*O.quantize_k_int4(K, 64, "f32", meta), *O.quantize_v_int4(V, vgroup, meta))
+    else:
+        host = (*O.quantize_k_int8(K, 64, "f32", meta), *O.quantize_v_int8(V, meta))
+    planes = [up(a) if i in (0, 3) else to_dev_half(a, meta) for i, a in enumerate(host)]
+    K64, V64 = (np.repeat(x, nrep, axis=1) for x in _dequant64(host, bits))
+    z = np.einsum("bhd,bhsd->bhs", Q.astype(np.float64), K64) / 8.0
+    assert np.abs(z).max() * np.log2(np.e) < 32
+    p = np.exp(z - z.max(-1, keepdims=True))
+    want = np.einsum("bhs,bhsd->bhd", p, V64) / p.sum(-1)[..., None]
+    lse64 = z.max(-1) + np.log(p.sum(-1))
+
+    def close(o, lse):
+        got = o[:, :, 0].double().cpu().numpy()
+        err = np.linalg.norm(got - want, axis=-1) / np.linalg.norm(want, axis=-1)
+        assert err.max() <= bound, (form, err.max())
+        # the logits' four roundings, and lse's own (below 32)
+        assert np.abs(lse[:, :, 0].double().cpu().numpy() - lse64).max() <= 4 * 2.0 ** -20 * np.log(2) + 2.0 ** -20
+
+    q = up(Q)[:, :, None]
+    o, lse = _decode(bits)(q, *planes, retention=1.0)
+    assert o.dtype == torch.float32
+    close(o, lse)
+    from flashquest_amd.kernel import flash_attn_sparse_fwd, flash_attn_sparse_int4_fwd
+    every = torch.ones(B, Hkv * nrep, 1, planes[1].shape[2], dtype=torch.bool, device="cuda:0")
+    op = flash_attn_sparse_fwd if bits == 8 else flash_attn_sparse_int4_fwd
+    close(*op(q, *planes, selection_mask=every))
