@@ -23,6 +23,7 @@
 #include <ATen/ops/empty.h>
 #include <torch/csrc/Exceptions.h>
 #include <torch/csrc/autograd/python_variable.h>
+#include <torch/csrc/utils/object_ptr.h>
 
 #include "fq_hip.h"
 
@@ -162,12 +163,14 @@ int tail_of(PyObject* k_obj, PyObject* v_obj, int nd, int64_t D, int64_t k_align
 
 PyObject* none() { Py_RETURN_NONE; }
 
-// decode(bits, Q, planes (6, or 8 with TurboQuant's raw metadata), retention, retention layer stride, sinks,
-//        window, k_max or -1, mode, page, sm_scale or None, return_lse, K_tail, V_tail, workspace, stream)
+// decode(bits, Q, planes (6, or 8 with TurboQuant's raw metadata), retention rows, sinks, window, k_max or -1,
+//        mode, page, sm_scale or None, return_lse, K_tail, V_tail, workspace, stream)
 //   -> (O, lse or None), or None
+// retention rows: a function of no arguments that gives (rows, layer stride), called once everything else is known
+// to be the plain case (it may copy to the device and launch), its errors raised.
 PyObject* decode(PyObject*, PyObject* const* a, Py_ssize_t n) {
     HANDLE_TH_ERRORS
-    if (n != 16) return none();
+    if (n != 15) return none();
     const int bits = (int)PyLong_AsLong(a[0]);
     const at::Tensor* Q = plain(a[1]);
     const Py_ssize_t np = PyTuple_Check(a[2]) ? PyTuple_GET_SIZE(a[2]) : 0;
@@ -179,14 +182,13 @@ PyObject* decode(PyObject*, PyObject* const* a, Py_ssize_t n) {
         if (!x || x->device() != Q->device()) return none();
         (i < 6 ? t[i] : raw[i - 6]) = x;
     }
-    const at::Tensor* ret = plain(a[3]);
-    const at::Tensor* ws = a[14] == Py_None ? nullptr : plain(a[14]);
+    const at::Tensor* ws = a[13] == Py_None ? nullptr : plain(a[13]);
     const int nd = (int)Q->dim();
-    if (!ret || !ws || nd != t[0]->dim() || Q->size(-2) != 1) return none();
-    const int sinks = (int)PyLong_AsLong(a[5]), window = (int)PyLong_AsLong(a[6]);
-    int k_max = (int)PyLong_AsLong(a[7]);
-    const int mode = (int)PyLong_AsLong(a[8]), page = (int)PyLong_AsLong(a[9]);
-    const bool want_lse = a[11] == Py_True;
+    if (!ws || nd != t[0]->dim() || Q->size(-2) != 1) return none();
+    const int sinks = (int)PyLong_AsLong(a[4]), window = (int)PyLong_AsLong(a[5]);
+    int k_max = (int)PyLong_AsLong(a[6]);
+    const int mode = (int)PyLong_AsLong(a[7]), page = (int)PyLong_AsLong(a[8]);
+    const bool want_lse = a[10] == Py_True;
 
     fq_int4_cache c{};
     fq_turbo_cache tc{};
@@ -209,10 +211,9 @@ PyObject* decode(PyObject*, PyObject* const* a, Py_ssize_t n) {
     q.q_strides[3] = 1;
     for (int i = 0; i < 4; ++i) q.o_strides[i] = q.q_strides[i];
     q.H_q = Hq;
-    q.sm_scale = a[10] == Py_None ? (float)(1.0 / std::sqrt((double)D)) : (float)PyFloat_AsDouble(a[10]);
-    q.retention_layer_stride = PyLong_AsLongLong(a[4]);
+    q.sm_scale = a[9] == Py_None ? (float)(1.0 / std::sqrt((double)D)) : (float)PyFloat_AsDouble(a[9]);
     fq_tail tail{};
-    const int has_tail = bits == 3 ? (a[12] == Py_None ? 0 : -1) : tail_of(a[12], a[13], nd, D, 1, 1, false, tail);
+    const int has_tail = bits == 3 ? (a[11] == Py_None ? 0 : -1) : tail_of(a[11], a[12], nd, D, 1, 1, false, tail);
     if (PyErr_Occurred() || has_tail < 0) {
         PyErr_Clear();
         return none();
@@ -228,6 +229,12 @@ PyObject* decode(PyObject*, PyObject* const* a, Py_ssize_t n) {
     }
     const size_t need = bits == 3 ? g_fq.ws_turbo(&tc, Hq) : g_fq.ws_int4(&c, Hq);
     if (need > (size_t)ws->numel()) return none();
+    const THPObjectPtr made(PyObject_CallNoArgs(a[3]));
+    if (!made) return nullptr;
+    const at::Tensor* ret =
+        PyTuple_Check(made.get()) && PyTuple_GET_SIZE(made.get()) == 2 ? plain(PyTuple_GET_ITEM(made.get(), 0)) : nullptr;
+    if (!ret) return none();
+    q.retention_layer_stride = PyLong_AsLongLong(PyTuple_GET_ITEM(made.get(), 1));
 
     at::Tensor O = at::empty(Q->sizes(), Q->options()), lse;
     q.out = O.data_ptr();
@@ -241,7 +248,7 @@ PyObject* decode(PyObject*, PyObject* const* a, Py_ssize_t n) {
     const float* r = (const float*)ret->data_ptr();
     void* w = ws->data_ptr();
     const size_t wn = (size_t)ws->numel();
-    fq_stream_t st = (fq_stream_t)PyLong_AsVoidPtr(a[15]);
+    fq_stream_t st = (fq_stream_t)PyLong_AsVoidPtr(a[14]);
     int64_t s0[5], s1[5];
     if (bits == 3) {
         strides(*raw[0], s0);

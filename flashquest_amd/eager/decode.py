@@ -54,16 +54,24 @@ def merge_two_attentions(O_a, lse_a, O_b, lse_b) -> torch.Tensor:
 
 def _native_decode(bits, Q, planes, H_kv, retention, head_pattern, num_sinks, window_pages, k_max_static, select_mode,
                    page_size, sm_scale, return_lse, K_tail, V_tail):
-    """The step through the native host path: (O, lse), or None for the general way."""
+    """The step through the native host path: ((O, lse), or None for the general
+    way; the retention rows if the path got as far as asking for them, which the
+    general way then takes over)."""
     host = _host.module()
     H_q = Q.shape[-3]
     if host is None or H_kv < 1 or H_q % H_kv:
-        return None
-    r, r_stride = _ops.retention_rows(retention, head_pattern, H_q, H_kv, Q.shape[0] if Q.dim() == 5 else 1, Q.device)
+        return None, None
+    rows = []
+
+    def retention_rows():
+        rows.append(_ops.retention_rows(retention, head_pattern, H_q, H_kv, Q.shape[0] if Q.dim() == 5 else 1,
+                                        Q.device))
+        return rows[0]
     stream = L.stream_handle(Q.device)
-    return host.decode(bits, Q, planes, r, r_stride, int(num_sinks), int(window_pages),
-                       -1 if k_max_static is None else int(k_max_static), L.SELECT_MODES[select_mode], int(page_size),
-                       sm_scale, bool(return_lse), K_tail, V_tail, L.workspace_if_any(Q.device, stream), stream)
+    res = host.decode(bits, Q, planes, retention_rows, int(num_sinks), int(window_pages),
+                      -1 if k_max_static is None else int(k_max_static), L.SELECT_MODES[select_mode], int(page_size),
+                      sm_scale, bool(return_lse), K_tail, V_tail, L.workspace_if_any(Q.device, stream), stream)
+    return res, rows[0] if rows else None
 
 
 _FUSED_TAIL_REFUSED = "the fused tail needs the matrix-core attention layout"
@@ -167,10 +175,11 @@ def quest_decode_int4(
     if D not in (64, 128):
         raise NotImplementedError(f"head_dim={D} not in (64, 128)")
     H_kv = K_scale.shape[-3]
+    rows = None
     if out is None and _rotation is None and not return_selection and not _direct:
-        res = _native_decode(4, Q, (K_packed, K_scale, K_mn, V_packed, V_scale, V_mn), H_kv, retention, head_pattern,
-                             num_sinks, window_pages, k_max_static, select_mode, page_size, sm_scale, return_lse,
-                             K_tail, V_tail)
+        res, rows = _native_decode(4, Q, (K_packed, K_scale, K_mn, V_packed, V_scale, V_mn), H_kv, retention,
+                                   head_pattern, num_sinks, window_pages, k_max_static, select_mode, page_size,
+                                   sm_scale, return_lse, K_tail, V_tail)
         if res is not None:
             return res
     nrep = Q.shape[-3] // H_kv if Q.shape[-3] % H_kv == 0 else 0
@@ -193,8 +202,10 @@ def quest_decode_int4(
     if H_q % cache.H_kv:
         raise ValueError(f"H_q={H_q} must be divisible by H_kv={cache.H_kv}")
     query = _ops.query(Q3, O3, lse, sm_scale)
-    r, query.retention_layer_stride = _ops.retention_rows(retention, head_pattern, H_q, cache.H_kv,
-                                                          Q3.shape[0] if Q3.dim() == 4 else 1, Q.device)
+    if rows is None:
+        rows = _ops.retention_rows(retention, head_pattern, H_q, cache.H_kv, Q3.shape[0] if Q3.dim() == 4 else 1,
+                                   Q.device)
+    r, query.retention_layer_stride = rows
     query.rotation_signs = None if _rotation is None else _rotation.data_ptr()
     k_max = -1 if k_max_static is None else min(int(k_max_static), P)
     mask = None
@@ -523,10 +534,11 @@ def quest_decode_int8(
     if D not in (64, 128):
         raise NotImplementedError(f"head_dim={D} not in (64, 128)")
     H_kv = K_scale.shape[-3]
+    rows = None
     if not return_selection and not _direct:
-        res = _native_decode(8, Q, (K_uint8, K_scale, K_mn, V_uint8, V_scale, V_mn), H_kv, retention, head_pattern,
-                             num_sinks, window_pages, k_max_static, select_mode, page_size, sm_scale, return_lse,
-                             K_tail, V_tail)
+        res, rows = _native_decode(8, Q, (K_uint8, K_scale, K_mn, V_uint8, V_scale, V_mn), H_kv, retention,
+                                   head_pattern, num_sinks, window_pages, k_max_static, select_mode, page_size,
+                                   sm_scale, return_lse, K_tail, V_tail)
         if res is not None:
             return res
     nrep = Q.shape[-3] // H_kv if Q.shape[-3] % H_kv == 0 else 0
@@ -548,8 +560,10 @@ def quest_decode_int8(
     if H_q % cache.H_kv:
         raise ValueError(f"H_q={H_q} must be divisible by H_kv={cache.H_kv}")
     query = _ops.query(Q3, O3, lse, sm_scale)
-    r, query.retention_layer_stride = _ops.retention_rows(retention, head_pattern, H_q, cache.H_kv,
-                                                          Q3.shape[0] if Q3.dim() == 4 else 1, Q.device)
+    if rows is None:
+        rows = _ops.retention_rows(retention, head_pattern, H_q, cache.H_kv, Q3.shape[0] if Q3.dim() == 4 else 1,
+                                   Q.device)
+    r, query.retention_layer_stride = rows
     k_max = -1 if k_max_static is None else min(int(k_max_static), P)
     mask = torch.empty(Q3.shape[:-1] + (P,), dtype=torch.bool, device=Q.device) if return_selection else None
     stream = L.stream_handle(Q.device)
@@ -628,10 +642,11 @@ def quest_decode_turbo(
     if K_scale_raw.dtype != torch.bfloat16 or K_mn_raw.dtype != torch.bfloat16:
         raise AssertionError("K_scale_raw / K_mn_raw must be bf16")
     H_kv = K_msb.shape[-3]
+    rows = None
     if not return_selection and not _direct:
-        res = _native_decode(3, Q, (K_msb, K_lsb, K_scale_turbo, V_msb, V_lsb, V_scale_turbo, K_scale_raw, K_mn_raw),
-                             H_kv, retention, head_pattern, num_sinks, window_pages, k_max_static, select_mode,
-                             page_size, sm_scale, return_lse, None, None)
+        res, rows = _native_decode(3, Q, (K_msb, K_lsb, K_scale_turbo, V_msb, V_lsb, V_scale_turbo, K_scale_raw,
+                                          K_mn_raw), H_kv, retention, head_pattern, num_sinks, window_pages, k_max_static,
+                                   select_mode, page_size, sm_scale, return_lse, None, None)
         if res is not None:
             return res
     nrep = Q.shape[-3] // H_kv if Q.shape[-3] % H_kv == 0 else 0
@@ -657,8 +672,10 @@ def quest_decode_turbo(
     ksr = K_scale_raw if K_scale_raw.stride(-1) == 1 else K_scale_raw.contiguous()
     kmr = K_mn_raw if K_mn_raw.stride(-1) == 1 else K_mn_raw.contiguous()
     query = _ops.query(Q3, O3, lse, sm_scale)
-    r, query.retention_layer_stride = _ops.retention_rows(retention, head_pattern, H_q, cache.H_kv,
-                                                          Q3.shape[0] if Q3.dim() == 4 else 1, Q.device)
+    if rows is None:
+        rows = _ops.retention_rows(retention, head_pattern, H_q, cache.H_kv, Q3.shape[0] if Q3.dim() == 4 else 1,
+                                   Q.device)
+    r, query.retention_layer_stride = rows
     k_max = -1 if k_max_static is None else min(int(k_max_static), P)
     mask = None
     if return_selection:

@@ -95,3 +95,33 @@ def test_errors_are_the_general_paths():
         quest_decode_int4(q, *planes[:2], planes[2].half(), *planes[3:], retention=0.3)
     with pytest.raises(ValueError):
         quantize_k_int4(torch.zeros(1, 1, 64, 63, device="cuda").bfloat16(), 64)
+
+
+@pytest.mark.parametrize("bits", [4, 8])
+@pytest.mark.parametrize("form,made", [("plain", 1), ("first_call", 1), ("q_strided", 1), ("q_subclass", 1), ("five_heads", 1),
+                                       ("six_heads_chunked", 2), ("f32_tail_d64", 1)])
+def test_retention_is_prepared_once(monkeypatch, bits, form, made):
+    """A call that the native path leaves to the general one has its retention rows
+    (copies and launches, with a head pattern) made once; chunked heads once a chunk."""
+    from flashquest_amd import _lib, _ops
+    from flashquest_amd.eager.decode import quest_decode_int4, quest_decode_int8
+    heads = {"five_heads": 10, "six_heads_chunked": 12}.get(form, 6)
+    D = 64 if form == "f32_tail_d64" else 128
+    c = (Int4Case if bits == 4 else Int8Case)(seed=6, B=1, Hq=heads, Hkv=2, S=64 * (520 if form == "six_heads_chunked" else 45),
+                                              D=D)
+    q, planes = c.q_dev(), list(c.device().values())
+    op = quest_decode_int4 if bits == 4 else quest_decode_int8
+    kw = dict(retention=torch.full((heads,), 0.3), head_pattern=torch.tensor([True, False]))
+    op(q, *planes, **kw)                     # the workspace is there
+    if form == "first_call":
+        monkeypatch.setattr(_lib, "_ws", {})
+    elif form == "q_strided":
+        q = torch.stack([q, q], dim=-1)[..., 0]
+    elif form == "q_subclass":
+        q = q.as_subclass(Sub)
+    elif form == "f32_tail_d64":
+        kw.update(K_tail=torch.randn(1, 2, 9, D, device="cuda"), V_tail=torch.randn(1, 2, 9, D, device="cuda"))
+    calls, rows = [], _ops.retention_rows
+    monkeypatch.setattr(_ops, "retention_rows", lambda *a: calls.append(a) or rows(*a))
+    op(q, *planes, **kw)
+    assert len(calls) == made
