@@ -201,7 +201,7 @@ PyObject* decode(PyObject*, PyObject* const* a, Py_ssize_t n) {
     if (k_max > P) k_max = P;
 
     fq_query q{};
-    q.q = Q->data_ptr();
+    q.q = q.out = Q->data_ptr();       // out: until O is there (the fused query below checks for one)
     q.q_dtype = q.out_dtype = dtype_code(*Q);
     if (q.q_dtype < 0) return none();
     // Q (..., H_q, 1, D) and O alike, contiguous: (l, b, h, d) strides

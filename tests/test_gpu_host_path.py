@@ -125,3 +125,31 @@ def test_retention_is_prepared_once(monkeypatch, bits, form, made):
     monkeypatch.setattr(_ops, "retention_rows", lambda *a: calls.append(a) or rows(*a))
     op(q, *planes, **kw)
     assert len(calls) == made
+
+
+@pytest.mark.parametrize("bits", [4, 8, 3])
+@pytest.mark.parametrize("nrep", [6, 8])
+def test_whole_steps_of_6_and_8_heads_go_natively(monkeypatch, bits, nrep):
+    """6 or 8 query heads per KV head that the library runs as one launch take the native path."""
+    from flashquest_amd.eager.decode import quest_decode_int4, quest_decode_int8, quest_decode_turbo
+    from tests.cases import to_dev_half
+    from tests.test_gpu_turbo_forms import _case, _device
+    B, Hkv = 13, 8                           # 104 KV heads: 208 virtual ones, past the 192 that fill the GPU
+    if bits == 3:
+        Q, host, raw = _case(5, B, nrep * Hkv, Hkv, 64 * 12)
+        q = to_dev_half(Q, "bf16")[:, :, None]
+        planes = _device(host, 64 * 12) + [to_dev_half(r, "bf16") for r in raw]
+        op = quest_decode_turbo
+    else:
+        c = (Int4Case if bits == 4 else Int8Case)(seed=5, B=B, Hq=nrep * Hkv, Hkv=Hkv, S=64 * 12)
+        q, planes = c.q_dev(), list(c.device().values())
+        op = quest_decode_int4 if bits == 4 else quest_decode_int8
+    op(q, *planes, retention=0.3)            # the workspace is there
+    host, got = _host.module(), []
+    decode = host.decode
+    monkeypatch.setattr(host, "decode", lambda *a: got.append(decode(*a)) or got[-1])
+    o, lse = op(q, *planes, retention=0.3)
+    assert len(got) == 1 and got[0] is not None and got[0][0] is o
+    monkeypatch.setattr(_host, "_module", None)
+    want = op(q, *planes, retention=0.3)
+    assert torch.equal(o, want[0]) and torch.equal(lse, want[1])
