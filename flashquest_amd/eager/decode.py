@@ -69,8 +69,9 @@ def _native_decode(bits, Q, planes, H_kv, retention, head_pattern, num_sinks, wi
         return rows[0]
     stream = L.stream_handle(Q.device)
     res = host.decode(bits, Q, planes, retention_rows, int(num_sinks), int(window_pages),
-                      -1 if k_max_static is None else int(k_max_static), L.SELECT_MODES[select_mode], int(page_size),
-                      sm_scale, bool(return_lse), K_tail, V_tail, L.workspace_if_any(Q.device, stream), stream)
+                      -1 if k_max_static is None else min(int(k_max_static), 0x7FFFFFFF), L.SELECT_MODES[select_mode],
+                      int(page_size), sm_scale, bool(return_lse), K_tail, V_tail,
+                      L.workspace_if_any(Q.device, stream), stream)
     return res, rows[0] if rows else None
 
 

@@ -153,3 +153,12 @@ def test_whole_steps_of_6_and_8_heads_go_natively(monkeypatch, bits, nrep):
     monkeypatch.setattr(_host, "_module", None)
     want = op(q, *planes, retention=0.3)
     assert torch.equal(o, want[0]) and torch.equal(lse, want[1])
+
+
+@pytest.mark.parametrize("k_max", [2 ** 31, 2 ** 32 + 1, 2 ** 63 - 1, 2 ** 70])
+def test_a_bound_past_32_bits_bounds_nothing(monkeypatch, k_max):
+    from flashquest_amd.eager.decode import quest_decode_int4
+    q, planes = _planes(4)
+    _both(monkeypatch, lambda: quest_decode_int4(q, *planes, retention=0.3, k_max_static=k_max))
+    assert torch.equal(quest_decode_int4(q, *planes, retention=0.3, k_max_static=k_max)[0],
+                       quest_decode_int4(q, *planes, retention=0.3)[0])
