@@ -197,3 +197,24 @@ def test_library_takes_six_and_eight_heads_per_kv_head_itself():
                 assert L.lib().fq_quest_fused_int4(cache, q, 4, 2, 16, mode) == want, (layers, Hq, mode)
         Q3 = torch.zeros(layers, 1, 72, D, dtype=torch.float16)
         assert L.lib().fq_quest_fused_int4(cache, _ops.query(Q3, Q3, None, None), 4, 2, 16, 0) < 0
+
+
+def test_a_stale_native_module_leaves_the_ctypes_path(monkeypatch, tmp_path):
+    """A module that does not load (built for another interpreter or torch), or whose
+    library entries are missing, is reported once and not used."""
+    import warnings
+    from flashquest_amd import _host
+    stale = tmp_path / "_fq_host.so"
+    stale.write_bytes(b"not a shared object")
+    for broken in (dict(_PATH=str(stale)), dict(_load=lambda: {}["fq_workspace_bytes"])):
+        with monkeypatch.context() as m:
+            m.setattr(_host, "_module", None)
+            m.setattr(_host, "_loaded", False)
+            m.setattr(_host, "_PATH", str(stale))
+            for k, v in broken.items():
+                m.setattr(_host, k, v)
+            with pytest.warns(RuntimeWarning, match="native host path"):
+                assert _host.module() is None
+            with warnings.catch_warnings():
+                warnings.simplefilter("error")
+                assert _host.module() is None
