@@ -218,3 +218,32 @@ def test_a_stale_native_module_leaves_the_ctypes_path(monkeypatch, tmp_path):
             with warnings.catch_warnings():
                 warnings.simplefilter("error")
                 assert _host.module() is None
+
+
+def _make(*args):
+    import os
+    import subprocess
+    from flashquest_amd.build import CSRC
+    env = {k: v for k, v in os.environ.items() if not k.startswith("MAKE")}
+    p = subprocess.run(["make", "-C", CSRC, "-n", *args], capture_output=True, text=True, env=env)
+    return p.returncode, p.stdout + p.stderr
+
+
+def test_the_build_without_torch_headers_leaves_the_native_module_out():
+    code, said = _make("-B", "PYTHON=false")
+    assert code == 0 and "libfq_hip.so" in said and "host_torch.cpp" not in said and "no _fq_host.so" in said
+    code, said = _make("-B")
+    assert code == 0 and "host_torch.cpp" in said
+
+
+def test_another_torch_or_interpreter_rebuilds_the_native_module(tmp_path):
+    out = tmp_path / "_fq_host.so"
+    out.write_bytes(b"")
+    stamp = tmp_path / "_fq_host.so.abi"
+    args = (f"HOST_OUT={out}", str(out))
+    stamp.write_text("torch 0.0 cpython-0\n")
+    assert "host_torch.cpp" in _make(*args)[1]
+    import importlib.metadata
+    import sysconfig
+    stamp.write_text(f"torch {importlib.metadata.version('torch')} {sysconfig.get_config_var('SOABI')}\n")
+    assert "host_torch.cpp" not in _make(*args)[1]
