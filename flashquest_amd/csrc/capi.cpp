@@ -35,6 +35,8 @@ hipError_t launch_prefill(const Int4Cache& c, const TailArgs& t, const void* q, 
                           const int64_t* o_s, int nrep, int Sq, int causal_off, float qk_scale, void* ws,
                           hipStream_t st);
 size_t prefill_workspace_bytes(const Int4Cache& c, int Skv, int Sq, int nrep, int causal_off);
+void prefill_plan(int Hkv, int B, int Skv, int Sq, int nrep, int causal_off, bool turbo, int* key_groups,
+                  int* key_splits);
 size_t prefill_turbo_workspace_bytes(int Hkv, int B, int Skv, int Sq, int nrep, int causal_off);
 hipError_t launch_prefill_turbo(const fq_turbo_cache& tc, const TailArgs& t, const void* q, const int64_t* q_s,
                                 void* out, const int64_t* o_s, int nrep, int Sq, int causal_off, float qk_scale,
@@ -1267,6 +1269,16 @@ size_t fq_prefill_workspace_bytes(const fq_int4_cache* cache, const fq_tail* tai
     if (bits != 4 && bits != 8) return 0;
     if (prefill_check(cache, tail, query, bits, c, t, &need)) return 0;
     return need;
+}
+
+int fq_prefill_plan(int32_t B, int32_t H_kv, int32_t n_rep, int32_t S_q, int32_t S_kv, int32_t causal_offset,
+                    int32_t bits, int32_t* key_groups, int32_t* key_splits) {
+    if (!key_groups || !key_splits) return fail(FQ_ERR_INVALID, "NULL output");
+    if (bits != 4 && bits != 8 && bits != 3) return fail(FQ_ERR_INVALID, "bits=%d", bits);
+    if (B < 1 || H_kv < 1 || n_rep < 1 || S_q < 1 || S_kv < 1 || causal_offset < 0)
+        return fail(FQ_ERR_INVALID, "B, H_kv, n_rep, S_q and S_kv must be >= 1, causal_offset >= 0");
+    prefill_plan(H_kv, B, S_kv, S_q, n_rep, causal_offset, bits == 3, key_groups, key_splits);
+    return FQ_OK;
 }
 
 static int prefill_turbo_check(const fq_turbo_cache* c, const fq_tail* tail, const fq_prefill* q, TailArgs& t,

@@ -1172,9 +1172,21 @@ size_t prefill_dense_bytes(int Hkv, int B, int Skv, int Sq, int nrep, int causal
     return n;
 }
 
+static bool prefill_single_pass(int Skv, int Sq, int nrep, int causal_off) {
+    return prefill_row_blocks(Sq, nrep) == 1 && prefill_keys_needed(Skv, Sq, causal_off) <= 1024;
+}
+
+void prefill_plan(int Hkv, int B, int Skv, int Sq, int nrep, int causal_off, bool turbo, int* key_groups,
+                  int* key_splits) {
+    DensePlan pl{0, 1};
+    if (turbo || !prefill_single_pass(Skv, Sq, nrep, causal_off))
+        pl = dense_plan((int64_t)Sq * nrep, (int64_t)Hkv * B, prefill_keys_needed(Skv, Sq, causal_off), causal_off);
+    *key_groups = pl.kg;
+    *key_splits = pl.ks;
+}
+
 size_t prefill_workspace_bytes(const Int4Cache& c, int Skv, int Sq, int nrep, int causal_off) {
-    const int64_t keys = prefill_keys_needed(Skv, Sq, causal_off);
-    if (prefill_row_blocks(Sq, nrep) == 1 && keys <= 1024) return 0;
+    if (prefill_single_pass(Skv, Sq, nrep, causal_off)) return 0;
     return prefill_dense_bytes(c.Hkv, c.B, Skv, Sq, nrep, causal_off);
 }
 

@@ -568,6 +568,14 @@ size_t fq_prefill_turbo_workspace_bytes(const fq_turbo_cache* cache, const fq_ta
 size_t fq_prefill_workspace_bytes(const fq_int4_cache* cache, const fq_tail* tail, const fq_prefill* query,
                                   int32_t bits);
 
+/* How a prefill of S_q queries over S_kv keys (n_rep query heads per KV head) is
+ * run, bits 4 / 8 / 3 (TurboQuant): key_groups 1 / 2 / 4 waves' key groups per
+ * workgroup (256 / key_groups query rows each) over key_splits slices of the key
+ * range (more than 1: a merge launch follows); key_groups 0: the single pass that
+ * dequantises its own tiles.  No reference counterpart. */
+int fq_prefill_plan(int32_t B, int32_t H_kv, int32_t n_rep, int32_t S_q, int32_t S_kv, int32_t causal_offset,
+                    int32_t bits, int32_t* key_groups, int32_t* key_splits);
+
 #ifdef __cplusplus
 }
 #endif

@@ -64,3 +64,51 @@ def test_prefill_argument_errors():
         assert lib.fq_prefill_int4(c, tail, q, None, 0, None) == want
     # a long prompt without its workspace
     assert lib.fq_prefill_int4(_cache(), tail, _query(Sq=256), None, 0, None) == L.FQ_ERR_WORKSPACE
+
+
+def _plan(Hq, Hkv, S, T, B=1, Sq=None, causal_offset=0, bits=4, **_):
+    kg, ks = ctypes.c_int32(-1), ctypes.c_int32(-1)
+    assert L.lib().fq_prefill_plan(B, Hkv, Hq // Hkv, S + T if Sq is None else Sq, S + T, causal_offset, bits, kg,
+                                   ks) == L.FQ_OK
+    return kg.value, ks.value
+
+
+def _blocks_with_empty_slices(plan, Hq, Hkv, S, T, Sq=None, causal_offset=0, **_):
+    kg, ks = plan
+    rep, rows_wg = Hq // Hkv, 256 // kg
+    rows = (S + T if Sq is None else Sq) * rep
+    n = 0
+    for first in range(0, rows, rows_wg):
+        last = min(rows, first + rows_wg) - 1
+        stages = -(-min(S + T, last // rep + causal_offset + 1) // 128)
+        n += -(-stages // -(-stages // ks)) < ks
+    return n
+
+
+def test_prefill_tests_take_the_forms_they_name():
+    """The shapes of the GPU tests below take the key groups and splits they are there
+    for, so that a change of the plan's constants cannot move them unseen."""
+    from tests.test_gpu_prefill_plans import FORMS, SPLIT_FORMS
+    for kw, plan, empty in FORMS + SPLIT_FORMS:
+        for bits in (4, 8, 3):
+            assert _plan(**kw, bits=bits) == plan, kw
+        assert _blocks_with_empty_slices(plan, **kw) == empty, kw
+    forms = {(kg, ks > 1) for _, (kg, ks), _ in FORMS + SPLIT_FORMS}
+    assert forms == {(kg, split) for kg in (1, 2, 4) for split in (False, True)}
+    # test_gpu_prefill.py's
+    assert _plan(Hq=24, Hkv=8, B=2, S=2048, T=30, Sq=800, causal_offset=1278) == (2, 1)
+    for kw, plan in [(dict(S=8192, T=30, Sq=64, causal_offset=8158), (4, 13)),
+                     (dict(S=4096, T=0, Sq=16, causal_offset=4080), (4, 8)),
+                     (dict(S=4096, T=5, Sq=200, causal_offset=3901, bits=8), (4, 7)),
+                     (dict(S=2048, T=64, Sq=300, Hq=8, causal_offset=1812), (4, 4)),
+                     (dict(S=4096, T=20, Sq=48, causal_offset=4068, bits=3), (4, 7))]:
+        assert _plan(**{"Hq": 6, "Hkv": 2, **kw}) == plan, kw
+    # the single pass, for the quantised caches with metadata per page alone
+    assert _plan(Hq=6, Hkv=2, S=256, T=3, Sq=40) == (0, 1) and _plan(Hq=6, Hkv=2, S=256, T=3, Sq=40, bits=3)[0] > 0
+
+
+def test_prefill_plan_arguments():
+    kg = ctypes.c_int32()
+    for bad in [(0, 2, 3, 8, 8, 0, 4), (1, 2, 3, 0, 8, 0, 4), (1, 2, 3, 8, 8, -1, 4), (1, 2, 3, 8, 8, 0, 5)]:
+        assert L.lib().fq_prefill_plan(*bad, kg, kg) == L.FQ_ERR_INVALID
+    assert L.lib().fq_prefill_plan(1, 2, 3, 8, 8, 0, 4, None, kg) == L.FQ_ERR_INVALID

@@ -218,9 +218,9 @@ def test_prefill_key_range_splits(kw):
     _check(PrefillCase(13, **kw))
 
 
-def test_prefill_key_range_splits_between_128_and_256_workgroups():
-    # 10 row blocks x 16 (sequence, KV head) pairs = 160 workgroups: split in 3
-    # key ranges so the 480 workgroups fill two rounds of the CUs
+def test_prefill_160_row_blocks():
+    # 10 blocks of 256 rows x 16 (sequence, KV head) pairs: 2 key groups and 304
+    # workgroups, no split (test_cpu_prefill.py; with splits: test_gpu_prefill_plans.py)
     _check(PrefillCase(21, B=2, Hq=24, Hkv=8, S=2048, T=30, Sq=800, causal_offset=2078 - 800))
 
 
