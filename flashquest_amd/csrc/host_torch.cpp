@@ -166,8 +166,8 @@ PyObject* none() { Py_RETURN_NONE; }
 // decode(bits, Q, planes (6, or 8 with TurboQuant's raw metadata), retention rows, sinks, window, k_max or -1,
 //        mode, page, sm_scale or None, return_lse, K_tail, V_tail, workspace, stream)
 //   -> (O, lse or None), or None
-// retention rows: a function of no arguments that gives (rows, layer stride), called once everything else is known
-// to be the plain case (it may copy to the device and launch), its errors raised.
+// retention rows: (rows, layer stride), or a function of no arguments that gives them, called once everything else
+// is known to be the plain case (it may copy to the device and launch), its errors raised.
 PyObject* decode(PyObject*, PyObject* const* a, Py_ssize_t n) {
     HANDLE_TH_ERRORS
     if (n != 15) return none();
@@ -229,7 +229,7 @@ PyObject* decode(PyObject*, PyObject* const* a, Py_ssize_t n) {
     }
     const size_t need = bits == 3 ? g_fq.ws_turbo(&tc, Hq) : g_fq.ws_int4(&c, Hq);
     if (need > (size_t)ws->numel()) return none();
-    const THPObjectPtr made(PyObject_CallNoArgs(a[3]));
+    const THPObjectPtr made(PyTuple_Check(a[3]) ? Py_NewRef(a[3]) : PyObject_CallNoArgs(a[3]));
     if (!made) return nullptr;
     const at::Tensor* ret =
         PyTuple_Check(made.get()) && PyTuple_GET_SIZE(made.get()) == 2 ? plain(PyTuple_GET_ITEM(made.get(), 0)) : nullptr;

@@ -8,6 +8,7 @@ packed cache, and merge with dense attention over the partial-page tail
 """
 from __future__ import annotations
 
+import functools
 import math
 
 import torch
@@ -52,27 +53,28 @@ def merge_two_attentions(O_a, lse_a, O_b, lse_b) -> torch.Tensor:
     return out.view(O_a.shape)
 
 
-def _native_decode(bits, Q, planes, H_kv, retention, head_pattern, num_sinks, window_pages, k_max_static, select_mode,
-                   page_size, sm_scale, return_lse, K_tail, V_tail):
-    """The step through the native host path: ((O, lse), or None for the general
-    way; the retention rows if the path got as far as asking for them, which the
-    general way then takes over)."""
-    host = _host.module()
-    H_q = Q.shape[-3]
-    if host is None or H_kv < 1 or H_q % H_kv:
-        return None, None
-    rows = []
+# query heads per KV head that a step can have whole on any layout; others only where it is not
+# the matrix cores' (wants_head_chunks), which pads or chunks them into steps of their own
+_WHOLE = (1, 2, 3, 4, 6, 8)
 
-    def retention_rows():
-        rows.append(_ops.retention_rows(retention, head_pattern, H_q, H_kv, Q.shape[0] if Q.dim() == 5 else 1,
-                                        Q.device))
-        return rows[0]
+
+def _native_decode(bits, Q, planes, H_kv, nrep, retention, head_pattern, num_sinks, window_pages, k_max_static,
+                   select_mode, page_size, sm_scale, return_lse, K_tail, V_tail):
+    """The step through the native host path: ((O, lse), or None for the general
+    way; the retention rows, which the general way then takes over, or None).
+    With 6 or 8 query heads per KV head the rows are made only if the library takes
+    the step whole: it is chunked otherwise, with rows of its own."""
+    host = _host.module()
+    if host is None or nrep == 0:
+        return None, None
+    args = (retention, head_pattern, nrep * H_kv, H_kv, Q.shape[0] if Q.dim() == 5 else 1, Q.device)
+    rows = functools.partial(_ops.retention_rows, *args) if nrep in (6, 8) else _ops.retention_rows(*args)
     stream = L.stream_handle(Q.device)
-    res = host.decode(bits, Q, planes, retention_rows, int(num_sinks), int(window_pages),
+    res = host.decode(bits, Q, planes, rows, int(num_sinks), int(window_pages),
                       -1 if k_max_static is None else min(int(k_max_static), 0x7FFFFFFF), L.SELECT_MODES[select_mode],
                       int(page_size), sm_scale, bool(return_lse), K_tail, V_tail,
                       L.workspace_if_any(Q.device, stream), stream)
-    return res, rows[0] if rows else None
+    return res, None if nrep in (6, 8) else rows
 
 
 _FUSED_TAIL_REFUSED = "the fused tail needs the matrix-core attention layout"
@@ -176,15 +178,17 @@ def quest_decode_int4(
     if D not in (64, 128):
         raise NotImplementedError(f"head_dim={D} not in (64, 128)")
     H_kv = K_scale.shape[-3]
+    H_q = Q.shape[-3]
+    nrep = H_q // H_kv if H_q % H_kv == 0 else 0
     rows = None
-    if out is None and _rotation is None and not return_selection and not _direct:
-        res, rows = _native_decode(4, Q, (K_packed, K_scale, K_mn, V_packed, V_scale, V_mn), H_kv, retention,
-                                   head_pattern, num_sinks, window_pages, k_max_static, select_mode, page_size,
-                                   sm_scale, return_lse, K_tail, V_tail)
+    if (out is None and _rotation is None and not return_selection and not _direct
+            and (nrep in _WHOLE or not _ops.wants_head_chunks(H_q, H_kv, D, page_size))):
+        res, rows = _native_decode(4, Q, (K_packed, K_scale, K_mn, V_packed, V_scale, V_mn), H_kv, nrep,
+                                   retention, head_pattern, num_sinks, window_pages, k_max_static, select_mode,
+                                   page_size, sm_scale, return_lse, K_tail, V_tail)
         if res is not None:
             return res
-    nrep = Q.shape[-3] // H_kv if Q.shape[-3] % H_kv == 0 else 0
-    if (not _direct and _ops.wants_head_chunks(Q.shape[-3], H_kv, D, page_size) and _rotation is None
+    if (not _direct and _ops.wants_head_chunks(H_q, H_kv, D, page_size) and _rotation is None
             and not _one_launch(4, Q, (K_packed, K_scale, K_mn, V_packed, V_scale, V_mn), nrep, page_size,
                                 select_mode, num_sinks, window_pages, k_max_static)):
         planes = (K_packed, K_scale, K_mn, V_packed, V_scale, V_mn)
@@ -195,7 +199,6 @@ def quest_decode_int4(
         return res if res is not None else _chunked_decode(4, Q, planes, H_kv, nrep, out, kw)
     layered = Q.dim() == 5
     Q3 = Q[..., 0, :]
-    H_q = Q3.shape[-2]
     P = K_scale.shape[-2]
     O3 = torch.empty_like(Q3) if out is None else out[..., 0, :]
     lse = torch.empty(Q3.shape[:-1], dtype=torch.float32, device=Q.device) if return_lse else None
@@ -535,15 +538,17 @@ def quest_decode_int8(
     if D not in (64, 128):
         raise NotImplementedError(f"head_dim={D} not in (64, 128)")
     H_kv = K_scale.shape[-3]
+    H_q = Q.shape[-3]
+    nrep = H_q // H_kv if H_q % H_kv == 0 else 0
     rows = None
-    if not return_selection and not _direct:
-        res, rows = _native_decode(8, Q, (K_uint8, K_scale, K_mn, V_uint8, V_scale, V_mn), H_kv, retention,
-                                   head_pattern, num_sinks, window_pages, k_max_static, select_mode, page_size,
-                                   sm_scale, return_lse, K_tail, V_tail)
+    if (not return_selection and not _direct
+            and (nrep in _WHOLE or not _ops.wants_head_chunks(H_q, H_kv, D, page_size))):
+        res, rows = _native_decode(8, Q, (K_uint8, K_scale, K_mn, V_uint8, V_scale, V_mn), H_kv, nrep,
+                                   retention, head_pattern, num_sinks, window_pages, k_max_static, select_mode,
+                                   page_size, sm_scale, return_lse, K_tail, V_tail)
         if res is not None:
             return res
-    nrep = Q.shape[-3] // H_kv if Q.shape[-3] % H_kv == 0 else 0
-    if (not _direct and _ops.wants_head_chunks(Q.shape[-3], H_kv, D, page_size)
+    if (not _direct and _ops.wants_head_chunks(H_q, H_kv, D, page_size)
             and not _one_launch(8, Q, (K_uint8, K_scale, K_mn, V_uint8, V_scale, V_mn), nrep, page_size,
                                 select_mode, num_sinks, window_pages, k_max_static)):
         planes = (K_uint8, K_scale, K_mn, V_uint8, V_scale, V_mn)
@@ -553,7 +558,6 @@ def quest_decode_int8(
         res = _padded_decode(8, Q, planes, H_kv, nrep, None, kw) if nrep in (5, 7) else None
         return res if res is not None else _chunked_decode(8, Q, planes, H_kv, nrep, None, kw)
     Q3 = Q[..., 0, :]
-    H_q = Q3.shape[-2]
     P = K_scale.shape[-2]
     O3 = torch.empty_like(Q3)
     lse = torch.empty(Q3.shape[:-1], dtype=torch.float32, device=Q.device) if return_lse else None
@@ -643,15 +647,17 @@ def quest_decode_turbo(
     if K_scale_raw.dtype != torch.bfloat16 or K_mn_raw.dtype != torch.bfloat16:
         raise AssertionError("K_scale_raw / K_mn_raw must be bf16")
     H_kv = K_msb.shape[-3]
+    H_q = Q.shape[-3]
+    nrep = H_q // H_kv if H_q % H_kv == 0 else 0
     rows = None
-    if not return_selection and not _direct:
+    if (not return_selection and not _direct
+            and (nrep in _WHOLE or not _ops.wants_head_chunks(H_q, H_kv, D, page_size))):
         res, rows = _native_decode(3, Q, (K_msb, K_lsb, K_scale_turbo, V_msb, V_lsb, V_scale_turbo, K_scale_raw,
-                                          K_mn_raw), H_kv, retention, head_pattern, num_sinks, window_pages, k_max_static,
-                                   select_mode, page_size, sm_scale, return_lse, None, None)
+                                          K_mn_raw), H_kv, nrep, retention, head_pattern, num_sinks, window_pages,
+                                   k_max_static, select_mode, page_size, sm_scale, return_lse, None, None)
         if res is not None:
             return res
-    nrep = Q.shape[-3] // H_kv if Q.shape[-3] % H_kv == 0 else 0
-    if (not _direct and _ops.wants_head_chunks(Q.shape[-3], H_kv, D, page_size)
+    if (not _direct and _ops.wants_head_chunks(H_q, H_kv, D, page_size)
             and not _one_launch(3, Q, (K_msb, K_lsb, K_scale_turbo, V_msb, V_lsb, V_scale_turbo), nrep, page_size,
                                 select_mode, num_sinks, window_pages, k_max_static, raw=(K_scale_raw, K_mn_raw))):
         planes = (K_msb, K_lsb, K_scale_turbo, V_msb, V_lsb, V_scale_turbo)
@@ -662,7 +668,6 @@ def quest_decode_turbo(
         res = _padded_decode(3, Q, planes, H_kv, nrep, None, kw, raw=raw) if nrep in (5, 7) else None
         return res if res is not None else _chunked_decode(3, Q, planes, H_kv, nrep, None, kw, raw=raw)
     Q3 = Q[..., 0, :]
-    H_q = Q3.shape[-2]
     P = K_scale_raw.shape[-2]
     O3 = torch.empty_like(Q3)
     lse = torch.empty(Q3.shape[:-1], dtype=torch.float32, device=Q.device) if return_lse else None
