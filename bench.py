@@ -300,7 +300,7 @@ def self_check(cache, dec, mask, k, args):
     """The timed kernel computes the right thing: its in-kernel selection equals
     the selection kernel's (split path) bit for bit on every group, and O of
     every layer agrees with the split path (several workgroups per KV group and
-    a merge launch, a different fp32 order) within the north-star 2e-3."""
+    a merge launch, a different fp32 order) within the decode bar, 2e-3."""
     from flashquest_amd import _lib as L
     o_fused = dec.O3.clone()
     smask = torch.zeros_like(mask)

@@ -17,8 +17,12 @@
 //         added at the end; grouped: a second operand), both multiplied by the same B = the codes as fp16 subnormals (bits =
 //         code, value = code * 2^-24, exact) into one fp32 accumulator; plus
 //         sum_t p_t * V_mn[t,g] on the VALU.  hi + lo equals the fp32 A to
-//         2^-22 relative (the lo part's own fp16 rounding), so the products
-//         carry fp32-level precision like the reference's fp32 p * v.
+//         2^-22 relative (the lo part's own fp16 rounding).  The sums are coarser:
+//         1e-4 to 5e-4 of |O| off 64 bits with float32 queries over 8192 tokens (5e-3
+//         with fp16 metadata, whose A is not scaled, and V of size 1e-3), 20 times
+//         INT8's with its larger codes: the matrix unit keeps less below the largest
+//         product when codes are subnormals.  16-bit outputs round at 2e-4 to 2e-3.
+//         D = 64 does both products in int8 digits instead (fused_common.h): 1e-6.
 //
 // Single pass per page: each wave owns every 4th page of its workgroup's
 // split, loads a page (K, V, metadata) one page ahead of the one it computes,

@@ -1,17 +1,19 @@
-// Cache writes on page completion: INT4 quantisation of whole 64-token pages
-// straight from their two sources (the bf16 partial-page tail and the newly
-// appended tokens), and the tail staging copy.  Reference semantics:
-// src/flashquest/cache/persistent_int4.py:69-132 (update_quantized) with the
-// quantisers of src/flashquest/kernel/kv_quant.py:131-205.
+// Cache writes on page completion: INT4 and INT8 quantisation of whole 64-token
+// pages straight from their two sources (the bf16 partial-page tail and the newly
+// appended tokens), and the tail staging copy; the same kernel serves the whole-tensor
+// quantisers.  Reference semantics: src/flashquest/cache/persistent_int4.py:69-132
+// (update_quantized) with the quantisers of src/flashquest/kernel/kv_quant.py:43-89,
+// 131-205.
 //
 // One workgroup of 256 threads per (page, batch * head).  Thread t owns 8
 // channels (c8 = t % (D/8)) of tokens r, r + RPP, ... (r = t / (D/8)): every
 // load is 16 contiguous bytes and the D/8 threads of a token read one
 // contiguous row.  K: per-channel min/max over the page (lane swaps, then
-// LDS across the 4 waves), scale arithmetic in the input dtype, codes by
-// fp32 division (the values quant_k_kernel computes).  V: per-token,
-// per-group min/max over the group's lanes, fp32 arithmetic (as
-// quant_v_kernel).  Codes are stored 4 bytes (8 channels) per thread and token.
+// LDS across the 4 waves), scale arithmetic in the input dtype, codes
+// the fp32 quotient's (the values quant_k_kernel computes by division).  V:
+// per-token, per-group min/max over the group's lanes, fp32 arithmetic (as
+// quant_v_kernel).  Codes are stored 8 channels per thread and token (INT4 4
+// bytes, INT8 8).
 //
 // A page has few bytes for its arithmetic, and its loads, arithmetic and stores do
 // not overlap (one round of workgroups at ordinary sizes), so it is bound by

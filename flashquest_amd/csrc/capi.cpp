@@ -433,10 +433,12 @@ static bool decode_selects_in_attention(const Int4Cache& c, const QueryArgs& q, 
 // each re-scoring the group's pages.  INT4 and INT8, unrotated; with head_dim
 // 64 every such step (those kernels have no scorer of their own).  Up to
 // kSplitScorePages pages the redundant scoring in every split is cheaper than the
-// launch it saves: one layer of 8 groups, with the scoring launch and without, 64
-// pages 19.9 / 17.4 us, 128 pages 20.5 / 18.8, 160 pages 21.4 / 20.1, 192 pages
-// 21.5 / 21.0 (INT8 23.7 / 23.9), 256 pages 23.3 / 24.6; 128 groups, 160 pages 35.5
-// / 33.5.
+// launch it saves.  One layer, INT4, per query head, with the scoring launch and
+// without, 8 / 32 / 128 groups: 24 / 8 heads, 64 pages 20.1 / 20.6 / 25.9 and 17.7 /
+// 18.3 / 22.5 us, 160 pages 21.6 / 23.7 / 34.2 and 20.4 / 23.2 / 32.5, 192 pages 21.8 /
+// 24.2 / 37.6 and 21.1 / 24.5 / 36.4, 256 pages 23.6 / 25.9 / 44.5 and 23.8 / 28.1 /
+// 44.2; 32 / 8 heads, whose scoring costs most, 160 pages 22.7 / 24.6 / 37.2 and 22.3
+// / 25.3 / 36.3.  INT8 and summed rows lie the same way.
 constexpr int kSplitScorePages = 160;
 static bool attend_from_scores(const Int4Cache& c, const QueryArgs& q, int bound) {
     if (c.D == 64) return true;

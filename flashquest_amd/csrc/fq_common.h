@@ -20,7 +20,13 @@ constexpr int kNoPage = 0x7FFF;
 // one launch with one workgroup per group (it scores, selects and attends
 // itself: a few pages per wave) even when the groups do not fill the GPU;
 // longer lists split each group over workgroups (behind a scoring launch where
-// scoring the group in each of them would cost more).
+// scoring the group in each of them would cost more).  The line was drawn against
+// split steps that all had the scoring launch.  One layer, 24 / 8 heads, 128 pages,
+// 37-token tail, 8 / 64 / 128 groups, one launch and split: per query head, lists of
+// 12 to 16 pages 18.3 / 18.4 / 19.0 us and 18.3 / 19.6 / 21.2, summed 18.8 / 18.7 /
+// 19.7 and 19.0 / 19.3 / 20.7; 24 pages (summed) 20.9 / 21.2 / 22.0 and 18.6 / 20.0 /
+// 21.6; 40 pages 24.5 / 24.9 / 25.8 and 18.6 / 20.7 / 24.1: past some 20 pages the
+// split step is the faster one now.
 constexpr int kFusedSmallPages = 40;
 constexpr int kMaxRows = 16;       // query rows per KV group in scoring (n_rep * S_q)
 constexpr float kLog2e = 1.4426950408889634f;

@@ -575,7 +575,7 @@ hipError_t launch_score(const Int4Cache& c, const QueryArgs& q, int S_q, const i
         FQ_BLOCK(16)
     } else if (q.nrep <= 4 && G < 192 && c.P <= 64 * kSelC) {     // few groups
         FQ_BLOCK(kSelC)
-    } else if (c.P > 64 * 8 && c.P <= 64 * 32 && q.nrep > 1 && select_mode == FQ_SELECT_PER_Q_HEAD) {
+    } else if (c.P > 64 * 8 && c.P <= 64 * 32 && select_mode == FQ_SELECT_PER_Q_HEAD) {     // more than 4 query heads
         if (c.P <= 64 * 16) hipLaunchKernelGGL(select_groups_rows_kernel<16>, dim3(G), dim3(kThreads), 0, st, sp);
         else hipLaunchKernelGGL(select_groups_rows_kernel<32>, dim3(G), dim3(kThreads), 0, st, sp);
     } else if (c.P <= 64 * 8) hipLaunchKernelGGL(select_groups_wave_kernel<8>, dim3(G), dim3(64), 0, st, sp, G);

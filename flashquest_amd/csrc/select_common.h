@@ -184,7 +184,7 @@ FQ_DEV ForcedPages forced_pages(int P, int num_sinks, int window) {
 // pages 64 j + lane with j = w (mod NW) alone, the counts meet in LDS, and each
 // wave writes its entries.  (Every wave ranking every page, as before, took
 // two thirds of the selection: 3.2 us a step with 3 query heads and 128 to 512
-// pages, now SELECT_NOTE.)  Ties and forced pages follow
+// pages, now 2.0.)  Ties and forced pages follow
 // wave_topk / wave_select_group; the entry list holds the forced pages first,
 // then the other selected pages, each part ascending.  NROWS = 1: one top-k of
 // the summed row with the group's largest retention (per_kv_head_sum); NROWS =

@@ -167,6 +167,8 @@ void attn_turbo_fused_kernel(TurboFusedParams a) {
     constexpr int D = 128, NW = 8, NT = 512;
     static_assert(NREP <= 4, "query heads per KV head");
     static_assert(!HCH || FUSED, "head chunks run in the fused kernel");
+    // a row takes two digit products a token: |A| <= 128 against |H| <= 85 and |L| <= 128
+    static_assert((int64_t)kMaxWgPages / NW * 64 * 128 * (85 + 128) < INT32_MAX, "a wave's int32 sums");
     __shared__ SplitLds<D, NREP, NW> s_split;
     __shared__ int s_ent[kMaxWgPages];
     __shared__ float s_qraw[HCH ? 2 * NREP : NREP][D];      // chunk_sum: every head of the cache head

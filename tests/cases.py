@@ -150,7 +150,7 @@ def fp64_selection_check(q, K_scale, K_mn, got_rows, retention, mode, num_sinks=
     return nrow, amb, mis, amb_diff
 
 
-TOL_O = 2e-3      # decode output vs the fp32 oracle, max-abs
+TOL_O = 2e-3      # the decode bar: decode output vs the fp32 oracle, max-abs
 
 
 def decode_tol(ref_o, out_dtype="f16"):

@@ -15,7 +15,7 @@ channels, planted pages, fp16 metadata, V in 32-channel groups) and check
   are counted as ambiguous, with how many of them the GPU resolved unlike
   the fp64 order, and printed);
 * O and lse of sampled layers against the oracle's fp64 attention over the
-  same selection: a flat 2e-3 max-abs for fp16 output (
+  same selection: a flat 2e-3 max-abs for fp16 output (the decode bar,
   output rounding included); the largest error per configuration is printed;
 * that asking for the mask does not change O (same kernel, bitwise);
 * the split path (several workgroups per group, merge launch) against the
@@ -49,7 +49,7 @@ LAYERS, P = 28, 512
 
 
 def _tol(ref_o):
-    """fp16 output: the flat 2e-3 north-star bar, output rounding included."""
+    """fp16 output: the flat 2e-3 decode bar, output rounding included."""
     return TOL_O
 
 

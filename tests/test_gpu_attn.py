@@ -8,7 +8,7 @@ from tests.cases import decode_tol, Int4Case, max_err, to_dev
 
 pytestmark = pytest.mark.gpu
 
-TOL_O = 2e-3      # fp16/bf16 output vs the fp32 oracle (plus output rounding, below)
+TOL_O = 2e-3      # the decode bar: fp16/bf16 output vs the fp32 oracle (plus output rounding, below)
 
 
 def _tol(case, ref_o):
