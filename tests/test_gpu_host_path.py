@@ -10,9 +10,18 @@ from tests.cases import Int4Case, Int8Case
 pytestmark = pytest.mark.gpu
 
 
-def _both(monkeypatch, call):
-    assert _host.module() is not None, "the native host path is built with the library"
-    got = call()
+def _both(monkeypatch, call, native=True):
+    """call() through the native path and without the module: the same results.  native: whether the module takes
+    every call made of it (None: either); a call before warms the workspace, without which it takes none."""
+    host = _host.module()
+    assert host is not None, "the native host path is built with the library"
+    call()
+    answers = []
+    with monkeypatch.context() as m:
+        for name in ("decode", "prefill", "quantize"):
+            m.setattr(host, name, lambda *a, f=getattr(host, name): answers.append(f(*a)) or answers[-1])
+        got = call()
+    assert answers and (native is None or all((x is not None) == native for x in answers))
     with monkeypatch.context() as m:
         m.setattr(_host, "_module", None)
         want = call()
@@ -24,8 +33,8 @@ def _both(monkeypatch, call):
             assert torch.equal(g, w)
 
 
-def _planes(bits, room=0, layers=0):
-    case = (Int4Case if bits == 4 else Int8Case)(seed=5, B=2, Hq=6, Hkv=2, S=64 * 45)
+def _planes(bits, room=0, layers=0, D=128):
+    case = (Int4Case if bits == 4 else Int8Case)(seed=5, B=2, Hq=6, Hkv=2, S=64 * 45, D=D)
     keys = ("K_packed", "K_scale", "K_mn", "V_packed", "V_scale", "V_mn") if bits == 4 else \
         ("K_uint8", "K_scale", "K_mn", "V_uint8", "V_scale", "V_mn")
     d, out = case.device(), []
@@ -41,14 +50,16 @@ class Sub(torch.Tensor):
 
 
 @pytest.mark.parametrize("bits", [4, 8])
-@pytest.mark.parametrize("form", ["plain", "layers", "room", "tail", "no_lse", "q_strided", "q_subclass", "misaligned", "k_max"])
+@pytest.mark.parametrize("form", ["plain", "layers", "room", "tail", "no_lse", "q_strided", "q_subclass", "misaligned", "k_max",
+                                  "d64", "d64_tail", "f32_query", "sum", "pattern", "layer_patterns", "head_retention"])
 def test_decode(monkeypatch, bits, form):
     from flashquest_amd.eager.decode import quest_decode_int4, quest_decode_int8
-    q, planes = _planes(bits, room=3 if form == "room" else 0, layers=2 if form == "layers" else 0)
+    D = 64 if form.startswith("d64") else 128
+    q, planes = _planes(bits, room=3 if form == "room" else 0, layers=2 if form in ("layers", "layer_patterns") else 0, D=D)
     kw = dict(retention=0.3)
-    if form == "tail":
-        kw.update(K_tail=torch.randn(2, 2, 64, 128, device="cuda").bfloat16()[:, :, :11],
-                  V_tail=torch.randn(2, 2, 64, 128, device="cuda").bfloat16()[:, :, :11])
+    if form.endswith("tail"):
+        kw.update(K_tail=torch.randn(2, 2, 64, D, device="cuda").bfloat16()[:, :, :11],
+                  V_tail=torch.randn(2, 2, 64, D, device="cuda").bfloat16()[:, :, :11])
     elif form == "no_lse":
         kw["return_lse"] = False
     elif form == "q_strided":
@@ -60,8 +71,33 @@ def test_decode(monkeypatch, bits, form):
         planes[0] = flat[2:].view(planes[0].shape).copy_(planes[0])
     elif form == "k_max":
         kw["k_max_static"] = 7
+    elif form == "f32_query":
+        q = q.float() * 1.001
+    elif form == "sum":
+        kw["select_mode"] = "per_kv_head_sum"
+    elif form == "pattern":
+        kw["head_pattern"] = torch.tensor([True, False])
+    elif form == "layer_patterns":
+        kw["head_pattern"] = torch.tensor([[True, False], [False, True]])
+    elif form == "head_retention":
+        kw["retention"] = torch.linspace(0.1, 0.6, 6)
     op = quest_decode_int4 if bits == 4 else quest_decode_int8
-    _both(monkeypatch, lambda: op(q, *planes, **kw))
+    _both(monkeypatch, lambda: op(q, *planes, **kw), native=form not in ("q_strided", "q_subclass", "misaligned"))
+
+
+@pytest.mark.parametrize("layers", [0, 2])
+@pytest.mark.parametrize("mode", ["per_q_head", "per_kv_head_sum"])
+def test_decode_turbo(monkeypatch, layers, mode):
+    from flashquest_amd.eager.decode import quest_decode_turbo
+    from tests.cases import to_dev_half
+    from tests.test_gpu_turbo_forms import _case, _device
+    S = 64 * 30 + 7
+    Q, host, raw = _case(9, 2, 6, 2, S)
+    planes = _device(host, S + 3) + [to_dev_half(r, "bf16") for r in raw]
+    q = to_dev_half(Q, "bf16")[:, :, None]
+    if layers:
+        q, planes = torch.stack([q] * layers), [torch.stack([p] * layers) for p in planes]
+    _both(monkeypatch, lambda: quest_decode_turbo(q, *planes, retention=0.3, select_mode=mode))
 
 
 @pytest.mark.parametrize("bits", [4, 8])
@@ -72,7 +108,7 @@ def test_prefill(monkeypatch, bits, tail, dtype):
     q = torch.randn(2, 6, 50, 128, device="cuda").to(dtype)
     kt, vt = (torch.randn(2, 2, tail, 128, device="cuda").to(dtype) for _ in range(2))
     op = flash_attn_prefill_int4 if bits == 4 else flash_attn_prefill_int8
-    _both(monkeypatch, lambda: (op(q, *planes, kt, vt, causal_offset=100),))
+    _both(monkeypatch, lambda: (op(q, *planes, kt, vt, causal_offset=100),), native=dtype == torch.bfloat16)
 
 
 @pytest.mark.parametrize("meta", [torch.bfloat16, torch.float16])
