@@ -649,7 +649,7 @@ static int quest_fused(const fq_int4_cache* cache, const fq_query* query, int32_
     mfma_head_chunks(c, q, num_sinks, window_pages, k_max, select_mode, s_max_for(c.P), nullptr);
     const AttnLaunch al = choose_split(c.L * c.B * c.Hkv, quest_bound(c, q, num_sinks, window_pages, k_max, select_mode),
                                        s_max_for(c.P));
-    return attn_selects_in_kernel(c, q, al) ? 1 : 0;
+    return c.D == 128 && attn_selects_in_kernel(c, q, al) ? 1 : 0;      // 64: always from a scoring launch's scores
 }
 
 int fq_quest_fused_int4(const fq_int4_cache* cache, const fq_query* query, int32_t num_sinks, int32_t window_pages,

@@ -794,8 +794,9 @@ class QuestDecoder:
 
     @property
     def fused(self) -> bool:
-        """True when attend() is the whole step: one attention kernel that scores
-        and selects its own pages (select() then launches nothing)."""
+        """True when one attention kernel scores and selects its own pages: attend()
+        is the whole step (select() launches nothing, or, where few KV groups are split
+        over several workgroups, the scores they select from)."""
         if self._padded is not None:
             return self._inner.fused
         if self._chunked is not None:

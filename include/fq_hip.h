@@ -300,8 +300,9 @@ int fq_quest_decode_int8_tail(const fq_int8_cache* cache, const fq_query* query,
 
 /* Whether fq_quest_attend_int4 scores and selects the pages inside its one
  * attention kernel for these arguments (1; fq_quest_select_int4 then launches
- * nothing unless scores_out or mask_out is given) or consumes page lists left
- * by fq_quest_select_int4 (0).  Negative: an FQ_ERR_* code for invalid
+ * nothing unless scores_out or mask_out is given, or, where few KV groups are
+ * split over several workgroups, the scores they select from) or consumes what
+ * fq_quest_select_int4 left (0: page lists, or scores with head_dim 64).  Negative: an FQ_ERR_* code for invalid
  * arguments.  No reference counterpart: it tells a caller (the benchmark) which
  * kernels one decode step runs. */
 int fq_quest_fused_int4(const fq_int4_cache* cache, const fq_query* query,

@@ -199,6 +199,21 @@ def test_library_takes_six_and_eight_heads_per_kv_head_itself():
         assert L.lib().fq_quest_fused_int4(cache, _ops.query(Q3, Q3, None, None), 4, 2, 16, 0) < 0
 
 
+
+@pytest.mark.parametrize("bits", [4, 8])
+@pytest.mark.parametrize("D,layers,want", [(128, 28, 1), (64, 28, 0), (64, 1, 0)])
+def test_64_channel_steps_take_the_selection_half(bits, D, layers, want):
+    """head_dim 64 attends from a scoring launch's scores, however many groups there are: not a single launch."""
+    Hkv, P = 8, 64
+    S, W = P * 64, D // 2 if bits == 4 else D
+    code = lambda: torch.zeros(layers, 1, Hkv, S, W, dtype=torch.uint8)
+    meta = lambda rows, n: torch.zeros(layers, 1, Hkv, rows, n, dtype=torch.bfloat16)
+    planes = (code(), meta(P, D), meta(P, D), code(), meta(S, 1), meta(S, 1))
+    cache, keep = (_ops.int4_cache if bits == 4 else _ops.int8_cache)(*planes, 64)
+    Q3 = torch.zeros(layers, 1, 24, D, dtype=torch.bfloat16)
+    fused = L.lib().fq_quest_fused_int4 if bits == 4 else L.lib().fq_quest_fused_int8
+    assert fused(cache, _ops.query(Q3, Q3, None, None), 4, 2, 16, 0) == want
+
 def test_a_stale_native_module_leaves_the_ctypes_path(monkeypatch, tmp_path):
     """A module that does not load (built for another interpreter or torch), or whose
     library entries are missing, is reported once and not used."""
